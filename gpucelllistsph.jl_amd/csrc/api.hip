@@ -92,6 +92,17 @@ __global__ void k_maxpairs(const int32_t* __restrict__ cnt, CellGeom g, unsigned
   if (val) atomicAdd(out, (unsigned long long)val);
 }
 
+// The smallest t with sqrt(t) >= r: r2 < t is then sqrt(r2) < r for every
+// double r2 (the square root is correctly rounded, so it is monotone), also on
+// lattices with neighbours at exactly r.
+double sqrt_threshold(double r) {
+  double t = r * r;
+  if (!(r > 0) || !std::isfinite(t)) return r > 0 ? t : 0.0;
+  while (t > 0 && std::sqrt(t) >= r) t = std::nextafter(t, 0.0);
+  while (std::sqrt(t) < r) t = std::nextafter(t, std::numeric_limits<double>::infinity());
+  return t;
+}
+
 int64_t ceil_div08(int64_t v) { return int64_t(std::ceil(double(v) / 0.8)); }
 
 }  // namespace
@@ -370,7 +381,11 @@ struct sph_s {
     C.fb_d[1] = p[SPH_BOUND_D];
     C.fb_r0[1] = p[SPH_BOUND_L];
     for (int k = 0; k < 2; ++k) C.fb_eta2[k] = 0.01 * (C.fb_r0[k] * C.fb_r0[k]);
+    for (int k = 0; k < 2; ++k) C.fb_t2[k] = sqrt_threshold(C.fb_r0[k]);
     C.st_2h = 2 * C.h;
+    C.st_t2 = sqrt_threshold(C.st_2h);
+    C.st_pi = 1.5 / C.st_2h;
+    C.dwr = -20.0 * C.dwnorm * C.Hinv;
     C.st_c = 1.5 * M_PI;
     C.st_01h = 0.1 * C.h;
     C.dpc_l0 = p[SPH_DPC_L0];
@@ -719,8 +734,10 @@ void run_steps(sph_s* const* P, unsigned count, LaunchSet& L, hipStream_t st, in
   std::vector<SceneDev<R>> descs(count);
   std::vector<StepFlags> flags(count);
   bool any_dpc = false, any_xsph = false, any_dtv = false;
+  L.gamma7 = true;
   for (unsigned i = 0; i < count; ++i) {
     sph_s* p = P[i];
+    L.gamma7 &= p->par[SPH_GAMMA] == 7;
     SphBufs<R>& B = p->bufs<R>();
     p->diag_pending = false;  // replaced by this call's
     p->ensure_nmask(B);
@@ -874,7 +891,7 @@ void run_steps(sph_s* const* P, unsigned count, LaunchSet& L, hipStream_t st, in
     // steps.  Kept for the next call while the launches, pass variants and
     // one-problem descriptor (baked into the graph) are unchanged.
     std::vector<unsigned char> key = {uint8_t(any_dpc), uint8_t(any_xsph), uint8_t(any_cspmn), uint8_t(any_dtv),
-                                      uint8_t(pv[0]), uint8_t(pv[1])};
+                                      uint8_t(pv[0]), uint8_t(pv[1]), uint8_t(L.gamma7)};
     if (L.one) {
       const unsigned char* d = static_cast<const unsigned char*>(L.one);
       key.insert(key.end(), d, d + sizeof(SceneDev<R>));

@@ -25,6 +25,10 @@ struct SphConst {
   double fb_d[2], fb_r0[2], fb_eta2[2];  // fbmolforce (0.4, 2dx) / (bound_D, bound_l); η² = 0.01 r0^2
   double st_2h, st_c, st_01h;            // 2h, 1.5π, 0.1h       :1393-1394
   double dpc_l0, dpc_l0inv, dpc_eta2, dpc_whinv, dpc_lim, dpc_wnorm, dpc_lambda, dpc_pmin, dpc_pmax;
+  double fb_t2[2];      // r < fb_r0 as a test of r²: r² < fb_t2, the smallest double whose square root is >= fb_r0
+  double st_t2;         // the same for r < 2h
+  double st_pi;         // 1.5π r/2h = π·r·st_pi
+  double dwr;           // dW/dr / r = dwr (1-u)^3: -20 dwnorm H⁻¹
   double xsph_c;        // 2m0 ε                   :1766
   double dt_eta2;       // (0.01h)^2               :1298
   double CFL, nui, tl0, tl1;
@@ -194,12 +198,15 @@ static_assert(sizeof(PartnerHX<2>) == 48 && sizeof(PartnerHX<3>) == 48, "partner
 // FP64 path: the pressure is stored (its EOS costs an FP64 division and a
 // power per partner), and pass 2's record always carries xⁿ (an FP64-exact
 // tⁿ separation cannot be derived from the half-step state).
+// They also store 1/ρ, which every pair divides by, where the record has the
+// room (all but the 3D half-step record, which a seventh word would widen).
 template <int D>
 struct alignas(16) PartnerN64 {
   double x[D];
   double v[D];
   double rho;
   double P;
+  double irho;  // 1/ρ
   int32_t pt;
 };
 template <int D>
@@ -207,6 +214,16 @@ struct alignas(16) PartnerH64 {
   double xn[D];
   double xh[D];
   double vh[D];
+  double rh;
+  double P;
+  double irh;  // 1/ρ½
+  int32_t pt;
+};
+template <>
+struct alignas(16) PartnerH64<3> {
+  double xn[3];
+  double xh[3];
+  double vh[3];
   double rh;
   double P;
   int32_t pt;
@@ -281,6 +298,7 @@ struct LaunchSet {
   int2* cmap = nullptr;
   int2* pmap512 = nullptr;
   unsigned pblocks = 0, ctiles = 0, count = 0, pblocks512 = 0;
+  bool gamma7 = true;  // γ = 7 in every problem (the FP64 passes have kernels for it)
   size_t scene_bytes = 0;
   // pass variants chosen by timing (-1: not yet)
   int pass_variant[2] = {-1, -1};

@@ -34,7 +34,7 @@ __device__ __forceinline__ double pf7(double x, int gamma, double ginv) {
     unsigned long long bits = (unsigned long long)__double_as_longlong(fabs(x));
     unsigned long long tb = 0x36cd000000000000ull + bits / 7ull;
     double t = copysign(__longlong_as_double((long long)tb), x);
-#pragma unroll
+#pragma unroll 1
     for (int it = 0; it < 2; ++it) {
       double t2 = t * t;
       double t3 = t2 * t;
@@ -87,6 +87,120 @@ __device__ __forceinline__ float dW_f(float u, float dwnorm) {
 __device__ __forceinline__ float dWr_f(float u, float dwr) {
   const float um1 = 1.0f - u;
   return u < 1.0f ? dwr * (um1 * um1 * um1) : 0.0f;
+}
+
+// FP64 pair arithmetic.  A pair of the Float64 path once cost ten IEEE
+// divisions (11 instructions each), a square root (~18) and powfancy7th: ~330
+// VALU instructions, and the passes were bound by them.  Here the divisions
+// share one reciprocal, 1/ρ comes with the partner's record, ∇W needs no
+// 1/r (dW/dr / r is a polynomial of r) and the hydrostatic term is its series.
+
+// 1/x, and sqrt(x) with sqrt(0) = 0: the hardware seed and Newton steps, to
+// about an ulp for normal x away from the ends of the FP64 range.
+__device__ __forceinline__ double rcp_d(double x) {
+  double r = __builtin_amdgcn_rcp(x);
+  r = __builtin_fma(__builtin_fma(-x, r, 1.0), r, r);
+  return __builtin_fma(__builtin_fma(-x, r, 1.0), r, r);
+}
+__device__ __forceinline__ double sqrt_d(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  double s = x * y, h = 0.5 * y;
+  const double e = __builtin_fma(-h, s, 0.5);
+  s = __builtin_fma(s, e, s);
+  h = __builtin_fma(h, e, h);
+  s = __builtin_fma(__builtin_fma(-s, s, x), h, s);
+  return x == 0.0 ? 0.0 : s;
+}
+// (dW/dr)/r at distance r, i.e. ∇W = dx · dWr_d (u/r = 1/H).  NaN for
+// coincident particles, as the reference's dW/r.
+__device__ __forceinline__ double dWr_d(double r2, double r, const SphConst& C) {
+  const double um1 = 1.0 - r * C.Hinv;
+  const double w = um1 > 0.0 ? C.dwr * (um1 * um1 * um1) : 0.0;
+  return r2 != 0.0 ? w : __builtin_nan("");
+}
+// ρ0·(powfancy7th(1+z) - 1) of the δ-SPH term.  powfancy7th stops two Halley
+// steps after a guess from the bit pattern, 3.87e-13 below the root near 1 (an
+// offset linear in z on either side of 0); that times ρ0 and the stiffness of
+// the term shows in ∂ρ/∂t, so results agree with the reference's only if it is
+// kept.  γ = 7 (G7), |z| < 2^-8 (z is ~1e-3 at most between partners of the
+// scenes here): the binomial series of the root plus that offset, within
+// 4e-16 of powfancy7th's real-number value (its own rounding is 2e-16) and
+// without its four divisions.  Other γ take pow, in kernels of their own: its
+// registers cost the γ = 7 kernels a wave per SIMD.
+template <bool G7>
+__device__ __forceinline__ double hydro_drho_d(double z, const SphConst& C) {
+  if constexpr (G7) {
+    if (fabs(z) < 0x1p-8) {
+      double t = __builtin_fma(z, 81549.0 / 5764801.0, -1989.0 / 117649.0);
+      t = __builtin_fma(z, t, 351.0 / 16807.0);
+      t = __builtin_fma(z, t, -65.0 / 2401.0);
+      t = __builtin_fma(z, t, 13.0 / 343.0);
+      t = __builtin_fma(z, t, -3.0 / 49.0);
+      t = __builtin_fma(z, t, 1.0 / 7.0 - 5.43e-12);
+      return C.rho0 * __builtin_fma(z, t, __builtin_fma(fabs(z), -5.84e-12, -3.8692e-13));
+    }
+    return C.rho0 * pf7(1 + z, 7, C.ginv) - C.rho0;
+  } else {
+    if (C.gamma == 7) return hydro_drho_d<true>(z, C);  // beside other γ in a batch
+    return C.rho0 * pf7(1 + z, C.gamma, C.ginv) - C.rho0;
+  }
+}
+// 1/ρb, 1/(ρa + ρb) and 1/(r² + η²) of a pair from one reciprocal; 1/ρb from
+// the record where it is stored.
+struct Inv3 {
+  double rhob, sum, den;
+};
+__device__ __forceinline__ Inv3 inv_stored(double irhob, double sum, double den) {
+  const double r = rcp_d(sum * den);
+  return {irhob, r * den, r * sum};
+}
+__device__ __forceinline__ Inv3 inv_all(double rhob, double sum, double den) {
+  const double bs = rhob * sum, r = rcp_d(bs * den), rd = r * den;
+  return {rd * sum, rd * rhob, r * bs};
+}
+template <int D>
+__device__ __forceinline__ Inv3 pair_inv(const PartnerN64<D>& q, double sum, double den) {
+  return inv_stored(q.irho, sum, den);
+}
+template <int D>
+__device__ __forceinline__ Inv3 pair_inv(const PartnerH64<D>& q, double sum, double den) {
+  return inv_stored(q.irh, sum, den);
+}
+__device__ __forceinline__ Inv3 pair_inv(const PartnerH64<3>& q, double sum, double den) {
+  return inv_all(q.rh, sum, den);
+}
+template <int D>
+__device__ __forceinline__ void set_irho(PartnerN64<D>& q) {
+  q.irho = 1.0 / q.rho;
+}
+template <int D>
+__device__ __forceinline__ void set_irho(PartnerH64<D>& q) {
+  q.irh = 1.0 / q.rh;
+}
+__device__ __forceinline__ void set_irho(PartnerH64<3>&) {}
+// sin(πs), |s| <= 1/2: its Taylor series (the first term dropped is below 2^-59)
+__device__ __forceinline__ double sinpi_d(double s) {
+  constexpr double p = 3.14159265358979323846, p2 = p * p;
+  constexpr double c3 = p * p2 / 6, c5 = c3 * p2 / 20, c7 = c5 * p2 / 42, c9 = c7 * p2 / 72, c11 = c9 * p2 / 110,
+                   c13 = c11 * p2 / 156, c15 = c13 * p2 / 210, c17 = c15 * p2 / 272, c19 = c17 * p2 / 342,
+                   c21 = c19 * p2 / 420;
+  const double w = s * s;
+  double t = __builtin_fma(w, c21, -c19);
+  t = __builtin_fma(w, t, c17);
+  t = __builtin_fma(w, t, -c15);
+  t = __builtin_fma(w, t, c13);
+  t = __builtin_fma(w, t, -c11);
+  t = __builtin_fma(w, t, c9);
+  t = __builtin_fma(w, t, -c7);
+  t = __builtin_fma(w, t, c5);
+  t = __builtin_fma(w, t, -c3);
+  return s * __builtin_fma(w, t, p);
+}
+// ∂v∂tpF! coefficient s·cos(1.5π r/2h)/(r + 0.1h) for r < 2h:
+// cos(πy) = -sin(π(y - 1/2)), y in [0, 1.5), folded into [-1/2, 1/2]
+__device__ __forceinline__ double surf_d(double r, const SphConst& C) {
+  const double y = r * C.st_pi;
+  return -C.s * sinpi_d(y > 1.0 ? 1.5 - y : y - 0.5) * rcp_d(r + C.st_01h);
 }
 
 // Tait EOS (src/gpukernels_sph.jl:691-697): 0 if ptype <= 1 and ρ < ρ0.
@@ -165,6 +279,13 @@ __device__ __forceinline__ double dotd(const double* a, const double* b) {
 #pragma clang fp contract(off)
   double s = a[0] * b[0] + a[1] * b[1];
   if (D == 3) s = s + a[2] * b[2];
+  return s;
+}
+// dotd with fused multiply-adds, where no comparison reads it
+template <int D>
+__device__ __forceinline__ double dotm(const double* a, const double* b) {
+  double s = __builtin_fma(a[1], b[1], a[0] * b[0]);
+  if (D == 3) s = __builtin_fma(a[2], b[2], s);
   return s;
 }
 template <int D>

@@ -378,6 +378,7 @@ __device__ __forceinline__ void reorder_one(const SphBufs<R>& B, const SphConst&
     B.PN[s] = P;
     rec.P = P;
     rec.pt = pt;
+    set_irho(rec);
   } else {
     const float P = eos_f(rv, pt, C);
     B.PN[s] = P;
@@ -819,6 +820,7 @@ __global__ void k_cspm_apply(SS ss) {
     N rec = ld_rec<N>(B.PRN, a, B.n);
     rec.rho = nr;
     rec.P = P;
+    set_irho(rec);
     st_rec(B.PRN, a, rec, B.n);
   } else {
     const float d = float(nr);

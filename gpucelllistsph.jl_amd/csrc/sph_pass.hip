@@ -16,9 +16,14 @@
 // evaluation with symplectic_update! and the Δt / rebuild reductions
 // (src/sphproblem.jl:277-335).
 //
-// R = double: the Float64 path.  Every expression is evaluated in the
-// reference's operation order with FMA contraction off, so branch decisions
-// (r < r0, cond < 0, clamps) see the same values as the reference would.
+// R = double: the Float64 path.  Squared distances, the branch decisions (r < r0
+// as a test of r², clamps) and the updates are evaluated in the reference's
+// operation order with FMA contraction off, so they see the same values as the
+// reference would.  The pair terms are the reference's to a few ulp: their ten
+// divisions, square roots and powfancy7th are the arithmetic of sph_device.hpp
+// (~85 VALU instructions per pair, ~330 as written; the passes are bound by
+// VALU issue).  1.02 M particles in 2D: a step 0.77 -> 0.50 ms; 191 k in 3D:
+// 1.45x per call.
 // R = float: the FP32-split path (density stored as ρ-ρ0, FP32 pair terms
 // summed in FP64, Float64 positions and Δt).
 #include <atomic>
@@ -35,7 +40,7 @@ namespace gclsph {
 // picks one per pass by timing them on live steps.
 //
 // ---- pass 1 ---------------------------------------------------------------
-template <int D, typename R, typename SS, bool Pipe, int W, int BS>
+template <int D, typename R, typename SS, bool Pipe, int W, int BS, bool G7>
 __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W))) void k_pass1(SS ss) {
 #pragma clang fp contract(off)
   GCLSPH_SCENE_BS(ss, BS);
@@ -64,61 +69,54 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W))) void k_
   const int nc = B.NC[a];
   if constexpr (std::is_same<R, double>::value) {
     const double rhoa = sa;
+    const double mPa = -C.m0 * (1.0 / rhoa);  // -m0/ρ_a of the pressure term
     const double Pa = B.PN[a];
     using Nb = PartnerN64<D>;
     auto fetch = [&](const int32_t b) { return ld_rec<Nb>(B.PRN, b, B.n); };
+    // ∇W = dx·dwr: terms along ∇W are gathered into one coefficient fg of dx,
+    // dx·∇W = r²·dwr, dv·∇W = (dv·dx)·dwr
     for_each_partner_fetch<Pipe, D>(B, a, nc, G, XM, C.dist2, fetch, [&](const int32_t, const Nb& q) {
+#pragma clang fp contract(fast)
       const int32_t ptb = q.pt;
-      double dx[3], dv[3], gw[3];
+      double dx[3], dv[3];
 #pragma unroll
       for (int d = 0; d < D; ++d) {
         dx[d] = xa[d] - q.x[d];
         dv[d] = va[d] - q.v[d];
       }
-      const double r2 = dotd<D>(dx, dx);
-      const double r = sqrt(r2);
-      const double u = r * C.Hinv;
-      const double dwk_r = dW_d(u, C.dwnorm) / r;
-#pragma unroll
-      for (int d = 0; d < D; ++d) gw[d] = dx[d] * dwk_r;
+      const double r2 = dotd<D>(dx, dx);  // unfused: the cut-offs below compare it
+      const double r = sqrt_d(r2);
+      const double dwr = dWr_d(r2, r, C);
       const double rhob = q.rho;
+      const Inv3 iv = pair_inv(q, rhoa + rhob, r2 + C.eta2);
+      const double dvdx = dotm<D>(dv, dx);
+      // the common terms are evaluated for every pair and selected
       const bool both = pta > 0 && ptb > 0;
+      {  // ∂ρ∂tDDT! (:579-625)
+        const double s = C.m0 * dwr * dvdx;
+        const double vd = C.DDTkh * ((rhob - rhoa) - hydro_drho_d<G7>(C.DDTgz * dx[1], C)) * iv.den;
+        const double sd = s - vd * (r2 * dwr) * (C.m0 * iv.rhob);
+        drho.add(both ? (pta > 1 ? sd : s) : 0.0);
+      }
+      double fg = (Pa + q.P) * iv.rhob * mPa;  // ∂v∂t! (:755-772)
+      {                                        // ∂v∂t_av! (:869-897), on approaching pairs
+        const double dmu = C.h * fmin(dvdx, 0.0) * iv.den;
+        const double dPi = (-C.alpha * C.c0 * dmu) * (2.0 * iv.sum);
+        fg -= both ? dPi * C.m0 : 0.0;
+      }
+      fg = same_kind(pta, ptb) ? fg * dwr : 0.0;
       double ax[3] = {0.0, 0.0, 0.0};
-      if (both) {  // ∂ρ∂tDDT! (:579-625)
-        double dot3 = -dotd<D>(dx, gw);
-        double s = C.m0 * dotd<D>(dv, gw);
-        if (pta > 1) {
-          double drhop = C.rho0 * pf7(1 + C.DDTgz * dx[1], C.gamma, C.ginv) - C.rho0;
-          double vd = C.DDTkh * (rhob - rhoa - drhop) / (r2 + C.eta2);
-          s += vd * dot3 * C.m0 / rhob;
-        }
-        drho.add(s);
-      }
-      if (same_kind(pta, ptb)) {  // ∂v∂t! (:755-772)
-        double Pfac = (Pa + q.P) / (rhoa * rhob);
-#pragma unroll
-        for (int d = 0; d < D; ++d) ax[d] += -C.m0 * Pfac * gw[d];
-      }
-      if (both) {  // ∂v∂t_av! (:869-897)
-        double cond = dotd<D>(dv, dx);
-        if (cond < 0) {
-          double dmu = C.h * cond / (r2 + C.eta2);
-          double dPi = (-C.alpha * C.c0 * dmu) / ((rhoa + rhob) * 0.5);
-#pragma unroll
-          for (int d = 0; d < D; ++d) ax[d] += -dPi * C.m0 * gw[d];
-        }
+      if (both) {
         if (F.nu_on) {  // ∂v∂t_visc! (:967-980)
-          double term = 4 * C.nu * C.m0 * dotd<D>(dx, gw) / ((rhoa + rhob) * (r2 + C.eta2));
+          const double term = 4 * C.nu * C.m0 * (r2 * dwr) * (iv.sum * iv.den);
 #pragma unroll
           for (int d = 0; d < D; ++d) ax[d] += term * dv[d];
         }
-        if (F.s_on && r < C.st_2h) {  // ∂v∂tpF! (:1387-1397)
-          double scos = C.s * cos(C.st_c * r / C.st_2h) / (r + C.st_01h);
-#pragma unroll
-          for (int d = 0; d < D; ++d) ax[d] += scos * dx[d] / C.m0;
-        }
+        if (F.s_on && r2 < C.st_t2) fg += surf_d(r, C) * (1.0 / C.m0);  // ∂v∂tpF! (:1387-1397)
       }
-      if ((pta > 0) != (ptb > 0) && r < C.fb_r0[0]) {  // fbmolforce! (:1891-1901)
+#pragma unroll
+      for (int d = 0; d < D; ++d) ax[d] += fg * dx[d];
+      if ((pta > 0) != (ptb > 0) && r2 < C.fb_t2[0]) {  // fbmolforce! (:1891-1901)
         double q1 = C.fb_r0[0] / (r + C.fb_eta2[0]);
         double Fc = C.fb_d[0] * (powi_d(q1, 12) - powi_d(q1, 4)) / (r2 + C.fb_eta2[0]);
 #pragma unroll
@@ -170,6 +168,7 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W))) void k_
     rec.rh = rv;
     rec.P = Ph;
     rec.pt = pta;
+    set_irho(rec);
     st_rec(B.PRH, a, rec, B.n);
   } else {
     // ---------------- FP32-split
@@ -300,7 +299,7 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W))) void k_
 }
 
 // ---- pass 2 + symplectic update ------------------------------------------
-template <int D, typename R, typename SS, bool Pipe, int W, int BS>
+template <int D, typename R, typename SS, bool Pipe, int W, int BS, bool G7>
 __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W))) void k_pass2(SS ss) {
 #pragma clang fp contract(off)
   GCLSPH_SCENE_BS(ss, BS);
@@ -333,67 +332,60 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W))) void k_
     R Pha, drho_v;
     if constexpr (std::is_same<R, double>::value) {
       const double rhoa = sha;
+      const double mPa = -C.m0 * (1.0 / rhoa);
       Pha = B.PH[a];
       using Nb = PartnerH64<D>;
       auto fetch = [&](const int32_t b) { return ld_rec<Nb>(B.PRH, b, B.n); };
       for_each_partner_fetch<Pipe, D>(B, a, nc, G, XM, C.dist2, fetch, [&](const int32_t, const Nb& q) {
+#pragma clang fp contract(fast)
         const int32_t ptb = q.pt;
-        double dxn[3], dx[3], dv[3], gw[3];
+        double dxn[3], dx[3], dv[3];
 #pragma unroll
         for (int d = 0; d < D; ++d) {
           dxn[d] = xa[d] - q.xn[d];
           dx[d] = xha[d] - q.xh[d];
           dv[d] = vha[d] - q.vh[d];
         }
-        // ∇W from pass 1 (positions xⁿ, src/sphproblem.jl:246,281)
+        // ∇W from pass 1 (positions xⁿ, src/sphproblem.jl:246,281): dxn·dwr
         const double r2n = dotd<D>(dxn, dxn);
-        const double rn = sqrt(r2n);
-        const double dwk_r = dW_d(rn * C.Hinv, C.dwnorm) / rn;
-#pragma unroll
-        for (int d = 0; d < D; ++d) gw[d] = dxn[d] * dwk_r;
+        const double rn = sqrt_d(r2n);
+        const double dwr = dWr_d(r2n, rn, C);
         const double r2 = dotd<D>(dx, dx);
         const double rhob = q.rh;
+        const Inv3 iv = pair_inv(q, rhoa + rhob, r2 + C.eta2);
+        const double dvdx = dotm<D>(dv, dx);
+        const double dxg = dotm<D>(dx, dxn) * dwr;  // dx·∇W
         const bool both = pta > 0 && ptb > 0;
+        {
+          const double s = C.m0 * dwr * dotm<D>(dv, dxn);
+          const double vd = C.DDTkh * ((rhob - rhoa) - hydro_drho_d<G7>(C.DDTgz * dx[1], C)) * iv.den;
+          const double sd = s - vd * dxg * (C.m0 * iv.rhob);
+          drho.add(both ? (pta > 1 ? sd : s) : 0.0);
+        }
+        double fg = (Pha + q.P) * iv.rhob * mPa;
+        {
+          const double dmu = C.h * fmin(dvdx, 0.0) * iv.den;
+          const double dPi = (-C.alpha * C.c0 * dmu) * (2.0 * iv.sum);
+          fg -= both ? dPi * C.m0 : 0.0;
+        }
+        fg = same_kind(pta, ptb) ? fg * dwr : 0.0;
         double ax[3] = {0.0, 0.0, 0.0};
         if (both) {
-          double dot3 = -dotd<D>(dx, gw);
-          double s = C.m0 * dotd<D>(dv, gw);
-          if (pta > 1) {
-            double drhop = C.rho0 * pf7(1 + C.DDTgz * dx[1], C.gamma, C.ginv) - C.rho0;
-            double vd = C.DDTkh * (rhob - rhoa - drhop) / (r2 + C.eta2);
-            s += vd * dot3 * C.m0 / rhob;
-          }
-          drho.add(s);
-        }
-        if (same_kind(pta, ptb)) {
-          double Pfac = (Pha + q.P) / (rhoa * rhob);
-#pragma unroll
-          for (int d = 0; d < D; ++d) ax[d] += -C.m0 * Pfac * gw[d];
-        }
-        if (both) {
-          double cond = dotd<D>(dv, dx);
-          if (cond < 0) {
-            double dmu = C.h * cond / (r2 + C.eta2);
-            double dPi = (-C.alpha * C.c0 * dmu) / ((rhoa + rhob) * 0.5);
-#pragma unroll
-            for (int d = 0; d < D; ++d) ax[d] += -dPi * C.m0 * gw[d];
-          }
           if (F.nu_on) {
-            double term = 4 * C.nu * C.m0 * dotd<D>(dx, gw) / ((rhoa + rhob) * (r2 + C.eta2));
+            const double term = 4 * C.nu * C.m0 * dxg * (iv.sum * iv.den);
 #pragma unroll
             for (int d = 0; d < D; ++d) ax[d] += term * dv[d];
           }
-          if (F.s_on) {
-            double r = sqrt(r2);
-            if (r < C.st_2h) {
-              double scos = C.s * cos(C.st_c * r / C.st_2h) / (r + C.st_01h);
+          if (F.s_on && r2 < C.st_t2) {
+            const double scos = surf_d(sqrt_d(r2), C) * (1.0 / C.m0);
 #pragma unroll
-              for (int d = 0; d < D; ++d) ax[d] += scos * dx[d] / C.m0;
-            }
+            for (int d = 0; d < D; ++d) ax[d] += scos * dx[d];
           }
         }
+#pragma unroll
+        for (int d = 0; d < D; ++d) ax[d] += fg * dxn[d];
         // fbmolforce! at xⁿ with (bound_D, bound_l) (src/sphproblem.jl:295)
-        if ((pta > 0) != (ptb > 0) && rn < C.fb_r0[1]) {
+        if ((pta > 0) != (ptb > 0) && r2n < C.fb_t2[1]) {
           double q1 = C.fb_r0[1] / (rn + C.fb_eta2[1]);
           double Fc = C.fb_d[1] * (powi_d(q1, 12) - powi_d(q1, 4)) / (r2n + C.fb_eta2[1]);
 #pragma unroll
@@ -443,6 +435,7 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W))) void k_
       rec.rho = rv;
       rec.P = Pn;
       rec.pt = pta;
+      set_irho(rec);
       st_rec(B.PRN, a, rec, B.n);  // partner record of the next step's pass 1
       if (F.ts) {
         red_acc = sqrt(dotd<D>(av, av));
@@ -628,13 +621,17 @@ template <int BS>
 unsigned pass_grid(const LaunchSet& L) {
   return BS == 256 ? L.pblocks : BS == 128 ? 2 * L.pblocks : L.pblocks512;
 }
-template <int D, typename R, bool Pipe, int W, int BS>
+template <int D, typename R, bool Pipe, int W, int BS, bool G7 = true>
 void pass1_as(const LaunchSet& L, hipStream_t s, size_t lds) {
-  with_scenes<R>(L, [&](auto ss) { k_pass1<D, R, decltype(ss), Pipe, W, BS><<<pass_grid<BS>(L), BS, lds, s>>>(ss); });
+  with_scenes<R>(L, [&](auto ss) {
+    k_pass1<D, R, decltype(ss), Pipe, W, BS, G7><<<pass_grid<BS>(L), BS, lds, s>>>(ss);
+  });
 }
-template <int D, typename R, bool Pipe, int W, int BS>
+template <int D, typename R, bool Pipe, int W, int BS, bool G7 = true>
 void pass2_as(const LaunchSet& L, hipStream_t s, size_t lds) {
-  with_scenes<R>(L, [&](auto ss) { k_pass2<D, R, decltype(ss), Pipe, W, BS><<<pass_grid<BS>(L), BS, lds, s>>>(ss); });
+  with_scenes<R>(L, [&](auto ss) {
+    k_pass2<D, R, decltype(ss), Pipe, W, BS, G7><<<pass_grid<BS>(L), BS, lds, s>>>(ss);
+  });
 }
 // Unused dynamic LDS per block of BS threads that leaves room for at most
 // kPassCapWaves waves per SIMD (B = 4·kPassCapWaves·64/BS blocks per CU: B
@@ -683,6 +680,12 @@ void pass2_cg(const LaunchSet& L, hipStream_t s, int cg, size_t lds) {
 // 1: 128, 2: 512 threads per block; oc 1: occupancy cap)
 template <int D, typename R>
 void launch_pass1(const LaunchSet& L, hipStream_t s, int variant) {
+  if constexpr (std::is_same<R, double>::value) {
+    if (!L.gamma7) {  // another γ: one kernel, whatever the variant
+      pass1_as<D, R, false, 1, 256, false>(L, s, 0);
+      return;
+    }
+  }
   const int cg = variant % kPassCodegen, bs = pass_block_size(variant);
   const size_t lds = pass_cap(variant) ? cap_lds(bs) : 0;
   switch (bs) {
@@ -693,6 +696,12 @@ void launch_pass1(const LaunchSet& L, hipStream_t s, int variant) {
 }
 template <int D, typename R>
 void launch_pass2(const LaunchSet& L, hipStream_t s, int variant) {
+  if constexpr (std::is_same<R, double>::value) {
+    if (!L.gamma7) {  // another γ: one kernel, whatever the variant
+      pass2_as<D, R, false, 1, 256, false>(L, s, 0);
+      return;
+    }
+  }
   const int cg = variant % kPassCodegen, bs = pass_block_size(variant);
   const size_t lds = pass_cap(variant) ? cap_lds(bs) : 0;
   switch (bs) {

@@ -75,6 +75,23 @@ def test_batch_3d_and_single_steps_interleaved(G, S):
             assert np.array_equal(f[name], r[name]), name
 
 
+def test_batch_of_uneven_gamma_matches_one_by_one(G, S):
+    """γ = 7 beside another γ in a Float64 batch takes the kernels of general γ:
+    the same steps as alone, bit for bit."""
+    scs = [golden_cases()["dam2d"][0], S.dam_break_2d(0.05, 0.5, 1.0, 2.0, 1.5)]
+    scs[1].params.gamma = 5
+    alone, probs = [make(G, sc, "f64") for sc in scs], [make(G, sc, "f64") for sc in scs]
+    batch = G.SPHBatch(probs)
+    for n in (1, 3):
+        for p in alone:
+            G.stepsolve_(p, n, timestepping=True)
+        G.batch_stepsolve_(batch, n, timestepping=True)
+    for a, b in zip(alone, probs):
+        fa, fb = fields(G, a), fields(G, b)
+        for name in fa:
+            assert np.array_equal(fa[name], fb[name]), name
+
+
 def test_batch_argument_errors(G, S):
     sc = golden_cases()["dam2d"][0]
     a, b = make(G, sc, "f64"), make(G, sc, "f32split")

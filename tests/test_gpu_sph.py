@@ -320,6 +320,27 @@ def test_gamma_other_than_7(G, O, S):
         G.SPHProblem.from_params(cl2, sc.params, sc.rho, sc.ptype, precision="f32split")
 
 
+@pytest.mark.parametrize("c0", [88.6, 47.0, 46.0, 20.0])
+def test_f64_hydrostatic_term_ranges(G, O, S, c0):
+    """The δ-SPH hydrostatic term of γ = 7 is a series while |ρ0 g Δy / Cb| < 2^-8
+    and powfancy7th beyond: sound speeds that keep every pair below the limit
+    (88.6: 1.5e-3), put the farthest pairs (Δy = 3 dx) beyond it and the nearer
+    ones below (47, 46), and most beyond it (20)."""
+    sc = S.dam_break_2d(0.05, 0.5, 1.0, 2.0, 1.5)
+    p = sc.params
+    p.c0 = c0
+    y = sc.points[1] + 0.05 * p.dx * (S.uniform01(3, sc.n, 0) - 0.5)
+    sc.points = (sc.points[0], y)
+    z = p.rho0 * p.g / (c0 * c0 * p.rho0 / 7) * p.H
+    assert (z < 2.0 ** -8) == (c0 == 88.6)
+    cl, oc, prob, ref = _pair(G, O, sc)
+    G.stepsolve_(prob, 3, timestepping=True)
+    ref.stepsolve(3, True)
+    got = gpu_fields(G, prob)
+    for f in ("x", "v", "rho", "P", "acc", "drho"):
+        assert rel_err(got[f], ref.get(f)) < TOL64[f], f
+
+
 def test_argument_errors(G, S):
     sc = S.dam_break_2d(0.05, 0.5, 1.0, 2.0, 1.5)
     cl = G.GPUCellList(sc.points, sc.cellsize, sc.dist)
