@@ -103,6 +103,21 @@ double sqrt_threshold(double r) {
   return t;
 }
 
+// Whether a set of n particles in all is stepped with a quad of lanes per
+// particle (same results): up to about where one lane per particle begins to
+// fill the chip.  Step time of one lane / of a quad: 2D FP32-split 1.35 at 1 k
+// to 14 k particles, 1.27 at 28 k, 1.13 at 54 k, 0.97 at 106 k; 2D FP64 1.38,
+// 1.27, 1.01, 0.91; 3D FP64 1.54 at 19 k, 1.17 at 54 k, 1.04 at 91 k, 0.96 at
+// 155 k; 3D FP32-split with every term 1.81, 1.33, 1.17, 0.99.
+// GCLSPH_PAIR_LANES=1|4 forces one of them.
+bool pair_quads(int64_t n, int dim, bool split) {
+  if (const char* env = std::getenv("GCLSPH_PAIR_LANES")) {
+    if (std::strcmp(env, "1") == 0) return false;
+    if (std::strcmp(env, "4") == 0) return true;
+  }
+  return n <= (dim == 2 ? (split ? 80000 : 50000) : (split ? 140000 : 110000));
+}
+
 int64_t ceil_div08(int64_t v) { return int64_t(std::ceil(double(v) / 0.8)); }
 
 }  // namespace
@@ -386,6 +401,8 @@ struct sph_s {
     C.st_t2 = sqrt_threshold(C.st_2h);
     C.st_pi = 1.5 / C.st_2h;
     C.dwr = -20.0 * C.dwnorm * C.Hinv;
+    C.av = 2 * C.alpha * C.c0 * C.h * C.m0;
+    C.nu4 = 4 * C.nu * C.m0;
     C.st_c = 1.5 * M_PI;
     C.st_01h = 0.1 * C.h;
     C.dpc_l0 = p[SPH_DPC_L0];
@@ -441,7 +458,8 @@ struct sph_s {
     C.f_dwnorm = float(C.dwnorm);
     C.f_inv_rho0 = float(1.0 / C.rho0);
     C.f_st_turn = float(C.st_c / (2.0 * M_PI * C.st_2h));
-    C.f_dwr = float(-20.0 * C.dwnorm * C.Hinv);
+    C.f_dwr = float(C.dwr);
+    C.f_inv_m0 = 1.0f / C.f_m0;
     for (int k = 0; k < 2; ++k) {
       C.f_fb_d[k] = float(C.fb_d[k]);
       C.f_fb_r0[k] = float(C.fb_r0[k]);
@@ -681,44 +699,49 @@ SphBufs<float>& sph_s::bufs<float>() {
   return Bf;
 }
 
-void LaunchSet::build(const int64_t* n, const int64_t* ncells, unsigned cnt, size_t bytes) {
+void LaunchSet::build(const int64_t* n, const int64_t* ncells, unsigned cnt, int dim, bool split, size_t bytes) {
   release();
   count = cnt;
   scene_bytes = bytes;
-  std::vector<int2> pm, cm, pm512;
+  std::vector<int2> pm, cm, pm512, qm;
+  auto blocks = [](std::vector<int2>& v, unsigned i, int64_t items, int64_t per) {
+    for (int64_t b = 0; b * per < items; ++b) v.push_back(make_int2(int(i), int(b)));
+  };
+  int64_t total = 0;
+  for (unsigned i = 0; i < cnt; ++i) total += n[i];
+  quad = pair_quads(total, dim, split);
   for (unsigned i = 0; i < cnt; ++i) {
-    const int64_t nb = (n[i] + kBlock - 1) / kBlock;
-    for (int64_t b = 0; b < nb; ++b) pm.push_back(make_int2(int(i), int(b)));
-    const int64_t nb512 = (n[i] + 511) / 512;  // the pass kernels' 512-thread blocks
-    for (int64_t b = 0; b < nb512; ++b) pm512.push_back(make_int2(int(i), int(b)));
-    const int64_t nt = (ncells[i] + 1 + 1023) / 1024;  // cnt[0..ncells] in 1024-cell tiles
-    for (int64_t t = 0; t < nt; ++t) cm.push_back(make_int2(int(i), int(t)));
+    blocks(pm, i, n[i], kBlock);
+    blocks(pm512, i, n[i], 512);  // the pass kernels' 512-thread blocks
+    if (quad) blocks(qm, i, n[i], 64);
+    blocks(cm, i, ncells[i] + 1, 1024);  // cnt[0..ncells] in 1024-cell tiles
   }
-  if (pm.empty()) pm.push_back(make_int2(0, 0));  // a no-op block (a >= n everywhere)
-  if (pm512.empty()) pm512.push_back(make_int2(0, 0));
+  for (auto* v : {&pm, &pm512, &qm})
+    if (v->empty()) v->push_back(make_int2(0, 0));  // a no-op block (a >= n everywhere)
   pblocks = unsigned(pm.size());
   pblocks512 = unsigned(pm512.size());
+  qblocks = unsigned(qm.size());
   ctiles = unsigned(cm.size());
   GCL_HIP(hipMalloc(&scenes, bytes * cnt));
-  GCL_HIP(hipMalloc(&pmap, sizeof(int2) * pm.size()));
-  GCL_HIP(hipMalloc(&pmap512, sizeof(int2) * pm512.size()));
-  GCL_HIP(hipMalloc(&cmap, sizeof(int2) * cm.size()));
-  GCL_HIP(hipMemcpy(pmap, pm.data(), sizeof(int2) * pm.size(), hipMemcpyHostToDevice));
-  GCL_HIP(hipMemcpy(pmap512, pm512.data(), sizeof(int2) * pm512.size(), hipMemcpyHostToDevice));
-  GCL_HIP(hipMemcpy(cmap, cm.data(), sizeof(int2) * cm.size(), hipMemcpyHostToDevice));
+  auto put = [](int2** dst, const std::vector<int2>& v) {
+    GCL_HIP(hipMalloc(dst, sizeof(int2) * v.size()));
+    GCL_HIP(hipMemcpy(*dst, v.data(), sizeof(int2) * v.size(), hipMemcpyHostToDevice));
+  };
+  put(&pmap, pm);
+  put(&pmap512, pm512);
+  put(&qmap, qm);
+  put(&cmap, cm);
 }
 
 void LaunchSet::release() {
   if (step_graph) (void)hipGraphExecDestroy(step_graph);
   step_graph = nullptr;
   graph_key.clear();
-  if (scenes) (void)hipFree(scenes);
-  if (pmap) (void)hipFree(pmap);
-  if (pmap512) (void)hipFree(pmap512);
-  if (cmap) (void)hipFree(cmap);
+  for (void* p : {scenes, (void*)pmap, (void*)cmap, (void*)pmap512, (void*)qmap})
+    if (p) (void)hipFree(p);
   scenes = nullptr;
-  pmap = cmap = pmap512 = nullptr;
-  pblocks = ctiles = count = pblocks512 = 0;
+  pmap = cmap = pmap512 = qmap = nullptr;
+  pblocks = ctiles = count = pblocks512 = qblocks = 0;
 }
 
 namespace {
@@ -789,7 +812,13 @@ void run_steps(sph_s* const* P, unsigned count, LaunchSet& L, hipStream_t st, in
       forced = true;
     }
   }
-  if (!forced && L.pass_variant[0] >= 0) {
+  const char* no_tune = std::getenv("GCLSPH_AUTOTUNE");
+  bool tune = !forced && L.pass_variant[0] < 0 && nsteps > kTuneTimed && !(no_tune && no_tune[0] == '0');
+  if (!forced && L.quad) {  // one shape, nothing to time; reported as variant 0, whose blocks it has
+    pv[0] = pv[1] = kPassQuad;
+    if (tune) L.pass_variant[0] = L.pass_variant[1] = 0;
+    tune = false;
+  } else if (!forced && L.pass_variant[0] >= 0) {
     pv[0] = L.pass_variant[0];
     pv[1] = L.pass_variant[1];
   }
@@ -815,8 +844,7 @@ void run_steps(sph_s* const* P, unsigned count, LaunchSet& L, hipStream_t st, in
     return any;
   };
   int64_t done = 0;
-  const char* no_tune = std::getenv("GCLSPH_AUTOTUNE");
-  if (!forced && L.pass_variant[0] < 0 && !timer && nsteps > kTuneTimed && !(no_tune && no_tune[0] == '0')) {
+  if (tune && !timer) {
     // Autotune on the first steps of the call (live steps: every variant
     // computes the same values).  Up to kTuneWarm untimed steps first, as
     // many as the call has beyond the kTuneTimed timed ones: the first dozen
@@ -1423,12 +1451,12 @@ int sph_create(gcl_t system, int prec, const double* params, const double* rho, 
       const SphConst C0 = P->make_const(0.0, 0.0);
       const StepFlags F0 = P->call_flags(false);
       if (prec == GCLSPH_F32SPLIT) {
-        P->own.build(&n, &nc, 1, sizeof(SceneDev<float>));
+        P->own.build(&n, &nc, 1, P->dim, true, sizeof(SceneDev<float>));
         P->upload_own<float>(C0, F0);
         if (P->dim == 2) launch_init_pn<2, float>(P->own, P->stream);
         else launch_init_pn<3, float>(P->own, P->stream);
       } else {
-        P->own.build(&n, &nc, 1, sizeof(SceneDev<double>));
+        P->own.build(&n, &nc, 1, P->dim, false, sizeof(SceneDev<double>));
         P->upload_own<double>(C0, F0);
         if (P->dim == 2) launch_init_pn<2, double>(P->own, P->stream);
         else launch_init_pn<3, double>(P->own, P->stream);
@@ -1608,7 +1636,7 @@ int sph_batch_create(const sph_t* problems, int32_t count, sph_batch_t* out) {
       nc[size_t(i)] = b->probs[size_t(i)]->G.ncells();
     }
     const size_t bytes = problems[0]->split() ? sizeof(SceneDev<float>) : sizeof(SceneDev<double>);
-    b->L.build(n.data(), nc.data(), unsigned(count), bytes);
+    b->L.build(n.data(), nc.data(), unsigned(count), problems[0]->dim, problems[0]->split(), bytes);
     *out = b.release();
   });
 }

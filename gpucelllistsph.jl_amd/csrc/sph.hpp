@@ -29,6 +29,8 @@ struct SphConst {
   double st_t2;         // the same for r < 2h
   double st_pi;         // 1.5π r/2h = π·r·st_pi
   double dwr;           // dW/dr / r = dwr (1-u)^3: -20 dwnorm H⁻¹
+  double av;            // 2 α c0 h m0: artificial viscosity coefficient of a pair
+  double nu4;           // 4 ν m0
   double xsph_c;        // 2m0 ε                   :1766
   double dt_eta2;       // (0.01h)^2               :1298
   double CFL, nui, tl0, tl1;
@@ -37,6 +39,7 @@ struct SphConst {
       f_dwnorm, f_fb_d[2], f_fb_r0[2], f_fb_eta2[2], f_st_2h, f_st_c, f_st_01h, f_xsph_c;
   float f_dpc_l0inv, f_dpc_eta2, f_dpc_whinv, f_dpc_lim, f_dpc_wnorm, f_dpc_lambda, f_dpc_pmin, f_dpc_pmax;
   float f_inv_rho0;  // 1/ρ0
+  float f_inv_m0;    // 1/m0
   float f_st_turn;   // 1.5π/(2h) in turns: cos(1.5π r/2h) = cos(2π · r·f_st_turn)
   float f_dwr;       // dW/dr / r = f_dwr (1-u)^3: -20 dwnorm H⁻¹
   double fcs[3];     // cell-frame spacing of the 3D FP32-split partner records: the
@@ -288,7 +291,8 @@ struct SceneDev {
 // problem is a batch of one).  Particle kernels run one block per 256 particles
 // of one problem; pmap maps a logical block to (problem, block of the problem);
 // pmap512 does the same for the 512-thread blocks of the pass kernels (their
-// 128-thread blocks halve the pmap entries).
+// 128-thread blocks halve the pmap entries), and qmap for the pair kernels' blocks
+// of 64 particles with a quad of lanes each.
 // Cell kernels run one block per 1024-cell tile; cmap maps a block to (problem,
 // tile).  Per-problem kernels run one block per problem.
 struct LaunchSet {
@@ -297,7 +301,9 @@ struct LaunchSet {
   int2* pmap = nullptr;
   int2* cmap = nullptr;
   int2* pmap512 = nullptr;
-  unsigned pblocks = 0, ctiles = 0, count = 0, pblocks512 = 0;
+  int2* qmap = nullptr;
+  unsigned pblocks = 0, ctiles = 0, count = 0, pblocks512 = 0, qblocks = 0;
+  bool quad = false;  // the pair kernels run a quad of lanes per particle
   bool gamma7 = true;  // γ = 7 in every problem (the FP64 passes have kernels for it)
   size_t scene_bytes = 0;
   // pass variants chosen by timing (-1: not yet)
@@ -306,7 +312,7 @@ struct LaunchSet {
   hipGraphExec_t step_graph = nullptr;
   std::vector<unsigned char> graph_key;
   // n[i] particles and ncells[i] cells of problem i
-  void build(const int64_t* n, const int64_t* ncells, unsigned count, size_t scene_bytes);
+  void build(const int64_t* n, const int64_t* ncells, unsigned count, int dim, bool split, size_t scene_bytes);
   void release();
 };
 
@@ -324,6 +330,8 @@ constexpr int kPassBlockSizes = 3;
 constexpr int kPassCaps = 2;
 constexpr int kPassCapWaves = 4;
 constexpr int kPassVariants = kPassCodegen * kPassBlockSizes * kPassCaps;
+// A quad of lanes per particle (sum_partners), for sets LaunchSet::quad marks.
+constexpr int kPassQuad = kPassVariants;
 // Steps the autotuner times: every code-generation variant at every block
 // size (the best shape at one block size need not be the best at another),
 // then the best of them with the cap and the two best once more; before them

@@ -67,26 +67,19 @@ __device__ __forceinline__ double dW_d(double u, double dwnorm) {
   }
   return 0.0;
 }
-__device__ __forceinline__ float W_f(float u, float wnorm) {
+// The FP32 pair arithmetic names its fused multiply-adds: every kernel that
+// evaluates a pair (and every copy of a pair body in an unrolled loop) then
+// rounds alike, which contraction by the compiler does not promise.
+__device__ __forceinline__ float W_f(float r, float Hinv, float wnorm) {
+#pragma clang fp contract(off)
+  const float u = r * Hinv;
   if (u < 1.0f) {
-    float um1 = 1.0f - u;
+    float um1 = __builtin_fmaf(-r, Hinv, 1.0f);
     um1 = um1 * um1;
     um1 = um1 * um1;
-    return ((1.0f + 4.0f * u) * um1) * wnorm;
+    return (__builtin_fmaf(4.0f, u, 1.0f) * um1) * wnorm;
   }
   return 0.0f;
-}
-__device__ __forceinline__ float dW_f(float u, float dwnorm) {
-  if (u < 1.0f) {
-    float um1 = 1.0f - u;
-    return -20.0f * u * (um1 * um1 * um1) * dwnorm;
-  }
-  return 0.0f;
-}
-// (dW/dr)/r at u = r/H, i.e. ∇W = dx · dWr_f: -20 (1-u)^3 dwnorm / H (u/r = 1/H).
-__device__ __forceinline__ float dWr_f(float u, float dwr) {
-  const float um1 = 1.0f - u;
-  return u < 1.0f ? dwr * (um1 * um1 * um1) : 0.0f;
 }
 
 // FP64 pair arithmetic.  A pair of the Float64 path once cost ten IEEE
@@ -98,11 +91,13 @@ __device__ __forceinline__ float dWr_f(float u, float dwr) {
 // 1/x, and sqrt(x) with sqrt(0) = 0: the hardware seed and Newton steps, to
 // about an ulp for normal x away from the ends of the FP64 range.
 __device__ __forceinline__ double rcp_d(double x) {
+#pragma clang fp contract(off)
   double r = __builtin_amdgcn_rcp(x);
   r = __builtin_fma(__builtin_fma(-x, r, 1.0), r, r);
   return __builtin_fma(__builtin_fma(-x, r, 1.0), r, r);
 }
 __device__ __forceinline__ double sqrt_d(double x) {
+#pragma clang fp contract(off)
   const double y = __builtin_amdgcn_rsq(x);
   double s = x * y, h = 0.5 * y;
   const double e = __builtin_fma(-h, s, 0.5);
@@ -111,12 +106,18 @@ __device__ __forceinline__ double sqrt_d(double x) {
   s = __builtin_fma(__builtin_fma(-s, s, x), h, s);
   return x == 0.0 ? 0.0 : s;
 }
-// (dW/dr)/r at distance r, i.e. ∇W = dx · dWr_d (u/r = 1/H).  NaN for
-// coincident particles, as the reference's dW/r.
-__device__ __forceinline__ double dWr_d(double r2, double r, const SphConst& C) {
-  const double um1 = 1.0 - r * C.Hinv;
+// (dW/dr)/r at distance r, i.e. ∇W = dx · dWr: -20 (1-u)^3 dwnorm / H (u/r =
+// 1/H).  FP64: NaN for coincident particles, as the reference's dW/r.
+__device__ __forceinline__ double dWr(double r2, double r, const SphConst& C) {
+#pragma clang fp contract(off)
+  const double um1 = __builtin_fma(-r, C.Hinv, 1.0);
   const double w = um1 > 0.0 ? C.dwr * (um1 * um1 * um1) : 0.0;
   return r2 != 0.0 ? w : __builtin_nan("");
+}
+__device__ __forceinline__ float dWr(float, float r, const SphConst& C) {
+#pragma clang fp contract(off)
+  const float um1 = __builtin_fmaf(-r, C.f_Hinv, 1.0f);
+  return um1 > 0.0f ? C.f_dwr * (um1 * um1 * um1) : 0.0f;
 }
 // ρ0·(powfancy7th(1+z) - 1) of the δ-SPH term.  powfancy7th stops two Halley
 // steps after a guess from the bit pattern, 3.87e-13 below the root near 1 (an
@@ -129,6 +130,7 @@ __device__ __forceinline__ double dWr_d(double r2, double r, const SphConst& C) 
 // registers cost the γ = 7 kernels a wave per SIMD.
 template <bool G7>
 __device__ __forceinline__ double hydro_drho_d(double z, const SphConst& C) {
+#pragma clang fp contract(off)
   if constexpr (G7) {
     if (fabs(z) < 0x1p-8) {
       double t = __builtin_fma(z, 81549.0 / 5764801.0, -1989.0 / 117649.0);
@@ -145,29 +147,40 @@ __device__ __forceinline__ double hydro_drho_d(double z, const SphConst& C) {
     return C.rho0 * pf7(1 + z, C.gamma, C.ginv) - C.rho0;
   }
 }
-// 1/ρb, 1/(ρa + ρb) and 1/(r² + η²) of a pair from one reciprocal; 1/ρb from
-// the record where it is stored.
+// 1/ρb, 1/(ρa + ρb) and 1/(r² + η²) of a pair: FP64 from one reciprocal, 1/ρb
+// from the record where it is stored; FP32 from the hardware reciprocals of
+// ρb(ρa + ρb) (densities near ρ0, so the product stays far from the FP32 range
+// limits) and r² + η².
+template <typename R>
 struct Inv3 {
-  double rhob, sum, den;
+  R rhob, sum, den;
 };
-__device__ __forceinline__ Inv3 inv_stored(double irhob, double sum, double den) {
+__device__ __forceinline__ Inv3<double> inv_stored(double irhob, double sum, double den) {
+#pragma clang fp contract(off)
   const double r = rcp_d(sum * den);
   return {irhob, r * den, r * sum};
 }
-__device__ __forceinline__ Inv3 inv_all(double rhob, double sum, double den) {
+__device__ __forceinline__ Inv3<double> inv_all(double rhob, double sum, double den) {
+#pragma clang fp contract(off)
   const double bs = rhob * sum, r = rcp_d(bs * den), rd = r * den;
   return {rd * sum, rd * rhob, r * bs};
 }
 template <int D>
-__device__ __forceinline__ Inv3 pair_inv(const PartnerN64<D>& q, double sum, double den) {
+__device__ __forceinline__ Inv3<double> pair_inv(const PartnerN64<D>& q, double, double sum, double den) {
   return inv_stored(q.irho, sum, den);
 }
 template <int D>
-__device__ __forceinline__ Inv3 pair_inv(const PartnerH64<D>& q, double sum, double den) {
+__device__ __forceinline__ Inv3<double> pair_inv(const PartnerH64<D>& q, double, double sum, double den) {
   return inv_stored(q.irh, sum, den);
 }
-__device__ __forceinline__ Inv3 pair_inv(const PartnerH64<3>& q, double sum, double den) {
+__device__ __forceinline__ Inv3<double> pair_inv(const PartnerH64<3>& q, double, double sum, double den) {
   return inv_all(q.rh, sum, den);
+}
+template <typename Q>
+__device__ __forceinline__ Inv3<float> pair_inv(const Q&, float rhob, float sum, float den) {
+#pragma clang fp contract(off)
+  const float r = __builtin_amdgcn_rcpf(rhob * sum);
+  return {sum * r, rhob * r, __builtin_amdgcn_rcpf(den)};
 }
 template <int D>
 __device__ __forceinline__ void set_irho(PartnerN64<D>& q) {
@@ -180,6 +193,7 @@ __device__ __forceinline__ void set_irho(PartnerH64<D>& q) {
 __device__ __forceinline__ void set_irho(PartnerH64<3>&) {}
 // sin(πs), |s| <= 1/2: its Taylor series (the first term dropped is below 2^-59)
 __device__ __forceinline__ double sinpi_d(double s) {
+#pragma clang fp contract(off)
   constexpr double p = 3.14159265358979323846, p2 = p * p;
   constexpr double c3 = p * p2 / 6, c5 = c3 * p2 / 20, c7 = c5 * p2 / 42, c9 = c7 * p2 / 72, c11 = c9 * p2 / 110,
                    c13 = c11 * p2 / 156, c15 = c13 * p2 / 210, c17 = c15 * p2 / 272, c19 = c17 * p2 / 342,
@@ -199,6 +213,7 @@ __device__ __forceinline__ double sinpi_d(double s) {
 // ∂v∂tpF! coefficient s·cos(1.5π r/2h)/(r + 0.1h) for r < 2h:
 // cos(πy) = -sin(π(y - 1/2)), y in [0, 1.5), folded into [-1/2, 1/2]
 __device__ __forceinline__ double surf_d(double r, const SphConst& C) {
+#pragma clang fp contract(off)
   const double y = r * C.st_pi;
   return -C.s * sinpi_d(y > 1.0 ? 1.5 - y : y - 0.5) * rcp_d(r + C.st_01h);
 }
@@ -213,52 +228,79 @@ __device__ __forceinline__ double eos_d(double rho, int32_t pt, const SphConst& 
 // both positive or both negative, without the 64-bit multiply.
 __device__ __forceinline__ bool same_kind(int32_t pa, int32_t pb) { return (pa > 0 && pb > 0) || (pa < 0 && pb < 0); }
 
-// FP32-split 1/ρb and 1/(ρa + ρb) from one hardware reciprocal of
-// ρb(ρa + ρb) (densities near ρ0, so the product stays far from the FP32
-// range limits).
-struct RhoInv {
-  float inv_rhob, inv_sum;
-};
-__device__ __forceinline__ RhoInv rho_inv2(float rhoa, float rhob) {
-  const float sum = rhoa + rhob;
-  const float R = __builtin_amdgcn_rcpf(rhob * sum);
-  return {sum * R, rhob * R};
-}
-
 // FP32-split EOS on δρ: P0((1+e)^7 - 1) = P0 e (7 + 21e + 35e² + 35e³ + 21e⁴ + 7e⁵ + e⁶).
 __device__ __forceinline__ float eos_f(float drho, int32_t pt, const SphConst& C) {
+#pragma clang fp contract(off)
   if (pt <= 1 && drho < 0.0f) return 0.0f;
-  float e = drho * C.f_inv_rho0;
-  float poly = 7.0f + e * (21.0f + e * (35.0f + e * (35.0f + e * (21.0f + e * (7.0f + e)))));
+  const float e = drho * C.f_inv_rho0;
+  float poly = __builtin_fmaf(e, 7.0f + e, 21.0f);
+  poly = __builtin_fmaf(e, poly, 35.0f);
+  poly = __builtin_fmaf(e, poly, 35.0f);
+  poly = __builtin_fmaf(e, poly, 21.0f);
+  poly = __builtin_fmaf(e, poly, 7.0f);
   return C.f_P0 * (e * poly);
 }
-// ρ0((1+z)^(1/7) - 1) without cancellation (FP32-split form of
-// ρ0*powfancy7th(1+z) - ρ0): binomial series, exact function for |z| > 1e-2.
-__device__ __forceinline__ float hydro_drho_f(float z, float rho0) {
+// dr - ρ0((1+z)^(1/7) - 1) without cancellation (the δ-SPH term's density
+// difference less its hydrostatic part): binomial series, exact function for
+// |z| > 1e-2.
+__device__ __forceinline__ float minus_hydro(float dr, float z, const SphConst& C) {
+#pragma clang fp contract(off)
+  float t;
   if (fabsf(z) < 1e-2f) {
-    float t = z * (1.0f / 7.0f + z * (-3.0f / 49.0f + z * (13.0f / 343.0f + z * (-65.0f / 2401.0f))));
-    return rho0 * t;
+    t = __builtin_fmaf(z, -65.0f / 2401.0f, 13.0f / 343.0f);
+    t = __builtin_fmaf(z, t, -3.0f / 49.0f);
+    t = z * __builtin_fmaf(z, t, 1.0f / 7.0f);
+  } else {
+    t = expm1f(log1pf(z) * (1.0f / 7.0f));
   }
-  return rho0 * expm1f(log1pf(z) * (1.0f / 7.0f));
+  return __builtin_fmaf(-C.f_rho0, t, dr);
 }
 
 // FP32-split ∂v∂tpF! coefficient s·cos(1.5π r/2h)/(r + 0.1h), for r < 2h: the
 // hardware cosine (argument in turns, here in [0, 0.75)) and reciprocal.
 __device__ __forceinline__ float surf_f(float r, const SphConst& C) {
+#pragma clang fp contract(off)
   return C.f_s * __builtin_amdgcn_cosf(r * C.f_st_turn) * __builtin_amdgcn_rcpf(r + C.f_st_01h);
 }
 
-template <typename R>
-struct Sum {  // plain sum
-  R s = R(0);
-  __device__ __forceinline__ void add(R v) { s += v; }
-  __device__ __forceinline__ R get() const { return s; }
+// Value of lane K of the quad (four consecutive lanes, all active).
+template <int K>
+__device__ __forceinline__ uint32_t quad_lane(uint32_t v) {
+  return uint32_t(__builtin_amdgcn_mov_dpp(int(v), K * 0x55, 0xf, 0xf, true));
+}
+template <int K>
+__device__ __forceinline__ float quad_lane(float v) {
+  return __uint_as_float(quad_lane<K>(__float_as_uint(v)));
+}
+template <int K>
+__device__ __forceinline__ double quad_lane(double v) {
+  return __hiloint2double(int(quad_lane<K>(uint32_t(__double2hiint(v)))), int(quad_lane<K>(uint32_t(__double2loint(v)))));
+}
+
+// The terms one partner adds to a particle's N sums, and the sums: FP64 in
+// both precisions (an FP32 term costs a conversion and an addition).
+template <int N, typename R>
+struct Terms {
+  R v[N] = {};
 };
-template <>
-struct Sum<float> {  // FP32 pair terms accumulated in FP64 (2 VALU per term, exact for ~30 terms)
-  double s = 0.0;
-  __device__ __forceinline__ void add(float v) { s += double(v); }
-  __device__ __forceinline__ float get() const { return float(s); }
+template <int N, typename R>
+struct Sums {
+  double s[N] = {};
+  __device__ __forceinline__ void add(const Terms<N, R>& t) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) s[i] += double(t.v[i]);
+  }
+  // the terms of the quad's four lanes, in lane order
+  __device__ __forceinline__ void add_quad(const Terms<N, R>& t) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      s[i] += double(quad_lane<0>(t.v[i]));
+      s[i] += double(quad_lane<1>(t.v[i]));
+      s[i] += double(quad_lane<2>(t.v[i]));
+      s[i] += double(quad_lane<3>(t.v[i]));
+    }
+  }
+  __device__ __forceinline__ R get(int i) const { return R(s[i]); }
 };
 
 template <int D>
@@ -282,16 +324,20 @@ __device__ __forceinline__ double dotd(const double* a, const double* b) {
   return s;
 }
 // dotd with fused multiply-adds, where no comparison reads it
+__device__ __forceinline__ double fma_(double a, double b, double c) { return __builtin_fma(a, b, c); }
+__device__ __forceinline__ float fma_(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 template <int D>
 __device__ __forceinline__ double dotm(const double* a, const double* b) {
-  double s = __builtin_fma(a[1], b[1], a[0] * b[0]);
-  if (D == 3) s = __builtin_fma(a[2], b[2], s);
+#pragma clang fp contract(off)
+  double s = fma_(a[1], b[1], a[0] * b[0]);
+  if (D == 3) s = fma_(a[2], b[2], s);
   return s;
 }
 template <int D>
 __device__ __forceinline__ float dotf(const float* a, const float* b) {
-  float s = a[0] * b[0] + a[1] * b[1];
-  if (D == 3) s = s + a[2] * b[2];
+#pragma clang fp contract(off)
+  float s = fma_(a[0], b[0], a[1] * b[1]);
+  if (D == 3) s = fma_(a[2], b[2], s);
   return s;
 }
 
@@ -332,10 +378,12 @@ struct ManyScenes {
   const int2* __restrict__ pmap;
   const int2* __restrict__ cmap;
   const int2* __restrict__ pmap512;  // (problem, 512-particle block of the problem)
+  const int2* __restrict__ qmap;     // (problem, 64-particle block of the problem): a quad of lanes per particle
 };
 // Blocks of BS threads (128, 256 or 512) over one problem's particles: m.y is
-// the block's index in units of BS particles, so particle a = m.y·BS + tid.
-template <int BS = kBlock, typename R>
+// the block's index in units of BS particles, so particle a = m.y·BS + tid;
+// Quad: blocks of 256 threads over 64 particles, m.y in units of 64.
+template <int BS = kBlock, bool Quad = false, typename R>
 __device__ __forceinline__ const SceneDev<R>& particle_scene(const OneScene<R>& s, int2& m) {
   m = make_int2(0, int(xcd_block()));
   return s.d;
@@ -351,11 +399,14 @@ __device__ __forceinline__ const SceneDev<R>& batch_scene(const ManyScenes<R>& s
   CS* c = (CS*)(s.S);
   return *(const SceneDev<R>*)(c + i);
 }
-template <int BS = kBlock, typename R>
+template <int BS = kBlock, bool Quad = false, typename R>
 __device__ __forceinline__ const SceneDev<R>& particle_scene(const ManyScenes<R>& s, int2& m) {
   static_assert(BS == 128 || BS == 256 || BS == 512, "block sizes of the particle maps");
+  static_assert(!Quad || BS == 256, "quads come in blocks of 256 threads");
   const unsigned L = xcd_block();
-  if constexpr (BS == 256) {
+  if constexpr (Quad) {
+    m = s.qmap[L];
+  } else if constexpr (BS == 256) {
     m = s.pmap[L];
   } else if constexpr (BS == 128) {  // halves of the 256-particle blocks
     const int2 e = s.pmap[L >> 1];
@@ -397,20 +448,26 @@ __device__ __forceinline__ StepFlags step_flags(const SceneDev<R>& sd) {
   return F;
 }
 
-// Binds the problem of this block of BS threads: B, C, G, F and the particle
-// index a.
-#define GCLSPH_SCENE_BS(ss, BS)                                \
-  int2 m;                                                      \
-  const SceneDev<R>& sd = particle_scene<BS, R>(ss, m);        \
-  const SphBufs<R>& B = sd.B;                                  \
-  const SphConst& C = sd.C;                                    \
-  const CellGeom& G = sd.G;                                    \
-  const StepFlags F = step_flags(sd);                          \
-  const int64_t a = int64_t(m.y) * (BS) + threadIdx.x;         \
-  (void)C;                                                     \
-  (void)G;                                                     \
+// Binds the problem of this block: B, C, G, F and the particle index a.
+#define GCLSPH_SCENE_OF(ss, BS, Quad)                         \
+  int2 m;                                                     \
+  const SceneDev<R>& sd = particle_scene<BS, Quad, R>(ss, m); \
+  const SphBufs<R>& B = sd.B;                                 \
+  const SphConst& C = sd.C;                                   \
+  const CellGeom& G = sd.G;                                   \
+  const StepFlags F = step_flags(sd);                         \
+  (void)C;                                                    \
+  (void)G;                                                    \
   (void)F
-#define GCLSPH_SCENE(ss) GCLSPH_SCENE_BS(ss, kBlock)
+#define GCLSPH_SCENE(ss)              \
+  GCLSPH_SCENE_OF(ss, kBlock, false); \
+  const int64_t a = int64_t(m.y) * kBlock + threadIdx.x
+// In the pair kernels: a particle per thread, or (Quad) per four threads, the
+// first of which writes its results.
+#define GCLSPH_SCENE_PAIR(ss, BS, Quad)                                                                   \
+  GCLSPH_SCENE_OF(ss, BS, Quad);                                                                          \
+  const int64_t a = (Quad) ? int64_t(m.y) * 64 + (threadIdx.x >> 2) : int64_t(m.y) * (BS) + threadIdx.x;  \
+  const bool writer = !(Quad) || (threadIdx.x & 3) == 0
 
 // Member bits of one window [lo, hi) (hi - lo <= 32) of a stencil row: bit j is
 // set when candidate lo + j is a partner of particle a, i.e. b != a and
@@ -751,6 +808,28 @@ struct Partners {
   }
   __device__ __forceinline__ int32_t take(NoWin&) { return take(); }
 
+  // The quad's four lanes hold the same state: lane i takes the i-th of the
+  // window's next four partners, or `none` (on = false) past its last.
+  template <typename W>
+  __device__ __forceinline__ int32_t take_quad(bool& on, const int32_t none, W& w) {
+    const uint32_t i = threadIdx.x & 3u;
+    const bool had = c != 0;
+    uint32_t m = c;
+    m = i > 0 ? m & (m - 1) : m;
+    m = i > 1 ? m & (m - 1) : m;
+    m = i > 2 ? m & (m - 1) : m;
+    on = m != 0;
+    const int32_t b = on ? cb + __builtin_ctz(m) : none;
+    if constexpr (Fr) {
+      w.k[0] = wk[0];
+      w.k[1] = wk[1];
+      w.k[2] = wk[2];
+    }
+    c = quad_lane<3>(m & (m - 1));
+    if (had && c == 0) fill();
+    return b;
+  }
+
   __device__ __forceinline__ void set_window(uint32_t code) {
     if constexpr (Fr) {
       // base-3 digits of code < 27: q / 3 = (q · 11) >> 5 for q < 27
@@ -832,55 +911,249 @@ __device__ __forceinline__ void for_each_partner(const SphBufs<R>& B, int64_t a,
 }
 
 // As for_each_partner, with the partner data split off: fetch(b) loads what
-// the body needs of partner b.  Pipe: the fetch of the next partner is issued
+// the body needs of partner b, body(partner, terms[, window]) evaluates what
+// the pair adds to the sums.  Pipe: the fetch of the next partner is issued
 // before the body of the current one runs, so the loads overlap the pair
 // arithmetic (at the cost of the registers holding both partners' data).
 // Frames (3D FP32-split readers of partner records): kt holds the particle's
-// separation constants and the body receives the partner's window constants
-// as a third argument.
-template <bool Pipe, int D, typename R, bool Frames = false, typename Fetch, typename F>
-__device__ __forceinline__ void for_each_partner_fetch(const SphBufs<R>& B, int64_t a, int nc, const CellGeom& G,
-                                                       const double* const* XM, double dist2, Fetch&& fetch,
-                                                       F&& body, const FrameK3* kt = nullptr) {
+// separation constants and the body receives the partner's window constants.
+//
+// Quad: the four lanes of a particle evaluate four partners of a window at
+// once and every lane adds their terms in partner order, so the sums are those
+// of one lane, bit for bit, whatever a launch chooses.  A particle's partners
+// are a serial loop (~36 trips in 2D, ~160 in 3D), and a small problem leaves
+// most of the 1024 SIMDs without a wave: there a quad finishes in about a
+// third of the trips.  With the chip full the extra selection and additions
+// (~50 instructions per trip beside a body of ~100) only cost.
+template <bool Pipe, bool Quad, int D, int N, typename R, bool Frames = false, typename Fetch, typename F>
+__device__ __forceinline__ Sums<N, R> sum_partners(const SphBufs<R>& B, int64_t a, int nc, const CellGeom& G,
+                                                   const double* const* XM, double dist2, Fetch&& fetch, F&& body,
+                                                   const FrameK3* kt = nullptr) {
   constexpr bool Fr = Frames && D == 3 && std::is_same<R, float>::value;
   using W = typename std::conditional<Fr, Win3, NoWin>::type;
   Partners<D, R, Fr> it(B, a, nc, G, XM, dist2, kt);
-  auto run = [&](const int32_t b, const auto& f, const W& w) {
-    if constexpr (Fr) body(b, f, w);
-    else body(b, f);
+  Sums<N, R> sum;
+  auto run = [&](const bool on, const auto& f, const W& w) {
+    if constexpr (Quad) {
+      Terms<N, R> t;
+      if (on) {
+        if constexpr (Fr) body(f, t, w);
+        else body(f, t);
+      }
+      sum.add_quad(t);
+    } else if (on) {
+      Terms<N, R> t;
+      if constexpr (Fr) body(f, t, w);
+      else body(f, t);
+      sum.add(t);
+    }
+  };
+  // this lane's next partner; `none` (a valid index) and on = false without one
+  auto take = [&](bool& on, const int32_t none, W& w) {
+    if constexpr (Quad) {
+      return it.take_quad(on, none, w);
+    } else {
+      on = it.has();
+      return on ? it.take(w) : none;
+    }
   };
   if constexpr (!Pipe) {
-    for (;;) {
-      const bool m = it.has();
-      if (!__any(m)) break;
-      if (m) {
-        W w;
-        const int32_t b = it.take(w);
-        run(b, fetch(b), w);
+    while (__any(it.has())) {
+      W w{};
+      bool on;
+      const int32_t b = take(on, int32_t(a), w);
+      if constexpr (Quad) {
+        run(on, fetch(b), w);
+      } else if (on) {
+        run(true, fetch(b), w);
       }
     }
-    return;
+    return sum;
   }
   // two partners in flight, alternating between two sets of registers; a lane
-  // without a next partner fetches its previous one (or itself) again, which
-  // is a valid address, and skips the body
-  bool m0 = it.has();
-  if (!__any(m0)) return;
+  // without a next partner fetches a valid address again and skips the body
+  if (!__any(it.has())) return sum;
   W w0{}, w1{};
-  int32_t b0 = m0 ? it.take(w0) : int32_t(a);
+  bool m0, m1;
+  int32_t b0 = take(m0, int32_t(a), w0);
   auto f0 = fetch(b0);
   for (;;) {
-    const bool m1 = it.has();
-    const int32_t b1 = m1 ? it.take(w1) : b0;
+    bool more = __any(it.has());
+    const int32_t b1 = take(m1, b0, w1);
     auto f1 = fetch(b1);
-    if (m0) run(b0, f0, w0);
-    if (!__any(m1)) break;
-    m0 = it.has();
-    b0 = m0 ? it.take(w0) : b1;
+    run(m0, f0, w0);
+    if (!more) break;
+    more = __any(it.has());
+    b0 = take(m0, b1, w0);
     f0 = fetch(b0);
-    if (m1) run(b1, f1, w1);
-    if (!__any(m0)) break;
+    run(m1, f1, w1);
+    if (!more) break;
   }
+  return sum;
+}
+
+// ---------------------------------------------------------------- the pair
+// Squared distance as the cut-offs compare it: FP64 unfused, as the reference
+// has it.
+template <int D>
+__device__ __forceinline__ double dist2_of(const double* dx) {
+  return dotd<D>(dx, dx);
+}
+template <int D>
+__device__ __forceinline__ float dist2_of(const float* dx) {
+  return dotf<D>(dx, dx);
+}
+__device__ __forceinline__ double root_of(double x) { return sqrt_d(x); }
+__device__ __forceinline__ float root_of(float x) { return __builtin_amdgcn_sqrtf(x); }
+// What a pair takes from its particle alone.
+template <typename R>
+struct Own {
+  R rho;   // ρ_a
+  R drho;  // what the records hold: ρ_a, or δρ_a in FP32-split
+  R P;
+  R mPi;   // -m0/ρ_a, of the pressure term
+  R kd;    // FP64: 2hδc0 of the δ-SPH term, which acts on ptype > 1 only
+  int32_t pt;
+};
+template <typename R>
+__device__ __forceinline__ Own<R> own_of(R drho, R P, int32_t pt, const SphConst& C) {
+#pragma clang fp contract(off)
+  Own<R> o;
+  o.drho = drho;
+  o.P = P;
+  o.pt = pt;
+  if constexpr (std::is_same<R, double>::value) {
+    o.rho = drho;
+    o.kd = pt > 1 ? C.DDTkh : 0.0;
+    o.mPi = -C.m0 * (1.0 / drho);
+  } else {
+    o.rho = C.f_rho0 + drho;
+    o.mPi = -C.f_m0 * __builtin_amdgcn_rcpf(o.rho);
+  }
+  return o;
+}
+
+// What the pair (a, b) adds to a's acceleration (t.v[0..D-1]) and ∂ρ/∂t
+// (t.v[D]): ∂ρ∂tDDT! (src/gpukernels_sph.jl:579-625), ∂v∂t! (:755-772), ∂v∂t_av!
+// (:869-897), ∂v∂t_visc! (:967-980), ∂v∂tpF! (:1387-1397) and the wall force k
+// (0: 2dx, 1: bound_l).  dx, dv: separation and relative velocity of the state
+// the rates are taken at; dg, rg2, rg: the separation (and its length) ∇W and
+// the wall force are taken at (xⁿ; Same: dx is it).  ∇W = dg·dwr, so the terms
+// along ∇W share one coefficient of dg.  The terms every pair has are evaluated
+// and selected, without branches.  q: the partner's record; rb, ptb, Pb its
+// density as held, type and pressure.
+template <int D, bool G7, bool Same, typename Q>
+__device__ __forceinline__ void pair_terms(const SphConst& C, const StepFlags& F, const Own<double>& o, const Q& q,
+                                           double rb, int32_t ptb, double Pb, const double* dx, const double* dv,
+                                           const double* dg, double rg2, double rg, int k, Terms<D + 1, double>& t) {
+#pragma clang fp contract(off)
+  const double dwr = dWr(rg2, rg, C);
+  const double r2 = Same ? rg2 : dist2_of<D>(dx);
+  const double dxdg = Same ? r2 : dotm<D>(dx, dg);
+  const double dvdx = dotm<D>(dv, dx);
+  const double dvdg = Same ? dvdx : dotm<D>(dv, dg);
+  const Inv3<double> iv = pair_inv(q, rb, o.rho + rb, r2 + C.eta2);
+  const bool both = o.pt > 0 && ptb > 0;
+  {  // ∂ρ/∂t: m0 dwr (dv·dg - kd (ρb - ρa - hydrostatic) (dx·dg) / (ρb (r² + η²)))
+    const double e = o.kd * ((rb - o.rho) - hydro_drho_d<G7>(C.DDTgz * dx[1], C)) * iv.den * dxdg;
+    const double s = C.m0 * dwr * fma_(-e, iv.rhob, dvdg);
+    t.v[D] = both ? s : 0.0;
+  }
+  double f = (o.P + Pb) * iv.rhob * o.mPi;             // pressure
+  const double av = C.av * fmin(dvdx, 0.0) * iv.den;  // artificial viscosity, approaching pairs
+  f = both ? fma_(av, iv.sum, f) : f;
+  f = same_kind(o.pt, ptb) ? f * dwr : 0.0;
+  double ax[3] = {0.0, 0.0, 0.0};
+  if (both) {
+    if (F.nu_on) {
+      const double term = C.nu4 * (dxdg * dwr) * (iv.sum * iv.den);
+#pragma unroll
+      for (int d = 0; d < D; ++d) ax[d] = term * dv[d];
+    }
+    if (F.s_on && r2 < C.st_t2) {
+      const double g = surf_d(Same ? rg : sqrt_d(r2), C) * (1.0 / C.m0);
+#pragma unroll
+      for (int d = 0; d < D; ++d) ax[d] = fma_(g, dx[d], ax[d]);
+    }
+  }
+  if ((o.pt > 0) != (ptb > 0) && rg2 < C.fb_t2[k]) {  // fbmolforce! (:1891-1901)
+    const double q1 = C.fb_r0[k] / (rg + C.fb_eta2[k]);
+    const double Fc = C.fb_d[k] * (powi_d(q1, 12) - powi_d(q1, 4)) / (rg2 + C.fb_eta2[k]);
+#pragma unroll
+    for (int d = 0; d < D; ++d) ax[d] = fma_(dg[d], Fc, ax[d]);
+  }
+#pragma unroll
+  for (int d = 0; d < D; ++d) t.v[d] = fma_(f, dg[d], ax[d]);
+}
+
+// FP32-split: the same terms in FP32.
+template <int D, bool G7, bool Same, typename Q>
+__device__ __forceinline__ void pair_terms(const SphConst& C, const StepFlags& F, const Own<float>& o, const Q& q,
+                                           float drb, int32_t ptb, float Pb, const float* dx, const float* dv,
+                                           const float* dg, float rg2, float rg, int k, Terms<D + 1, float>& t) {
+#pragma clang fp contract(off)
+  const float dwr = dWr(rg2, rg, C);
+  const float r2 = Same ? rg2 : dotf<D>(dx, dx);
+  const float dvdx = dotf<D>(dv, dx);
+  const float rhob = C.f_rho0 + drb;
+  const Inv3<float> iv = pair_inv(q, rhob, o.rho + rhob, r2 + C.f_eta2);
+  const bool both = o.pt > 0 && ptb > 0;
+  const float dxg = (Same ? r2 : dotf<D>(dx, dg)) * dwr;  // dx·∇W
+  {
+    const float s = C.f_m0 * dwr * (Same ? dvdx : dotf<D>(dv, dg));
+    const float vd = C.f_DDTkh * minus_hydro(drb - o.drho, C.f_DDTgz * dx[1], C) * iv.den;
+    const float sd = fma_(-(vd * dxg * C.f_m0), iv.rhob, s);
+    t.v[D] = both ? (o.pt > 1 ? sd : s) : 0.0f;
+  }
+  const float Pt = (o.P + Pb) * iv.rhob * o.mPi;
+  float f = same_kind(o.pt, ptb) ? Pt : 0.0f;
+  {
+    const float dmu = C.f_h * fminf(dvdx, 0.0f) * iv.den;  // AV acts on approaching pairs only
+    const float dPi = (-C.f_alpha * C.f_c0 * dmu) * (2.0f * iv.sum);
+    f -= both ? dPi * C.f_m0 : 0.0f;
+  }
+  f *= dwr;
+  float ax[3] = {0.0f, 0.0f, 0.0f};
+  if (both) {
+    if (F.nu_on) {
+      const float term = 4.0f * C.f_nu * C.f_m0 * dxg * (iv.sum * iv.den);
+#pragma unroll
+      for (int d = 0; d < D; ++d) ax[d] = term * dv[d];
+    }
+    if (F.s_on) {
+      const float r = Same ? rg : __builtin_amdgcn_sqrtf(r2);
+      if (r < C.f_st_2h) {
+        const float g = surf_f(r, C);
+        if constexpr (Same) {
+          f = fma_(g, C.f_inv_m0, f);
+        } else {
+#pragma unroll
+          for (int d = 0; d < D; ++d) ax[d] = fma_(g * dx[d], C.f_inv_m0, ax[d]);
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int d = 0; d < D; ++d) ax[d] = fma_(f, dg[d], ax[d]);
+  if ((o.pt > 0) != (ptb > 0) && rg < C.f_fb_r0[k]) {
+    // wall force: FP32 while q = r0/(r + η²) < 32 (q^12 < 1.2e18, far inside
+    // the FP32 range), FP64 for the (rare) closer pairs
+    const float q1 = C.f_fb_r0[k] * __builtin_amdgcn_rcpf(rg + C.f_fb_eta2[k]);
+    if (q1 < 32.0f) {
+      const float q2 = q1 * q1, q4 = q2 * q2, q8 = q4 * q4;
+      const float Fc = C.f_fb_d[k] * fma_(q4, q8, -q4) * __builtin_amdgcn_rcpf(rg2 + C.f_fb_eta2[k]);
+#pragma unroll
+      for (int d = 0; d < D; ++d) ax[d] = fma_(dg[d], Fc, ax[d]);
+    } else {
+      const double p1 = C.fb_r0[k] / (double(rg) + C.fb_eta2[k]);
+      const double p2 = p1 * p1, p4 = p2 * p2, p8 = p4 * p4;
+      const double Fc = C.fb_d[k] * (p4 * p8 - p4) / (double(rg2) + C.fb_eta2[k]);
+#pragma unroll
+      for (int d = 0; d < D; ++d) ax[d] += float(double(dg[d]) * Fc);
+    }
+  }
+#pragma unroll
+  for (int d = 0; d < D; ++d) t.v[d] = ax[d];
 }
 
 __device__ __forceinline__ double nanmax(double a, double b) { return (a > b || a != a) ? a : b; }
@@ -911,7 +1184,7 @@ __device__ __forceinline__ void block_max(double v, bool active, double* slots, 
 template <typename R, typename Fn>
 inline void with_scenes(const LaunchSet& L, Fn&& f) {
   if (L.one) f(OneScene<R>{*static_cast<const SceneDev<R>*>(L.one)});
-  else f(ManyScenes<R>{static_cast<const SceneDev<R>*>(L.scenes), L.pmap, L.cmap, L.pmap512});
+  else f(ManyScenes<R>{static_cast<const SceneDev<R>*>(L.scenes), L.pmap, L.cmap, L.pmap512, L.qmap});
 }
 
 }  // namespace gclsph

@@ -492,10 +492,10 @@ __global__ __launch_bounds__(256) void k_reorder_nmask2(SS ss) {
 
 // ---- corrections after the update (src/sphproblem.jl:303-322) --------------
 // dpcreg! (src/gpukernels_sph.jl:1500-1553): ∑Δv_dpc into DV; P = EOS(ρ^{n+1}).
-template <int D, typename R, typename SS>
+template <int D, typename R, bool Quad, typename SS>
 __global__ __launch_bounds__(256) void k_dpc_sum(SS ss) {
 #pragma clang fp contract(off)
-  GCLSPH_SCENE(ss);
+  GCLSPH_SCENE_PAIR(ss, kBlock, Quad);
   if (!F.dpc_on) return;
   const StepCtl* ctl = B.ctl;
   const int p = ctl->parity, q = p ^ 1, pp = ctl->pparity, rebuilt = ctl->rebuilt;
@@ -520,16 +520,16 @@ __global__ __launch_bounds__(256) void k_dpc_sum(SS ss) {
   using Nb = typename Records<D, R>::N;
   auto fetch = [&](const int32_t b) { return ld_rec<Nb>(B.PRN, b, B.n); };
   const R Pa = B.PN[a];
-  if (F.want_out) B.PBUF[a] = Pa;
+  if (F.want_out && writer) B.PBUF[a] = Pa;
   if (pta <= 0) {  // every DPC pair needs ptype > 0 on both sides
 #pragma unroll
-    for (int d = 0; d < D; ++d) B.DV[d][a] = R(0);
+    for (int d = 0; d < D; ++d)
+      if (writer) B.DV[d][a] = R(0);
     return;
   }
   if constexpr (std::is_same<R, double>::value) {
     const double rhoa = RHO[a];
-    double sum[3] = {0.0, 0.0, 0.0};
-    for_each_partner_fetch<true, D>(B, a, nc, G, XM, C.dist2, fetch, [&](const int32_t, const Nb& n) {
+    const auto sum = sum_partners<true, Quad, D, D, R>(B, a, nc, G, XM, C.dist2, fetch, [&](const Nb& n, auto& t) {
       if (n.pt <= 0) return;
       double dx[3], dv[3];
 #pragma unroll
@@ -552,23 +552,22 @@ __global__ __launch_bounds__(256) void k_dpc_sum(SS ss) {
       if (vr < 0) {
         double vrdr = vr / (r2 + C.dpc_eta2);
 #pragma unroll
-        for (int d = 0; d < D; ++d) sum[d] += kk * (-vrdr * dx[d]);
+        for (int d = 0; d < D; ++d) t.v[d] = kk * (-vrdr * dx[d]);
       } else {
         double tvar = 2 * dt * Pb_dpc / ((rhoa + rhob) * (r2 + C.dpc_eta2));
 #pragma unroll
-        for (int d = 0; d < D; ++d) sum[d] += tvar * dx[d];
+        for (int d = 0; d < D; ++d) t.v[d] = tvar * dx[d];
       }
     });
 #pragma unroll
-    for (int d = 0; d < D; ++d) B.DV[d][a] = sum[d];
+    for (int d = 0; d < D; ++d)
+      if (writer) B.DV[d][a] = sum.get(d);
   } else {
-#pragma clang fp contract(fast)
     const float rhoa = C.f_rho0 + RHO[a];
     const float fdt = float(dt);
-    Sum<float> sum[3];
     const FrameK3 kt = particle_k<D, R>(B, C, G, a, xa);
-    for_each_partner_fetch<true, D, R, true>(B, a, nc, G, XM, C.dist2, fetch, [&](const int32_t, const Nb& n,
-                                                                         const auto&... win) {
+    const auto sum = sum_partners<true, Quad, D, D, R, true>(B, a, nc, G, XM, C.dist2, fetch, [&](const Nb& n, auto& t,
+                                                                                          const auto&... win) {
       if (rec_pt(n) <= 0) return;
       float dx[3], dv[3];
 #pragma unroll
@@ -578,8 +577,8 @@ __global__ __launch_bounds__(256) void k_dpc_sum(SS ss) {
       }
       const float rhob = C.f_rho0 + n.rho;
       const float r2 = dotf<D>(dx, dx);
-      const float u = __builtin_amdgcn_sqrtf(r2) * C.f_dpc_l0inv;
-      const float w = W_f(u, C.f_dpc_wnorm);
+      const float r = __builtin_amdgcn_sqrtf(r2), u = r * C.f_dpc_l0inv;
+      const float w = W_f(r, C.f_dpc_l0inv, C.f_dpc_wnorm);
       const float chi = __builtin_amdgcn_sqrtf(w * C.f_dpc_whinv);
       const float kk = u < C.f_dpc_lim ? 1.0f : chi;
       const float lo = C.f_dpc_lambda * fabsf(Pa + rec_P(n, C)), cap = C.f_dpc_lambda * C.f_dpc_pmax;
@@ -591,15 +590,16 @@ __global__ __launch_bounds__(256) void k_dpc_sum(SS ss) {
       if (vr < 0.0f) {
         const float vrdr = vr * den;
 #pragma unroll
-        for (int d = 0; d < D; ++d) sum[d].add(kk * (-vrdr * dx[d]));
+        for (int d = 0; d < D; ++d) t.v[d] = kk * (-vrdr * dx[d]);
       } else {
         const float tvar = 2.0f * fdt * Pb_dpc * __builtin_amdgcn_rcpf(rhoa + rhob) * den;
 #pragma unroll
-        for (int d = 0; d < D; ++d) sum[d].add(tvar * dx[d]);
+        for (int d = 0; d < D; ++d) t.v[d] = tvar * dx[d];
       }
     }, &kt);
 #pragma unroll
-    for (int d = 0; d < D; ++d) B.DV[d][a] = sum[d].get();
+    for (int d = 0; d < D; ++d)
+      if (writer) B.DV[d][a] = sum.get(d);
   }
 }
 
@@ -657,10 +657,10 @@ __global__ void k_xsph_rec(SS ss) {
 }
 
 // xsphcorr! + update_xsphcorr! (src/gpukernels_sph.jl:1757-1838): W at xⁿ.
-template <int D, typename R, typename SS>
+template <int D, typename R, bool Quad, typename SS>
 __global__ __launch_bounds__(256) void k_xsph(SS ss) {
 #pragma clang fp contract(off)
-  GCLSPH_SCENE(ss);
+  GCLSPH_SCENE_PAIR(ss, kBlock, Quad);
   if (!F.xsph_on) return;
   const StepCtl* ctl = B.ctl;
   const int p = ctl->parity, q = p ^ 1, pp = ctl->pparity, rebuilt = ctl->rebuilt;
@@ -688,8 +688,7 @@ __global__ __launch_bounds__(256) void k_xsph(SS ss) {
   double out[3];
   if constexpr (std::is_same<R, double>::value) {
     const double rhoa = RHO[a];
-    double sum[3] = {0.0, 0.0, 0.0};
-    for_each_partner_fetch<true, D>(B, a, nc, G, XM, C.dist2, fetch, [&](const int32_t, const Nb& n) {
+    const auto sum = sum_partners<true, Quad, D, D, R>(B, a, nc, G, XM, C.dist2, fetch, [&](const Nb& n, auto& t) {
       if (n.pt <= 1) return;
       double dx[3];
 #pragma unroll
@@ -698,30 +697,29 @@ __global__ __launch_bounds__(256) void k_xsph(SS ss) {
       const double w = W_d(r * C.Hinv, C.wnorm);
       const double xs = C.xsph_c * w / (rhoa + n.rho);
 #pragma unroll
-      for (int d = 0; d < D; ++d) sum[d] += (n.v[d] - va[d]) * xs;
+      for (int d = 0; d < D; ++d) t.v[d] = (n.v[d] - va[d]) * xs;
     });
 #pragma unroll
-    for (int d = 0; d < D; ++d) out[d] = sum[d];
+    for (int d = 0; d < D; ++d) out[d] = sum.get(d);
   } else {
-#pragma clang fp contract(fast)
     const float rhoa = C.f_rho0 + RHO[a];
-    Sum<float> sum[3];
     const FrameK3 kt = particle_k<D, R>(B, C, G, a, xa);
-    for_each_partner_fetch<true, D, R, true>(B, a, nc, G, XM, C.dist2, fetch, [&](const int32_t, const Nb& n,
-                                                                         const auto&... win) {
+    const auto sum = sum_partners<true, Quad, D, D, R, true>(B, a, nc, G, XM, C.dist2, fetch, [&](const Nb& n, auto& t,
+                                                                                          const auto&... win) {
       if (rec_pt(n) <= 1) return;
       float dx[3];
 #pragma unroll
       for (int d = 0; d < D; ++d) dx[d] = sep_x(xa, n, d, win...);
       const float r = __builtin_amdgcn_sqrtf(dotf<D>(dx, dx));
-      const float w = W_f(r * C.f_Hinv, C.f_wnorm);
+      const float w = W_f(r, C.f_Hinv, C.f_wnorm);
       const float xs = C.f_xsph_c * w * __builtin_amdgcn_rcpf(rhoa + (C.f_rho0 + n.rho));
 #pragma unroll
-      for (int d = 0; d < D; ++d) sum[d].add((n.v[d] - va[d]) * xs);
+      for (int d = 0; d < D; ++d) t.v[d] = (n.v[d] - va[d]) * xs;
     }, &kt);
 #pragma unroll
-    for (int d = 0; d < D; ++d) out[d] = double(sum[d].get());
+    for (int d = 0; d < D; ++d) out[d] = double(sum.get(d));
   }
+  if (!writer) return;
   double fr[3];
   particle_frame<D, R>(B, C, G, a, fr);
   using N = typename Records<D, R>::N;
@@ -737,10 +735,10 @@ __global__ __launch_bounds__(256) void k_xsph(SS ss) {
 }
 
 // cspmcorr! (src/gpukernels_sph.jl:1693-1719): ρ = Σ m0 W / Σ m0 W / ρ_b, W at xⁿ.
-template <int D, typename R, typename SS>
+template <int D, typename R, bool Quad, typename SS>
 __global__ __launch_bounds__(256) void k_cspm_sum(SS ss) {
 #pragma clang fp contract(off)
-  GCLSPH_SCENE(ss);
+  GCLSPH_SCENE_PAIR(ss, kBlock, Quad);
   if (!F.cspm_fire) return;
   const StepCtl* ctl = B.ctl;
   const int p = ctl->parity, q = p ^ 1, pp = ctl->pparity, rebuilt = ctl->rebuilt;
@@ -772,34 +770,36 @@ __global__ __launch_bounds__(256) void k_cspm_sum(SS ss) {
       return n;
     };
     if constexpr (std::is_same<R, double>::value) {
-      for_each_partner_fetch<true, D>(B, a, nc, G, XM, C.dist2, fetch, [&](const int32_t, const Nb& n) {
+      const auto sum = sum_partners<true, Quad, D, 2, R>(B, a, nc, G, XM, C.dist2, fetch, [&](const Nb& n, auto& t) {
         if (n.pt <= 0) return;
         double dx[3];
 #pragma unroll
         for (int d = 0; d < D; ++d) dx[d] = xa[d] - n.x[d];
         const double w = W_d(sqrt(dotd<D>(dx, dx)) * C.Hinv, C.wnorm);
-        s1 += C.m0 * w;
-        s2 += w * C.m0 / n.rho;
+        t.v[0] = C.m0 * w;
+        t.v[1] = w * C.m0 / n.rho;
       });
+      s1 = sum.s[0];
+      s2 = sum.s[1];
     } else {
       // on δρ: with e = δρ_b/ρ0, ρ' - ρ0 = ρ0 Σ m0W e/(1+e) / Σ m0W/(1+e), which
       // is s1/s2 - ρ0 without the cancellation against ρ0
-#pragma clang fp contract(fast)
-      for_each_partner_fetch<true, D>(B, a, nc, G, XM, C.dist2, fetch, [&](const int32_t, const Nb& n) {
+      const auto sum = sum_partners<true, Quad, D, 2, R>(B, a, nc, G, XM, C.dist2, fetch, [&](const Nb& n, auto& t) {
         if (n.pt <= 0) return;
         float dx[3];
 #pragma unroll
         for (int d = 0; d < D; ++d) dx[d] = float(xa[d] - n.x[d]);
-        const float w = W_f(__builtin_amdgcn_sqrtf(dotf<D>(dx, dx)) * C.f_Hinv, C.f_wnorm);
-        const float e = n.rho * (1.0f / C.f_rho0);
-        const float mw = C.f_m0 * w * __builtin_amdgcn_rcpf(1.0f + e);
-        s1 += double(mw * e);
-        s2 += double(mw);
+        const float w = W_f(__builtin_amdgcn_sqrtf(dotf<D>(dx, dx)), C.f_Hinv, C.f_wnorm);
+        const float inv_rho0 = 1.0f / C.f_rho0, e = n.rho * inv_rho0;
+        const float mw = C.f_m0 * w * __builtin_amdgcn_rcpf(fma_(n.rho, inv_rho0, 1.0f));
+        t.v[0] = mw * e;
+        t.v[1] = mw;
       });
-      s1 *= C.rho0;
+      s1 = sum.s[0] * C.rho0;
+      s2 = sum.s[1];
     }
   }
-  B.TMP[a] = s1 / s2;  // ρ (FP64 path) or ρ - ρ0 (FP32-split); NaN without partners
+  if (writer) B.TMP[a] = s1 / s2;  // ρ (FP64 path) or ρ - ρ0 (FP32-split); NaN without partners
 }
 
 template <int D, typename R, typename SS>
@@ -1213,7 +1213,8 @@ void launch_init_pn(const LaunchSet& L, hipStream_t s) {
 template <int D, typename R>
 void launch_dpc(const LaunchSet& L, hipStream_t s) {
   with_scenes<R>(L, [&](auto ss) {
-    k_dpc_sum<D, R, decltype(ss)><<<L.pblocks, kBlock, 0, s>>>(ss);
+    if (L.quad) k_dpc_sum<D, R, true, decltype(ss)><<<L.qblocks, kBlock, 0, s>>>(ss);
+    else k_dpc_sum<D, R, false, decltype(ss)><<<L.pblocks, kBlock, 0, s>>>(ss);
     k_dpc_apply<D, R, decltype(ss)><<<L.pblocks, kBlock, 0, s>>>(ss);
   });
 }
@@ -1221,13 +1222,15 @@ template <int D, typename R>
 void launch_xsph(const LaunchSet& L, hipStream_t s) {
   with_scenes<R>(L, [&](auto ss) {
     k_xsph_rec<D, R, decltype(ss)><<<L.pblocks, kBlock, 0, s>>>(ss);
-    k_xsph<D, R, decltype(ss)><<<L.pblocks, kBlock, 0, s>>>(ss);
+    if (L.quad) k_xsph<D, R, true, decltype(ss)><<<L.qblocks, kBlock, 0, s>>>(ss);
+    else k_xsph<D, R, false, decltype(ss)><<<L.pblocks, kBlock, 0, s>>>(ss);
   });
 }
 template <int D, typename R>
 void launch_cspm(const LaunchSet& L, hipStream_t s) {
   with_scenes<R>(L, [&](auto ss) {
-    k_cspm_sum<D, R, decltype(ss)><<<L.pblocks, kBlock, 0, s>>>(ss);
+    if (L.quad) k_cspm_sum<D, R, true, decltype(ss)><<<L.qblocks, kBlock, 0, s>>>(ss);
+    else k_cspm_sum<D, R, false, decltype(ss)><<<L.pblocks, kBlock, 0, s>>>(ss);
     k_cspm_apply<D, R, decltype(ss)><<<L.pblocks, kBlock, 0, s>>>(ss);
   });
 }

@@ -40,10 +40,10 @@ namespace gclsph {
 // picks one per pass by timing them on live steps.
 //
 // ---- pass 1 ---------------------------------------------------------------
-template <int D, typename R, typename SS, bool Pipe, int W, int BS, bool G7>
+template <int D, typename R, typename SS, bool Pipe, int W, int BS, bool G7, bool Quad>
 __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W))) void k_pass1(SS ss) {
 #pragma clang fp contract(off)
-  GCLSPH_SCENE_BS(ss, BS);
+  GCLSPH_SCENE_PAIR(ss, BS, Quad);
   const StepCtl* ctl = B.ctl;
   const int p = ctl->parity, pp = ctl->pparity, rebuilt = ctl->rebuilt;
   const double dt = ctl->dt;
@@ -64,75 +64,32 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W))) void k_
   }
   const R sa = RHO[a];
   const int32_t pta = PT[a];
-  Sum<R> acc[3], drho;
+  constexpr int kDrho = D;  // sums: D accelerations, ∂ρ/∂t
 
   const int nc = B.NC[a];
   if constexpr (std::is_same<R, double>::value) {
-    const double rhoa = sa;
-    const double mPa = -C.m0 * (1.0 / rhoa);  // -m0/ρ_a of the pressure term
-    const double Pa = B.PN[a];
+    const Own<R> own = own_of<R>(sa, B.PN[a], pta, C);
     using Nb = PartnerN64<D>;
     auto fetch = [&](const int32_t b) { return ld_rec<Nb>(B.PRN, b, B.n); };
-    // ∇W = dx·dwr: terms along ∇W are gathered into one coefficient fg of dx,
-    // dx·∇W = r²·dwr, dv·∇W = (dv·dx)·dwr
-    for_each_partner_fetch<Pipe, D>(B, a, nc, G, XM, C.dist2, fetch, [&](const int32_t, const Nb& q) {
-#pragma clang fp contract(fast)
-      const int32_t ptb = q.pt;
+    const auto sum = sum_partners<Pipe, Quad, D, D + 1, R>(B, a, nc, G, XM, C.dist2, fetch, [&](const Nb& q, auto& t) {
       double dx[3], dv[3];
 #pragma unroll
       for (int d = 0; d < D; ++d) {
         dx[d] = xa[d] - q.x[d];
         dv[d] = va[d] - q.v[d];
       }
-      const double r2 = dotd<D>(dx, dx);  // unfused: the cut-offs below compare it
-      const double r = sqrt_d(r2);
-      const double dwr = dWr_d(r2, r, C);
-      const double rhob = q.rho;
-      const Inv3 iv = pair_inv(q, rhoa + rhob, r2 + C.eta2);
-      const double dvdx = dotm<D>(dv, dx);
-      // the common terms are evaluated for every pair and selected
-      const bool both = pta > 0 && ptb > 0;
-      {  // ∂ρ∂tDDT! (:579-625)
-        const double s = C.m0 * dwr * dvdx;
-        const double vd = C.DDTkh * ((rhob - rhoa) - hydro_drho_d<G7>(C.DDTgz * dx[1], C)) * iv.den;
-        const double sd = s - vd * (r2 * dwr) * (C.m0 * iv.rhob);
-        drho.add(both ? (pta > 1 ? sd : s) : 0.0);
-      }
-      double fg = (Pa + q.P) * iv.rhob * mPa;  // ∂v∂t! (:755-772)
-      {                                        // ∂v∂t_av! (:869-897), on approaching pairs
-        const double dmu = C.h * fmin(dvdx, 0.0) * iv.den;
-        const double dPi = (-C.alpha * C.c0 * dmu) * (2.0 * iv.sum);
-        fg -= both ? dPi * C.m0 : 0.0;
-      }
-      fg = same_kind(pta, ptb) ? fg * dwr : 0.0;
-      double ax[3] = {0.0, 0.0, 0.0};
-      if (both) {
-        if (F.nu_on) {  // ∂v∂t_visc! (:967-980)
-          const double term = 4 * C.nu * C.m0 * (r2 * dwr) * (iv.sum * iv.den);
-#pragma unroll
-          for (int d = 0; d < D; ++d) ax[d] += term * dv[d];
-        }
-        if (F.s_on && r2 < C.st_t2) fg += surf_d(r, C) * (1.0 / C.m0);  // ∂v∂tpF! (:1387-1397)
-      }
-#pragma unroll
-      for (int d = 0; d < D; ++d) ax[d] += fg * dx[d];
-      if ((pta > 0) != (ptb > 0) && r2 < C.fb_t2[0]) {  // fbmolforce! (:1891-1901)
-        double q1 = C.fb_r0[0] / (r + C.fb_eta2[0]);
-        double Fc = C.fb_d[0] * (powi_d(q1, 12) - powi_d(q1, 4)) / (r2 + C.fb_eta2[0]);
-#pragma unroll
-        for (int d = 0; d < D; ++d) ax[d] += dx[d] * Fc;
-      }
-#pragma unroll
-      for (int d = 0; d < D; ++d) acc[d].add(ax[d]);
+      const double r2 = dist2_of<D>(dx);
+      pair_terms<D, G7, true>(C, F, own, q, q.rho, q.pt, q.P, dx, dv, dx, r2, root_of(r2), 0, t);
     });
     // ∂v∂t_addgrav!, then the half-step updates (:270-274)
     double av[3];
 #pragma unroll
-    for (int d = 0; d < D; ++d) av[d] = acc[d].get();
+    for (int d = 0; d < D; ++d) av[d] = sum.get(d);
+    if (!writer) return;
     av[1] = av[1] - C.g;
     double rh0, vh0[3], xh0[3];
     if (F.synced_prev) {
-      rh0 = rhoa;
+      rh0 = sa;
 #pragma unroll
       for (int d = 0; d < D; ++d) {
         vh0[d] = va[d];
@@ -148,7 +105,7 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W))) void k_
       }
     }
     const double hdt = dt * 0.5;
-    double rv = rh0 + drho.get() * hdt;
+    double rv = rh0 + sum.get(kDrho) * hdt;
     if (rv < C.rho0 && pta < 0) rv = C.rho0;
     const double Ph = eos_d(rv, pta, C);
     B.RH[a] = rv;
@@ -172,91 +129,30 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W))) void k_
     st_rec(B.PRH, a, rec, B.n);
   } else {
     // ---------------- FP32-split
-#pragma clang fp contract(fast)
-    const float dra = sa;
-    const float rhoa = C.f_rho0 + dra;
-    const float inv_rhoa = __builtin_amdgcn_rcpf(rhoa);
-    const float mPa = -C.f_m0 * inv_rhoa;  // -m0/ρ_a of the pressure term
-    const float Pa = B.PN[a];
+    const Own<R> own = own_of<R>(sa, B.PN[a], pta, C);
     using Nb = PartnerN<D>;
     auto fetch = [&](const int32_t b) { return ld_rec<Nb>(B.PRN, b, B.n); };
     const FrameK3 kt = particle_k<D, R>(B, C, G, a, xa);
-    // ∇W = dx·dwr, so every term along ∇W is gathered into one coefficient fg
-    // of dx, and dx·∇W = r²·dwr, dv·∇W = (dv·dx)·dwr.
-    for_each_partner_fetch<Pipe, D, R, true>(B, a, nc, G, XM, C.dist2, fetch, [&](const int32_t, const Nb& q, const auto&... win) {
-      const int32_t ptb = rec_pt(q);
+    const auto sum = sum_partners<Pipe, Quad, D, D + 1, R, true>(B, a, nc, G, XM, C.dist2, fetch,
+                                                                 [&](const Nb& q, auto& t, const auto&... win) {
       float dx[3], dv[3];
 #pragma unroll
       for (int d = 0; d < D; ++d) {
         dx[d] = sep_x(xa, q, d, win...);
         dv[d] = va[d] - q.v[d];
       }
-      const float r2 = dotf<D>(dx, dx);
-      const float r = __builtin_amdgcn_sqrtf(r2);
-      const float dwr = dWr_f(r * C.f_Hinv, C.f_dwr);
-      const float inv_den = __builtin_amdgcn_rcpf(r2 + C.f_eta2);
-      const float dvdx = dotf<D>(dv, dx);
-      const float drb = q.rho;
-      const float rhob = C.f_rho0 + drb;
-      const RhoInv ri = rho_inv2(rhoa, rhob);
-      const float inv_rhob = ri.inv_rhob;
-      // The common terms are evaluated for every pair and selected (no
-      // divergent branches in the hot loop): continuity + δ-SPH, pressure, AV.
-      const bool both = pta > 0 && ptb > 0;
-      float ax[3] = {0.0f, 0.0f, 0.0f};
-      {
-        const float s = C.f_m0 * dwr * dvdx;
-        const float drhop = hydro_drho_f(C.f_DDTgz * dx[1], C.f_rho0);
-        const float vd = C.f_DDTkh * ((drb - dra) - drhop) * inv_den;
-        const float sd = s - vd * (r2 * dwr) * C.f_m0 * inv_rhob;
-        drho.add(both ? (pta > 1 ? sd : s) : 0.0f);
-      }
-      const float Pt = (Pa + rec_P(q, C)) * inv_rhob * mPa;
-      float fg = same_kind(pta, ptb) ? Pt : 0.0f;
-      {
-        const float dmu = C.f_h * fminf(dvdx, 0.0f) * inv_den;  // AV acts on approaching pairs only
-        const float dPi = (-C.f_alpha * C.f_c0 * dmu) * (2.0f * ri.inv_sum);
-        fg -= both ? dPi * C.f_m0 : 0.0f;
-      }
-      if (both) {
-        if (F.nu_on) {
-          float term = 4.0f * C.f_nu * C.f_m0 * (r2 * dwr) * (ri.inv_sum * inv_den);
-#pragma unroll
-          for (int d = 0; d < D; ++d) ax[d] += term * dv[d];
-        }
-      }
-      fg *= dwr;
-      if (both && F.s_on && r < C.f_st_2h) fg += surf_f(r, C) * (1.0f / C.f_m0);
-#pragma unroll
-      for (int d = 0; d < D; ++d) ax[d] += fg * dx[d];
-      if ((pta > 0) != (ptb > 0) && r < C.f_fb_r0[0]) {
-        // wall force: FP32 while q = r0/(r + η²) < 32 (q^12 < 1.2e18, far inside
-        // the FP32 range), FP64 for the (rare) closer pairs
-        const float q1 = C.f_fb_r0[0] * __builtin_amdgcn_rcpf(r + C.f_fb_eta2[0]);
-        if (q1 < 32.0f) {
-          const float q2 = q1 * q1, q4 = q2 * q2, q8 = q4 * q4;
-          const float Fc = C.f_fb_d[0] * (q4 * q8 - q4) * __builtin_amdgcn_rcpf(r2 + C.f_fb_eta2[0]);
-#pragma unroll
-          for (int d = 0; d < D; ++d) ax[d] += dx[d] * Fc;
-        } else {
-          double p1 = C.fb_r0[0] / (double(r) + C.fb_eta2[0]);
-          double p2 = p1 * p1, p4 = p2 * p2, p8 = p4 * p4;
-          double Fc = C.fb_d[0] * (p4 * p8 - p4) / (double(r2) + C.fb_eta2[0]);
-#pragma unroll
-          for (int d = 0; d < D; ++d) ax[d] += float(double(dx[d]) * Fc);
-        }
-      }
-#pragma unroll
-      for (int d = 0; d < D; ++d) acc[d].add(ax[d]);
+      const float r2 = dist2_of<D>(dx);
+      pair_terms<D, G7, true>(C, F, own, q, q.rho, rec_pt(q), rec_P(q, C), dx, dv, dx, r2, root_of(r2), 0, t);
     }, &kt);
     float av[3];
 #pragma unroll
-    for (int d = 0; d < D; ++d) av[d] = acc[d].get();
+    for (int d = 0; d < D; ++d) av[d] = sum.get(d);
+    if (!writer) return;
     av[1] = av[1] - C.f_g;
     float rh0, vh0[3];
     double xh0[3];
     if (F.synced_prev) {
-      rh0 = dra;
+      rh0 = sa;
 #pragma unroll
       for (int d = 0; d < D; ++d) {
         vh0[d] = va[d];
@@ -272,7 +168,7 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W))) void k_
       }
     }
     const float hdt = float(dt * 0.5);
-    float rv = rh0 + drho.get() * hdt;
+    float rv = fma_(sum.get(kDrho), hdt, rh0);
     if (rv < 0.0f && pta < 0) rv = 0.0f;
     B.RH[a] = rv;
     const float Ph = eos_f(rv, pta, C);
@@ -283,8 +179,8 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W))) void k_
 #pragma unroll
     for (int d = 0; d < D; ++d) {
       float vv = vh0[d];
-      if (pta > 1) vv += av[d] * hdt;
-      const double xh = xh0[d] + double(vv) * (dt * 0.5);
+      if (pta > 1) vv = fma_(av[d], hdt, vv);
+      const double xh = fma_(double(vv), dt * 0.5, xh0[d]);
       B.VH[d][a] = vv;
       B.XH[d][a] = xh;
       put_x(rec.h, d, xh, fr);
@@ -299,10 +195,10 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W))) void k_
 }
 
 // ---- pass 2 + symplectic update ------------------------------------------
-template <int D, typename R, typename SS, bool Pipe, int W, int BS, bool G7>
+template <int D, typename R, typename SS, bool Pipe, int W, int BS, bool G7, bool Quad>
 __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W))) void k_pass2(SS ss) {
 #pragma clang fp contract(off)
-  GCLSPH_SCENE_BS(ss, BS);
+  GCLSPH_SCENE_PAIR(ss, BS, Quad);
   StepCtl* ctl = B.ctl;
   const int p = ctl->parity, q = p ^ 1, pp = ctl->pparity, rebuilt = ctl->rebuilt;
   const double dt = ctl->dt;
@@ -326,19 +222,18 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W))) void k_
     }
     const R sha = RH[a];
     const int32_t pta = PT[a];
-    Sum<R> acc[3], drho;
+    constexpr int kDrho = D;  // sums: D accelerations, ∂ρ/∂t
     const int nc = B.NC[a];
     R av[3];
     R Pha, drho_v;
     if constexpr (std::is_same<R, double>::value) {
       const double rhoa = sha;
-      const double mPa = -C.m0 * (1.0 / rhoa);
       Pha = B.PH[a];
+      const Own<R> own = own_of<R>(sha, Pha, pta, C);
       using Nb = PartnerH64<D>;
       auto fetch = [&](const int32_t b) { return ld_rec<Nb>(B.PRH, b, B.n); };
-      for_each_partner_fetch<Pipe, D>(B, a, nc, G, XM, C.dist2, fetch, [&](const int32_t, const Nb& q) {
-#pragma clang fp contract(fast)
-        const int32_t ptb = q.pt;
+      const auto sum = sum_partners<Pipe, Quad, D, D + 1, R>(B, a, nc, G, XM, C.dist2, fetch,
+                                                             [&](const Nb& q, auto& t) {
         double dxn[3], dx[3], dv[3];
 #pragma unroll
         for (int d = 0; d < D; ++d) {
@@ -346,108 +241,64 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W))) void k_
           dx[d] = xha[d] - q.xh[d];
           dv[d] = vha[d] - q.vh[d];
         }
-        // ∇W from pass 1 (positions xⁿ, src/sphproblem.jl:246,281): dxn·dwr
-        const double r2n = dotd<D>(dxn, dxn);
-        const double rn = sqrt_d(r2n);
-        const double dwr = dWr_d(r2n, rn, C);
-        const double r2 = dotd<D>(dx, dx);
-        const double rhob = q.rh;
-        const Inv3 iv = pair_inv(q, rhoa + rhob, r2 + C.eta2);
-        const double dvdx = dotm<D>(dv, dx);
-        const double dxg = dotm<D>(dx, dxn) * dwr;  // dx·∇W
-        const bool both = pta > 0 && ptb > 0;
-        {
-          const double s = C.m0 * dwr * dotm<D>(dv, dxn);
-          const double vd = C.DDTkh * ((rhob - rhoa) - hydro_drho_d<G7>(C.DDTgz * dx[1], C)) * iv.den;
-          const double sd = s - vd * dxg * (C.m0 * iv.rhob);
-          drho.add(both ? (pta > 1 ? sd : s) : 0.0);
-        }
-        double fg = (Pha + q.P) * iv.rhob * mPa;
-        {
-          const double dmu = C.h * fmin(dvdx, 0.0) * iv.den;
-          const double dPi = (-C.alpha * C.c0 * dmu) * (2.0 * iv.sum);
-          fg -= both ? dPi * C.m0 : 0.0;
-        }
-        fg = same_kind(pta, ptb) ? fg * dwr : 0.0;
-        double ax[3] = {0.0, 0.0, 0.0};
-        if (both) {
-          if (F.nu_on) {
-            const double term = 4 * C.nu * C.m0 * dxg * (iv.sum * iv.den);
-#pragma unroll
-            for (int d = 0; d < D; ++d) ax[d] += term * dv[d];
-          }
-          if (F.s_on && r2 < C.st_t2) {
-            const double scos = surf_d(sqrt_d(r2), C) * (1.0 / C.m0);
-#pragma unroll
-            for (int d = 0; d < D; ++d) ax[d] += scos * dx[d];
-          }
-        }
-#pragma unroll
-        for (int d = 0; d < D; ++d) ax[d] += fg * dxn[d];
-        // fbmolforce! at xⁿ with (bound_D, bound_l) (src/sphproblem.jl:295)
-        if ((pta > 0) != (ptb > 0) && r2n < C.fb_t2[1]) {
-          double q1 = C.fb_r0[1] / (rn + C.fb_eta2[1]);
-          double Fc = C.fb_d[1] * (powi_d(q1, 12) - powi_d(q1, 4)) / (r2n + C.fb_eta2[1]);
-#pragma unroll
-          for (int d = 0; d < D; ++d) ax[d] += dxn[d] * Fc;
-        }
-#pragma unroll
-        for (int d = 0; d < D; ++d) acc[d].add(ax[d]);
+        // ∇W from pass 1 (positions xⁿ, src/sphproblem.jl:246,281); the wall
+        // force at xⁿ with (bound_D, bound_l) (:295)
+        const double r2n = dist2_of<D>(dxn);
+        pair_terms<D, G7, false>(C, F, own, q, q.rh, q.pt, q.P, dx, dv, dxn, r2n, root_of(r2n), 1, t);
       });
 #pragma unroll
-      for (int d = 0; d < D; ++d) av[d] = acc[d].get();
+      for (int d = 0; d < D; ++d) av[d] = sum.get(d);
       av[1] = av[1] - C.g;
-      drho_v = drho.get();
-      // symplectic_update! (src/gpukernels_sph.jl:1204-1245)
-      const double epsi = -(drho_v / rhoa) * dt;
-      double rv = B.RHO[p][a] * (2 - epsi) / (2 + epsi);
-      if (rv < C.rho0 && pta <= 1) rv = C.rho0;
-      const double Pn = eos_d(rv, pta, C);
-      B.RHO[q][a] = rv;
-      B.PN[a] = Pn;
-      if (F.corr_on) B.RH2[a] = rv;
-      const double ml = pta > 1 ? 1.0 : 0.0;
-      double xn[3], vn[3];
-      PartnerN64<D> rec{};
+      drho_v = sum.get(kDrho);
+      if (writer) {
+        // symplectic_update! (src/gpukernels_sph.jl:1204-1245)
+        const double epsi = -(drho_v / rhoa) * dt;
+        double rv = B.RHO[p][a] * (2 - epsi) / (2 + epsi);
+        if (rv < C.rho0 && pta <= 1) rv = C.rho0;
+        const double Pn = eos_d(rv, pta, C);
+        B.RHO[q][a] = rv;
+        B.PN[a] = Pn;
+        if (F.corr_on) B.RH2[a] = rv;
+        const double ml = pta > 1 ? 1.0 : 0.0;
+        double xn[3], vn[3];
+        PartnerN64<D> rec{};
 #pragma unroll
-      for (int d = 0; d < D; ++d) {
-        double vv = B.V[p][d][a];
-        double nv = vv + av[d] * dt * ml;
-        double dd = (vv + nv) * 0.5 * dt;
-        double cd = dd;
-        if (F.need_cdx) {
-          cd = (rebuilt ? 0.0 : B.CDX[d][a]) + dd;
-          B.CDX[d][a] = cd;
+        for (int d = 0; d < D; ++d) {
+          double vv = B.V[p][d][a];
+          double nv = vv + av[d] * dt * ml;
+          double dd = (vv + nv) * 0.5 * dt;
+          double cd = dd;
+          if (F.need_cdx) {
+            cd = (rebuilt ? 0.0 : B.CDX[d][a]) + dd;
+            B.CDX[d][a] = cd;
+          }
+          red_cdx = fmax(red_cdx, fabs(cd)) + (cd != cd ? cd : 0.0);
+          double xv = xa[d] + dd;
+          xn[d] = xv;
+          vn[d] = nv;
+          B.V[q][d][a] = nv;
+          B.X[q][d][a] = xv;
+          rec.x[d] = xv;
+          rec.v[d] = nv;
+          if (F.corr_on) {
+            B.VH2[d][a] = nv;
+            B.XH2[d][a] = xv;
+          }
         }
-        red_cdx = fmax(red_cdx, fabs(cd)) + (cd != cd ? cd : 0.0);
-        double xv = xa[d] + dd;
-        xn[d] = xv;
-        vn[d] = nv;
-        B.V[q][d][a] = nv;
-        B.X[q][d][a] = xv;
-        rec.x[d] = xv;
-        rec.v[d] = nv;
-        if (F.corr_on) {
-          B.VH2[d][a] = nv;
-          B.XH2[d][a] = xv;
+        rec.rho = rv;
+        rec.P = Pn;
+        rec.pt = pta;
+        set_irho(rec);
+        st_rec(B.PRN, a, rec, B.n);  // partner record of the next step's pass 1
+        if (F.ts) {
+          red_acc = sqrt(dotd<D>(av, av));
+          if (F.visc_in_pass2) red_visc = fabs(C.h * dotd<D>(vn, xn) / (dotd<D>(xn, xn) + C.dt_eta2));
         }
-      }
-      rec.rho = rv;
-      rec.P = Pn;
-      rec.pt = pta;
-      set_irho(rec);
-      st_rec(B.PRN, a, rec, B.n);  // partner record of the next step's pass 1
-      if (F.ts) {
-        red_acc = sqrt(dotd<D>(av, av));
-        if (F.visc_in_pass2) red_visc = fabs(C.h * dotd<D>(vn, xn) / (dotd<D>(xn, xn) + C.dt_eta2));
       }
     } else {
-#pragma clang fp contract(fast)
-      const float dra = sha;
-      const float rhoa = C.f_rho0 + dra;
-      const float inv_rhoa = __builtin_amdgcn_rcpf(rhoa);
-      const float mPa = -C.f_m0 * inv_rhoa;  // -m0/ρ_a of the pressure term
+      const float rhoa = C.f_rho0 + sha;
       Pha = B.PH[a];
+      const Own<R> own = own_of<R>(sha, Pha, pta, C);
       // tⁿ separation from the half-step state when x½ = xⁿ + v½·Δt/2, else
       // from the displacement x½ - xⁿ that pass 1 appended to the records
       // xⁿa - xⁿb = (x½a - x½b) - (da - db) with d = x½ - xⁿ, the displacement
@@ -463,143 +314,79 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W))) void k_
       constexpr bool derive = decltype(derive_c)::value;
       using Nb = std::conditional_t<derive, PartnerH<D>, PartnerHX<D>>;
       auto fetch = [&](const int32_t b) { return ld_rec<Nb>(B.PRH, b, B.n); };
-      for_each_partner_fetch<Pipe, D, R, true>(B, a, nc, G, XM, C.dist2, fetch, [&](const int32_t, const Nb& r,
-                                                                            const auto&... win) {
+      return sum_partners<Pipe, Quad, D, D + 1, R, true>(B, a, nc, G, XM, C.dist2, fetch,
+                                                         [&](const Nb& r, auto& t, const auto&... win) {
         const PartnerH<D>* qp;
         if constexpr (derive) qp = &r;
         else qp = &r.h;
         const PartnerH<D>& q = *qp;
-        const int32_t ptb = rec_pt(q);
         float dxn[3], dx[3], dv[3];
 #pragma unroll
         for (int d = 0; d < D; ++d) {
           dx[d] = sep_x(xha, q, d, win...);
           dv[d] = vha[d] - q.vh[d];
-          if constexpr (derive) dxn[d] = dx[d] - dv[d] * fhdt;
+          if constexpr (derive) dxn[d] = fma_(-dv[d], fhdt, dx[d]);
           else dxn[d] = dx[d] - (dna[d] - r.dn[d]);
         }
-        // ∇W from pass 1 (positions xⁿ): ∇W = dxn·dwr; terms along ∇W are
-        // gathered into one coefficient fg of dxn
-        const float r2n = dotf<D>(dxn, dxn);
-        const float rn = __builtin_amdgcn_sqrtf(r2n);
-        const float dwr = dWr_f(rn * C.f_Hinv, C.f_dwr);
-        const float r2 = dotf<D>(dx, dx);
-        const float inv_den = __builtin_amdgcn_rcpf(r2 + C.f_eta2);
-        const float dvdx = dotf<D>(dv, dx);
-        const float drb = q.rh;
-        const float rhob = C.f_rho0 + drb;
-        const RhoInv ri = rho_inv2(rhoa, rhob);
-        const float inv_rhob = ri.inv_rhob;
-        // common terms evaluated for every pair and selected, as in pass 1
-        const bool both = pta > 0 && ptb > 0;
-        float ax[3] = {0.0f, 0.0f, 0.0f};
-        const float dxg = dotf<D>(dx, dxn) * dwr;  // dx·∇W
-        {
-          const float s = C.f_m0 * dwr * dotf<D>(dv, dxn);
-          const float drhop = hydro_drho_f(C.f_DDTgz * dx[1], C.f_rho0);
-          const float vd = C.f_DDTkh * ((drb - dra) - drhop) * inv_den;
-          const float sd = s - vd * dxg * C.f_m0 * inv_rhob;
-          drho.add(both ? (pta > 1 ? sd : s) : 0.0f);
-        }
-        if (both) {
-          if (F.nu_on) {
-            float term = 4.0f * C.f_nu * C.f_m0 * dxg * (ri.inv_sum * inv_den);
-#pragma unroll
-            for (int d = 0; d < D; ++d) ax[d] += term * dv[d];
-          }
-          if (F.s_on) {
-            const float r = __builtin_amdgcn_sqrtf(r2);
-            if (r < C.f_st_2h) {
-              const float scos = surf_f(r, C);
-#pragma unroll
-              for (int d = 0; d < D; ++d) ax[d] += scos * dx[d] * (1.0f / C.f_m0);
-            }
-          }
-        }
-        const float Pt = (Pha + rec_P(q, C)) * inv_rhob * mPa;
-        float fg = same_kind(pta, ptb) ? Pt : 0.0f;
-        {
-          const float dmu = C.f_h * fminf(dvdx, 0.0f) * inv_den;
-          const float dPi = (-C.f_alpha * C.f_c0 * dmu) * (2.0f * ri.inv_sum);
-          fg -= both ? dPi * C.f_m0 : 0.0f;
-        }
-        fg *= dwr;
-#pragma unroll
-        for (int d = 0; d < D; ++d) ax[d] += fg * dxn[d];
-        if ((pta > 0) != (ptb > 0) && rn < C.f_fb_r0[1]) {
-          // wall force: FP32 while q < 32, FP64 for closer pairs (as in pass 1)
-          const float q1 = C.f_fb_r0[1] * __builtin_amdgcn_rcpf(rn + C.f_fb_eta2[1]);
-          if (q1 < 32.0f) {
-            const float q2 = q1 * q1, q4 = q2 * q2, q8 = q4 * q4;
-            const float Fc = C.f_fb_d[1] * (q4 * q8 - q4) * __builtin_amdgcn_rcpf(r2n + C.f_fb_eta2[1]);
-#pragma unroll
-            for (int d = 0; d < D; ++d) ax[d] += dxn[d] * Fc;
-          } else {
-            double p1 = C.fb_r0[1] / (double(rn) + C.fb_eta2[1]);
-            double p2 = p1 * p1, p4 = p2 * p2, p8 = p4 * p4;
-            double Fc = C.fb_d[1] * (p4 * p8 - p4) / (double(r2n) + C.fb_eta2[1]);
-#pragma unroll
-            for (int d = 0; d < D; ++d) ax[d] += float(double(dxn[d]) * Fc);
-          }
-        }
-#pragma unroll
-        for (int d = 0; d < D; ++d) acc[d].add(ax[d]);
+        const float r2n = dist2_of<D>(dxn);
+        pair_terms<D, G7, false>(C, F, own, q, q.rh, rec_pt(q), rec_P(q, C), dx, dv, dxn, r2n, root_of(r2n), 1, t);
       }, &kt);
       };
-      if (F.synced_prev) gather(std::true_type{});
-      else gather(std::false_type{});
+      const auto sum = F.synced_prev ? gather(std::true_type{}) : gather(std::false_type{});
 #pragma unroll
-      for (int d = 0; d < D; ++d) av[d] = acc[d].get();
+      for (int d = 0; d < D; ++d) av[d] = sum.get(d);
       av[1] = av[1] - C.f_g;
-      drho_v = drho.get();
-      // symplectic update on δρ: ρ(2-ε)/(2+ε) - ρ0 = (2δρ - ε(2ρ0 + δρ)) / (2 + ε)
-      const float fdt = float(dt);
-      const float epsi = -(drho_v / rhoa) * fdt;
-      const float dr_n = B.RHO[p][a];
-      float rv = (2.0f * dr_n - epsi * (2.0f * C.f_rho0 + dr_n)) / (2.0f + epsi);
-      if (rv < 0.0f && pta <= 1) rv = 0.0f;
-      B.RHO[q][a] = rv;
-      const float Pn = eos_f(rv, pta, C);
-      B.PN[a] = Pn;
-      if (F.corr_on) B.RH2[a] = rv;
-      const float ml = pta > 1 ? 1.0f : 0.0f;
-      double xn[3], vn[3];
-      PartnerN<D> rec{};
-      double fr[3];
-      particle_frame<D, R>(B, C, G, a, fr);
+      drho_v = sum.get(kDrho);
+      if (writer) {
+        // symplectic update on δρ: ρ(2-ε)/(2+ε) - ρ0 = (2δρ - ε(2ρ0 + δρ)) / (2 + ε)
+        const float fdt = float(dt);
+        const float erate = -(drho_v / rhoa), epsi = erate * fdt;
+        const float dr_n = B.RHO[p][a];
+          float rv = fma_(2.0f, dr_n, -(epsi * fma_(2.0f, C.f_rho0, dr_n))) / fma_(erate, fdt, 2.0f);
+        if (rv < 0.0f && pta <= 1) rv = 0.0f;
+        B.RHO[q][a] = rv;
+        const float Pn = eos_f(rv, pta, C);
+        B.PN[a] = Pn;
+        if (F.corr_on) B.RH2[a] = rv;
+        const float ml = pta > 1 ? 1.0f : 0.0f;
+        double xn[3], vn[3];
+        PartnerN<D> rec{};
+        double fr[3];
+        particle_frame<D, R>(B, C, G, a, fr);
 #pragma unroll
-      for (int d = 0; d < D; ++d) {
-        float vv = B.V[p][d][a];
-        float nv = vv + av[d] * fdt * ml;
-        double dd = (double(vv) + double(nv)) * 0.5 * dt;
-        double cd = dd;
-        if (F.need_cdx) {
-          cd = (rebuilt ? 0.0 : B.CDX[d][a]) + dd;
-          B.CDX[d][a] = cd;
+        for (int d = 0; d < D; ++d) {
+          float vv = B.V[p][d][a];
+          float nv = fma_(av[d] * fdt, ml, vv);
+          const double vm = (double(vv) + double(nv)) * 0.5;
+          double cd = vm * dt;
+          if (F.need_cdx) {
+            cd = fma_(vm, dt, rebuilt ? 0.0 : B.CDX[d][a]);
+            B.CDX[d][a] = cd;
+          }
+          red_cdx = fmax(red_cdx, fabs(cd)) + (cd != cd ? cd : 0.0);
+          const double xv = fma_(vm, dt, xa[d]);
+          xn[d] = xv;
+          vn[d] = nv;
+          B.V[q][d][a] = nv;
+          B.X[q][d][a] = xv;
+          put_x(rec, d, xv, fr);
+          rec.v[d] = nv;
+          if (F.corr_on) {
+            B.VH2[d][a] = nv;
+            B.XH2[d][a] = xv;
+          }
         }
-        red_cdx = fmax(red_cdx, fabs(cd)) + (cd != cd ? cd : 0.0);
-        double xv = xa[d] + dd;
-        xn[d] = xv;
-        vn[d] = nv;
-        B.V[q][d][a] = nv;
-        B.X[q][d][a] = xv;
-        put_x(rec, d, xv, fr);
-        rec.v[d] = nv;
-        if (F.corr_on) {
-          B.VH2[d][a] = nv;
-          B.XH2[d][a] = xv;
+        rec.rho = rv;
+        set_pt(rec, pta, Pn);
+        st_rec(B.PRN, a, rec, B.n);  // partner record of the next step's pass 1
+        if (F.ts) {
+          float a2 = dotf<D>(av, av);
+          red_acc = sqrt(double(a2));
+          if (F.visc_in_pass2) red_visc = fabs(C.h * dotd<D>(vn, xn) / (dotd<D>(xn, xn) + C.dt_eta2));
         }
-      }
-      rec.rho = rv;
-      set_pt(rec, pta, Pn);
-      st_rec(B.PRN, a, rec, B.n);  // partner record of the next step's pass 1
-      if (F.ts) {
-        float a2 = dotf<D>(av, av);
-        red_acc = sqrt(double(a2));
-        if (F.visc_in_pass2) red_visc = fabs(C.h * dotd<D>(vn, xn) / (dotd<D>(xn, xn) + C.dt_eta2));
       }
     }
-    if (F.want_out) {
+    if (F.want_out && writer) {
 #pragma unroll
       for (int d = 0; d < D; ++d) B.ACC[d][a] = av[d];
       B.DRHO[a] = drho_v;
@@ -621,16 +408,16 @@ template <int BS>
 unsigned pass_grid(const LaunchSet& L) {
   return BS == 256 ? L.pblocks : BS == 128 ? 2 * L.pblocks : L.pblocks512;
 }
-template <int D, typename R, bool Pipe, int W, int BS, bool G7 = true>
+template <int D, typename R, bool Pipe, int W, int BS, bool G7 = true, bool Quad = false>
 void pass1_as(const LaunchSet& L, hipStream_t s, size_t lds) {
   with_scenes<R>(L, [&](auto ss) {
-    k_pass1<D, R, decltype(ss), Pipe, W, BS, G7><<<pass_grid<BS>(L), BS, lds, s>>>(ss);
+    k_pass1<D, R, decltype(ss), Pipe, W, BS, G7, Quad><<<Quad ? L.qblocks : pass_grid<BS>(L), BS, lds, s>>>(ss);
   });
 }
-template <int D, typename R, bool Pipe, int W, int BS, bool G7 = true>
+template <int D, typename R, bool Pipe, int W, int BS, bool G7 = true, bool Quad = false>
 void pass2_as(const LaunchSet& L, hipStream_t s, size_t lds) {
   with_scenes<R>(L, [&](auto ss) {
-    k_pass2<D, R, decltype(ss), Pipe, W, BS, G7><<<pass_grid<BS>(L), BS, lds, s>>>(ss);
+    k_pass2<D, R, decltype(ss), Pipe, W, BS, G7, Quad><<<Quad ? L.qblocks : pass_grid<BS>(L), BS, lds, s>>>(ss);
   });
 }
 // Unused dynamic LDS per block of BS threads that leaves room for at most
@@ -686,6 +473,10 @@ void launch_pass1(const LaunchSet& L, hipStream_t s, int variant) {
       return;
     }
   }
+  if (variant == kPassQuad) {
+    pass1_as<D, R, true, 1, 256, true, true>(L, s, 0);
+    return;
+  }
   const int cg = variant % kPassCodegen, bs = pass_block_size(variant);
   const size_t lds = pass_cap(variant) ? cap_lds(bs) : 0;
   switch (bs) {
@@ -701,6 +492,10 @@ void launch_pass2(const LaunchSet& L, hipStream_t s, int variant) {
       pass2_as<D, R, false, 1, 256, false>(L, s, 0);
       return;
     }
+  }
+  if (variant == kPassQuad) {
+    pass2_as<D, R, true, 1, 256, true, true>(L, s, 0);
+    return;
   }
   const int cg = variant % kPassCodegen, bs = pass_block_size(variant);
   const size_t lds = pass_cap(variant) ? cap_lds(bs) : 0;

@@ -519,6 +519,38 @@ def test_pass_variants_bit_identical(G, monkeypatch, prec):
             assert np.array_equal(np.asarray(a), np.asarray(b)), v
 
 
+@pytest.mark.parametrize("prec", ["f64", "f32split"])
+@pytest.mark.parametrize("case", ["dam2d", "dam2d_allphys", "dam3d_allphys", 1, 3, 63, 65, 129])
+def test_pair_quads_equal_one_lane(G, S, monkeypatch, prec, case):
+    """Small problems give a particle four lanes in the pair kernels, which add
+    their terms in the order of one lane: bit-identical steps, from the
+    membership store and (GCLSPH_NMASK_CAP) the stencil scan, with every
+    correction, skipped rebuilds, and particle counts around a block of 64."""
+    if isinstance(case, int):
+        k = np.arange(case)
+        p, dist = S.standard_params(0.02, 2)
+        p.xsph_eps, p.cspmn, p.dpc_l0 = 0.5, 2, 0.03
+        x = 0.1 + (k % 9) * 0.02 + 0.004 * S.uniform01(7, case, 0)
+        y = 0.1 + (k // 9) * 0.02 + 0.004 * S.uniform01(7, case, 1)
+        sc, steps, ts = S.Scene(2, (x, y), np.full(case, 1001.0), np.where(k % 7 == 3, 1, 2), p, dist, (dist, dist)), 5, True
+    else:
+        sc, steps, ts = golden_cases()[case]
+
+    def run(lanes, cap=None):
+        monkeypatch.setenv("GCLSPH_PAIR_LANES", lanes)
+        if cap is not None:
+            monkeypatch.setenv("GCLSPH_NMASK_CAP", str(cap))
+        cl = G.GPUCellList(sc.points, sc.cellsize, sc.dist)
+        prob = G.SPHProblem.from_params(cl, sc.params, sc.rho, sc.ptype, v=sc.v, precision=prec)
+        out = [G.stepsolve_(prob, n, timestepping=ts) for n in (1, steps + 1)]
+        return out + [np.asarray(gpu_fields(G, prob)[f]) for f in FIELDS]
+
+    ref = run("1")
+    for cap in (None, 2, 0):
+        for a, b in zip(run("4", cap), ref):
+            assert np.array_equal(np.asarray(a), np.asarray(b), equal_nan=True)
+
+
 @pytest.mark.parametrize("n", [1, 2, 63, 65, 257, 1000])
 def test_tiny_and_ragged_problems(G, O, S, n):
     """Problems of 1 and 2 particles and counts that leave the last wave or
