@@ -66,12 +66,13 @@ void gather(const T* src, T* dst, const int32_t* perm, int64_t n, hipStream_t s)
   GCL_HIP(hipGetLastError());
 }
 
-__global__ void k_maxpairs(const int32_t* __restrict__ cnt, CellGeom g, unsigned long long* out) {
+__global__ void k_maxpairs(const int32_t* __restrict__ start, CellGeom g, unsigned long long* out) {
   int64_t c = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   int64_t nc = g.ncells();
   long long val = 0;
   if (c < nc) {
-    int32_t nn = cnt[c];
+    auto points = [&](int64_t i) { return start[i + 1] - start[i]; };
+    int32_t nn = points(c);
     if (nn > 0) {
       // мaxpairs half stencil (src/gpukernels_cls.jl:130-167, :184-286)
       const int o2[4][3] = {{-1, 1, 0}, {0, 1, 0}, {1, 1, 0}, {1, 0, 0}};
@@ -84,7 +85,7 @@ __global__ void k_maxpairs(const int32_t* __restrict__ cnt, CellGeom g, unsigned
       for (int o = 0; o < no; ++o) {
         const int* off = g.dim == 2 ? o2[o] : o3[o];
         int64_t jx = ix + off[0], jy = iy + off[1], jz = iz + off[2];
-        if (jx >= 0 && jx < gx && jy >= 0 && jy < gy && jz >= 0 && jz < gz) m += cnt[jx + gx * (jy + gy * jz)];
+        if (jx >= 0 && jx < gx && jy >= 0 && jy < gy && jz >= 0 && jz < gz) m += points(jx + gx * (jy + gy * jz));
       }
       val = (long long)(double(int32_t(nn * (nn - 1))) * 0.5) + m * (long long)nn;
     }
@@ -141,6 +142,7 @@ struct gcl_s {
   hipStream_t stream = nullptr;
   sph_s* attached = nullptr;
   bool pairs_valid = true;
+  int32_t maxpoint = 0;  // read back from sb.maxcell with the pair count
 
   size_t tsize() const { return prec == 32 ? 4 : 8; }
 
@@ -183,15 +185,15 @@ struct gcl_s {
 
   // update! (src/celllist.jl:95-134) for a standalone cell list.
   void update(bool fillzero) {
-    bin_sort(G, prec, xo, n, false, sb, nullptr, stream, nullptr, nullptr, xs);
-    int32_t maxpoint = read_maxcell();
-    if (maxpoint > mppcell) mppcell = int64_t(std::ceil(double(maxpoint) * 1.05 + 1));
+    bin_sort(G, prec, xo, n, false, sb, stream, xs);
+    GCL_HIP(hipMemcpyAsync(&maxpoint, sb.maxcell, 4, hipMemcpyDeviceToHost, stream));
     bool fresh = false;  // a reallocated buffer is zero-filled whole
     if (pairsn > pb.capacity || double(pairsn) < double(pb.capacity) * 0.6) {
       pb.set_capacity(ceil_div08(pairsn), stream);
       fresh = true;
     }
-    int64_t total = count_pairs(xs);
+    const int64_t total = count_pairs(xs);
+    if (maxpoint > mppcell) mppcell = int64_t(std::ceil(double(maxpoint) * 1.05 + 1));
     if (total > pb.capacity) {
       pb.set_capacity(ceil_div08(total), stream);
       fresh = true;
@@ -606,6 +608,7 @@ struct sph_s {
     F.write_xrb = 1;
     upload_own<R>(make_const(0.0, 0.0), F);
     launch_rebuild<D, R>(own, stream);
+    launch_commit_rebuild<D, R>(own, stream);
     GCL_HIP(hipGetLastError());
     masks_valid = true;
     // per-particle arrays outside the reorder follow the new order
@@ -714,7 +717,7 @@ void LaunchSet::build(const int64_t* n, const int64_t* ncells, unsigned cnt, int
     blocks(pm, i, n[i], kBlock);
     blocks(pm512, i, n[i], 512);  // the pass kernels' 512-thread blocks
     if (quad) blocks(qm, i, n[i], 64);
-    blocks(cm, i, ncells[i] + 1, 1024);  // cnt[0..ncells] in 1024-cell tiles
+    blocks(cm, i, ncells[i], kTile);
   }
   for (auto* v : {&pm, &pm512, &qm})
     if (v->empty()) v->push_back(make_int2(0, 0));  // a no-op block (a >= n everywhere)
@@ -786,8 +789,6 @@ void run_steps(sph_s* const* P, unsigned count, LaunchSet& L, hipStream_t st, in
   if (count == 1) L.one = descs.data();
   else GCL_HIP(hipMemcpyAsync(L.scenes, descs.data(), sizeof(SceneDev<R>) * count, hipMemcpyHostToDevice, st));
   sph_s* timer = (count == 1 && P[0]->timing) ? P[0] : nullptr;
-  bool any_cspmn = false;
-  for (unsigned i = 0; i < count; ++i) any_cspmn |= flags[i].cspmn > 0;
   // Pass variants (same results, different code generation): forced by
   // GCLSPH_PASS_VARIANT=<pass1>,<pass2>, else the ones this launch set chose by
   // timing, else the fastest measured on the dam-break scenes per dimension
@@ -916,10 +917,12 @@ void run_steps(sph_s* const* P, unsigned count, LaunchSet& L, hipStream_t st, in
   if (graph) {
     // The step as a captured graph, replayed for the remaining steps: every
     // per-step decision lives in the control blocks, so one capture serves all
-    // steps.  Kept for the next call while the launches, pass variants and
-    // one-problem descriptor (baked into the graph) are unchanged.
-    std::vector<unsigned char> key = {uint8_t(any_dpc), uint8_t(any_xsph), uint8_t(any_cspmn), uint8_t(any_dtv),
-                                      uint8_t(pv[0]), uint8_t(pv[1]), uint8_t(L.gamma7)};
+    // steps but those that end with CSPM (every cspmn-th, 15 by default), which
+    // are launched: its two kernels cost a step that does not need them 9 us.
+    // Kept for the next call while the launches, pass variants and one-problem
+    // descriptor (baked into the graph) are unchanged.
+    std::vector<unsigned char> key = {uint8_t(any_dpc), uint8_t(any_xsph), uint8_t(any_dtv),
+                                      uint8_t(pv[0]),   uint8_t(pv[1]),    uint8_t(L.gamma7)};
     if (L.one) {
       const unsigned char* d = static_cast<const unsigned char*>(L.one);
       key.insert(key.end(), d, d + sizeof(SceneDev<R>));
@@ -929,14 +932,17 @@ void run_steps(sph_s* const* P, unsigned count, LaunchSet& L, hipStream_t st, in
       L.step_graph = nullptr;
       hipGraph_t g = nullptr;
       GCL_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-      launch_step(any_cspmn, pv[0], pv[1], nullptr);
+      launch_step(false, pv[0], pv[1], nullptr);
       GCL_HIP(hipStreamEndCapture(st, &g));
       const hipError_t e = hipGraphInstantiate(&L.step_graph, g, nullptr, nullptr, 0);
       (void)hipGraphDestroy(g);
       GCL_HIP(e);
       L.graph_key = std::move(key);
     }
-    for (int64_t it = done + 1; it <= nsteps; ++it) GCL_HIP(hipGraphLaunch(L.step_graph, st));
+    for (int64_t it = done + 1; it <= nsteps; ++it) {
+      if (cspm_at(it)) launch_step(true, pv[0], pv[1], nullptr);
+      else GCL_HIP(hipGraphLaunch(L.step_graph, st));
+    }
   } else {
     auto mark_begin = [&]() { return timer ? timer->mark_begin(st) : hipEvent_t(nullptr); };
     auto mark_end = [&](int stage, hipEvent_t e) {
@@ -1154,7 +1160,7 @@ int gcl_create(int dim, int prec, int64_t n, const double* const* pts, const dou
     g->sb.alloc(n, g->G.ncells());
     g->pb.alloc(n, dim == 2 && n <= kPairEntriesMaxPoints ? kPairEntries2D : 0);
     // cellmap! with the Float64 MIN (:55), then fillcells_naive! (:66)
-    bin_sort(g->G, prec, g->xo, n, true, g->sb, nullptr, g->stream, nullptr, nullptr, g->xs);
+    bin_sort(g->G, prec, g->xo, n, true, g->sb, g->stream, g->xs);
     int32_t maxc = g->read_maxcell();
     int64_t maxpoint = int64_t(std::ceil(double(maxc) * 1.05 + 1));  // :57-58
     g->mppcell = mppcell < maxpoint ? maxpoint : mppcell;
@@ -1162,7 +1168,7 @@ int gcl_create(int dim, int prec, int64_t n, const double* const* pts, const dou
       unsigned long long* d = nullptr;
       GCL_HIP(hipMalloc(&d, 8));
       GCL_HIP(hipMemsetAsync(d, 0, 8, g->stream));
-      k_maxpairs<<<grid_for(g->G.ncells()), kBlock, 0, g->stream>>>(g->sb.cnt, g->G, d);
+      k_maxpairs<<<grid_for(g->G.ncells()), kBlock, 0, g->stream>>>(g->sb.start, g->G, d);
       GCL_HIP(hipGetLastError());
       unsigned long long v = 0;
       GCL_HIP(hipMemcpyAsync(&v, d, 8, hipMemcpyDeviceToHost, g->stream));
@@ -1326,8 +1332,11 @@ int gcl_get_cellpnum(gcl_t h, int32_t* out) {
     GCL_CHECK(h != nullptr && out != nullptr, kErrArgument, "NULL argument");
     SortBuffers& sb = h->attached ? h->attached->sb : h->sb;
     hipStream_t s = h->attached ? h->attached->stream : h->stream;
-    GCL_HIP(hipMemcpyAsync(out, sb.cnt, 4 * size_t(h->G.ncells()), hipMemcpyDeviceToHost, s));
+    const size_t nc = size_t(h->G.ncells());
+    std::vector<int32_t> start(nc + 1);
+    GCL_HIP(hipMemcpyAsync(start.data(), sb.start, 4 * (nc + 1), hipMemcpyDeviceToHost, s));
     GCL_HIP(hipStreamSynchronize(s));
+    for (size_t c = 0; c < nc; ++c) out[c] = start[c + 1] - start[c];
   });
 }
 
@@ -1360,7 +1369,7 @@ int gcl_maxpairs(gcl_t h, int64_t* out) {
     unsigned long long* d = nullptr;
     GCL_HIP(hipMalloc(&d, 8));
     GCL_HIP(hipMemsetAsync(d, 0, 8, s));
-    k_maxpairs<<<grid_for(h->G.ncells()), kBlock, 0, s>>>(sb.cnt, h->G, d);
+    k_maxpairs<<<grid_for(h->G.ncells()), kBlock, 0, s>>>(sb.start, h->G, d);
     GCL_HIP(hipGetLastError());
     unsigned long long v = 0;
     GCL_HIP(hipMemcpyAsync(&v, d, 8, hipMemcpyDeviceToHost, s));
@@ -1408,8 +1417,6 @@ int sph_create(gcl_t system, int prec, const double* params, const double* rho, 
     }
     // cell structure of the system's last update!
     GCL_HIP(hipMemcpyAsync(P->sb.start, system->sb.start, 4 * size_t(P->G.ncells() + 1), hipMemcpyDeviceToDevice,
-                           P->stream));
-    GCL_HIP(hipMemcpyAsync(P->sb.cnt, system->sb.cnt, 4 * size_t(P->G.ncells() + 1), hipMemcpyDeviceToDevice,
                            P->stream));
     GCL_HIP(hipMemcpyAsync(P->sb.skey, system->sb.skey, 4 * size_t(n), hipMemcpyDeviceToDevice, P->stream));
     GCL_HIP(hipMemcpyAsync(P->sb.perm, system->sb.perm, 4 * size_t(n), hipMemcpyDeviceToDevice, P->stream));

@@ -45,16 +45,16 @@ __device__ __forceinline__ void store_pair(int2* out, int64_t o, int32_t a, int3
 }
 
 template <typename T, int D>
-__global__ void k_cellmap(XPtrs xp, XPtrs xalt, const int* sel, int64_t n, CellGeom g, int use_off64,
-                          int32_t* __restrict__ key, int32_t* __restrict__ slot, int32_t* __restrict__ cnt,
-                          const int* flag, int aggregate, const int32_t* __restrict__ order) {
-  if (flag && *flag == 0) return;
+__global__ void k_cellmap(XPtrs src, int64_t n, CellGeom g, int use_off64, int32_t* __restrict__ key,
+                          int32_t* __restrict__ slot, int32_t* __restrict__ cnt, const int32_t* __restrict__ order,
+                          uint64_t* __restrict__ scan_tmp, int32_t* __restrict__ maxcell) {
   const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  clear_scan_words(scan_tmp, g.ncells(), t, int64_t(gridDim.x) * blockDim.x);
+  if (t == 0) *maxcell = 0;
   if (t >= n) return;
   // items in the previous binning's order when there is one: neighbouring
   // threads then mostly share a cell, which the wave-aggregated slots need
   const int64_t i = order ? int64_t(order[t]) : t;
-  const XPtrs& src = (sel && *sel) ? xalt : xp;
   int32_t c[3] = {1, 1, 1};
 #pragma unroll
   for (int k = 0; k < D; ++k) c[k] = cell_coord<T>(static_cast<const T*>(src.p[k])[i], g, k, use_off64);
@@ -62,11 +62,19 @@ __global__ void k_cellmap(XPtrs xp, XPtrs xalt, const int* sel, int64_t n, CellG
   const int32_t k = int32_t(lin);
   // cell and arrival slot in visiting order t (contiguous stores)
   key[t] = k;
-  if (!aggregate) {
-    slot[t] = atomicAdd(&cnt[lin], 1);
-    return;
-  }
   slot[t] = wave_aggregated_slot(cnt, k);
+}
+
+// Cell starts from the histogram, which is zero again afterwards.
+__global__ __launch_bounds__(kScanThreads) void k_cell_starts(int32_t* cnt, int32_t* start, int64_t ncells,
+                                                              uint64_t* words, int32_t* maxcell) {
+  scan_tile<true>(cnt, start, ncells, words, maxcell);
+}
+
+// Offsets of the pairs from their counts.
+__global__ __launch_bounds__(kScanThreads) void k_pair_offsets(int32_t* cnt, int64_t* off, int64_t n,
+                                                               uint64_t* words) {
+  scan_tile<false>(cnt, off, n, words, nullptr);
 }
 
 // Item visited t-th (order as in k_cellmap) to its arrival slot: tmp holds
@@ -74,8 +82,7 @@ __global__ void k_cellmap(XPtrs xp, XPtrs xalt, const int* sel, int64_t n, CellG
 // the rank below need not write it).
 __global__ void k_scatter(const int32_t* __restrict__ key, const int32_t* __restrict__ slot,
                           const int32_t* __restrict__ start, int32_t* __restrict__ tmp, int32_t* __restrict__ skey,
-                          const int32_t* __restrict__ order, int64_t n, const int* flag) {
-  if (flag && *flag == 0) return;
+                          const int32_t* __restrict__ order, int64_t n) {
   int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (t >= n) return;
   const int32_t c = key[t];
@@ -90,15 +97,12 @@ __global__ void k_scatter(const int32_t* __restrict__ key, const int32_t* __rest
 // separate gather of the positions.
 template <typename T, int D, bool Pos>
 __global__ void k_rank(const int32_t* __restrict__ start, const int32_t* __restrict__ tmp, int32_t* __restrict__ perm,
-                       const int32_t* __restrict__ skey, int64_t n, const int* flag, XPtrs xp, XPtrs xalt,
-                       const int* sel, XPtrs xsp) {
-  if (flag && *flag == 0) return;
+                       const int32_t* __restrict__ skey, int64_t n, XPtrs src, XPtrs xsp) {
   int64_t s = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (s >= n) return;
   int32_t i = tmp[s];
   T x[3];
   if constexpr (Pos) {
-    const XPtrs& src = (sel && *sel) ? xalt : xp;
 #pragma unroll
     for (int k = 0; k < D; ++k) x[k] = static_cast<const T*>(src.p[k])[i];
   }
@@ -170,8 +174,10 @@ __device__ __forceinline__ uint32_t pair_window(const T* const* x, T xa0, T xa1,
 // them in the same order.
 template <typename T, int D>
 __global__ void k_pair_count(XPtrs xsp, const int32_t* __restrict__ start, const int32_t* __restrict__ skey,
-                             int64_t n, CellGeom g, T dist2max, int32_t* __restrict__ cnt) {
+                             int64_t n, CellGeom g, T dist2max, int32_t* __restrict__ cnt,
+                             uint64_t* __restrict__ scan_tmp) {
   int64_t s = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  clear_scan_words(scan_tmp, n, s, int64_t(gridDim.x) * blockDim.x);
   if (s >= n) return;
   const T* x[3] = {static_cast<const T*>(xsp.p[0]), static_cast<const T*>(xsp.p[1]),
                    static_cast<const T*>(xsp.p[D == 3 ? 2 : 1])};
@@ -216,8 +222,9 @@ __global__ __launch_bounds__(256) void k_pair_count2(XPtrs xsp, const int32_t* _
                                                      const int32_t* __restrict__ skey, int64_t n, CellGeom g,
                                                      T dist2max, int32_t* __restrict__ cnt,
                                                      uint64_t* __restrict__ ent, int32_t* __restrict__ nent,
-                                                     int entcap) {
+                                                     int entcap, uint64_t* __restrict__ scan_tmp) {
 #pragma clang fp contract(off)
+  clear_scan_words(scan_tmp, n, int64_t(blockIdx.x) * kBlock + threadIdx.x, int64_t(gridDim.x) * kBlock);
   using T2 = typename Vec2<T>::type;
   __shared__ T2 lds[kBlock / 64][kCountWave + 4];  // +4: window reads run up to 3 past a row's end
   const int w = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
@@ -441,38 +448,24 @@ __global__ __launch_bounds__(256) void k_pair_emit_wave(XPtrs xsp, const int32_t
   }
 }
 
-template <typename T>
-void bin_sort_t(const CellGeom& g, const void* const* x, int64_t n, bool use_off64, SortBuffers& sb, const int* flag,
-                hipStream_t s, const void* const* x_alt, const int* sel, void* const* xs) {
-  XPtrs xp{{x[0], x[1], g.dim == 3 ? x[2] : x[1]}};
-  XPtrs xa = xp;
-  if (x_alt) xa = XPtrs{{x_alt[0], x_alt[1], g.dim == 3 ? x_alt[2] : x_alt[1]}};
-  int64_t nc = g.ncells();
-  fill_i32(sb.cnt, nc + 1, 0, flag, s);
-  if (g.dim == 2)
-    k_cellmap<T, 2><<<grid_for(n), kBlock, 0, s>>>(xp, xa, sel, n, g, use_off64 ? 1 : 0, sb.key, sb.slot, sb.cnt, flag, 1,
-                                                   sb.sorted ? sb.perm : nullptr);
-  else
-    k_cellmap<T, 3><<<grid_for(n), kBlock, 0, s>>>(xp, xa, sel, n, g, use_off64 ? 1 : 0, sb.key, sb.slot, sb.cnt, flag, 1,
-                                                   sb.sorted ? sb.perm : nullptr);
+template <typename T, int D>
+void bin_sort_t(const CellGeom& g, const void* const* x, int64_t n, bool use_off64, SortBuffers& sb, hipStream_t s,
+                void* const* xs) {
+  const XPtrs xp{{x[0], x[1], x[D - 1]}};
+  const XPtrs xsp = xs ? XPtrs{{xs[0], xs[1], xs[D - 1]}} : XPtrs{{nullptr, nullptr, nullptr}};
+  const int64_t nc = g.ncells();
+  const int32_t* order = sb.sorted ? sb.perm : nullptr;
+  k_cellmap<T, D><<<grid_for(n), kBlock, 0, s>>>(xp, n, g, use_off64 ? 1 : 0, sb.key, sb.slot, sb.cnt, order,
+                                                 sb.scan_tmp, sb.maxcell);
   GCL_HIP(hipGetLastError());
-  fill_i32(sb.maxcell, 1, 0, flag, s);
-  exclusive_scan_i32(sb.cnt, sb.start, nc, sb.scan_tmp, flag, s, sb.maxcell);
-  k_scatter<<<grid_for(n), kBlock, 0, s>>>(sb.key, sb.slot, sb.start, sb.tmp, sb.skey, sb.sorted ? sb.perm : nullptr, n,
-                                           flag);
+  k_cell_starts<<<unsigned(scan_tiles(nc)), kScanThreads, 0, s>>>(sb.cnt, sb.start, nc, sb.scan_tmp, sb.maxcell);
   GCL_HIP(hipGetLastError());
-  const XPtrs xsp = xs ? XPtrs{{xs[0], xs[1], g.dim == 3 ? xs[2] : xs[1]}} : XPtrs{{nullptr, nullptr, nullptr}};
-  if (!xs)
-    k_rank<T, 2, false><<<grid_for(n), kBlock, 0, s>>>(sb.start, sb.tmp, sb.perm, sb.skey, n, flag, xp, xa, sel,
-                                                        xsp);
-  else if (g.dim == 2)
-    k_rank<T, 2, true><<<grid_for(n), kBlock, 0, s>>>(sb.start, sb.tmp, sb.perm, sb.skey, n, flag, xp, xa, sel,
-                                                       xsp);
-  else
-    k_rank<T, 3, true><<<grid_for(n), kBlock, 0, s>>>(sb.start, sb.tmp, sb.perm, sb.skey, n, flag, xp, xa, sel,
-                                                       xsp);
+  k_scatter<<<grid_for(n), kBlock, 0, s>>>(sb.key, sb.slot, sb.start, sb.tmp, sb.skey, order, n);
   GCL_HIP(hipGetLastError());
-  if (!flag) sb.sorted = true;  // perm now holds a permutation of [0, n) (a flagged sort may not have run)
+  if (xs) k_rank<T, D, true><<<grid_for(n), kBlock, 0, s>>>(sb.start, sb.tmp, sb.perm, sb.skey, n, xp, xsp);
+  else k_rank<T, D, false><<<grid_for(n), kBlock, 0, s>>>(sb.start, sb.tmp, sb.perm, sb.skey, n, xp, xsp);
+  GCL_HIP(hipGetLastError());
+  sb.sorted = true;  // perm now holds a permutation of [0, n)
 }
 
 }  // namespace
@@ -487,9 +480,11 @@ void SortBuffers::alloc(int64_t n_, int64_t ncells_) {
   GCL_HIP(hipMalloc(&tmp, sizeof(int32_t) * size_t(n)));
   GCL_HIP(hipMalloc(&perm, sizeof(int32_t) * size_t(n)));
   GCL_HIP(hipMalloc(&skey, sizeof(int32_t) * size_t(n)));
-  GCL_HIP(hipMalloc(&cnt, sizeof(int32_t) * size_t(ncells + 1)));
+  GCL_HIP(hipMalloc(&cnt, sizeof(int32_t) * size_t(ncells)));
+  GCL_HIP(hipMemset(cnt, 0, sizeof(int32_t) * size_t(ncells)));
+  GCL_HIP(hipStreamSynchronize(nullptr));  // the sorts run on other streams
   GCL_HIP(hipMalloc(&start, sizeof(int32_t) * size_t(ncells + 1)));
-  GCL_HIP(hipMalloc(&scan_tmp, sizeof(int64_t) * scan_tmp_elems(ncells)));
+  GCL_HIP(hipMalloc(&scan_tmp, sizeof(uint64_t) * size_t(scan_words(ncells))));
   GCL_HIP(hipMalloc(&maxcell, sizeof(int32_t) * 4));
 }
 
@@ -506,7 +501,7 @@ void PairBuffers::alloc(int64_t n_, int entcap_) {
   n = n_;
   GCL_HIP(hipMalloc(&cnt, sizeof(int32_t) * size_t(n + 1)));
   GCL_HIP(hipMalloc(&off, sizeof(int64_t) * size_t(n + 1)));
-  GCL_HIP(hipMalloc(&scan_tmp, sizeof(int64_t) * scan_tmp_elems(n)));
+  GCL_HIP(hipMalloc(&scan_tmp, sizeof(uint64_t) * size_t(scan_words(n))));
   entcap = entcap_;
   if (entcap > 0) {
     GCL_HIP(hipMalloc(&ent, sizeof(uint64_t) * size_t(entcap) * size_t(n)));
@@ -544,9 +539,14 @@ void PairBuffers::release() {
 }
 
 void bin_sort(const CellGeom& g, int prec, const void* const* x, int64_t n, bool use_off64, SortBuffers& sb,
-              const int* flag, hipStream_t s, const void* const* x_alt, const int* sel, void* const* xs) {
-  if (prec == 32) bin_sort_t<float>(g, x, n, use_off64, sb, flag, s, x_alt, sel, xs);
-  else bin_sort_t<double>(g, x, n, use_off64, sb, flag, s, x_alt, sel, xs);
+              hipStream_t s, void* const* xs) {
+  if (prec == 32) {
+    if (g.dim == 2) bin_sort_t<float, 2>(g, x, n, use_off64, sb, s, xs);
+    else bin_sort_t<float, 3>(g, x, n, use_off64, sb, s, xs);
+  } else {
+    if (g.dim == 2) bin_sort_t<double, 2>(g, x, n, use_off64, sb, s, xs);
+    else bin_sort_t<double, 3>(g, x, n, use_off64, sb, s, xs);
+  }
 }
 
 void gather_positions(int dim, int prec, const void* const* x, void* const* xs, const int32_t* perm, int64_t n,
@@ -570,11 +570,12 @@ void pair_count(const CellGeom& g, int prec, const void* const* xs, const int32_
   auto run = [&](auto d2) {
     using T = decltype(d2);
     if (g.dim == 3)
-      k_pair_count<T, 3><<<grid_for(n), kBlock, 0, s>>>(xsp, start, skey, n, g, d2, pb.cnt);
+      k_pair_count<T, 3><<<grid_for(n), kBlock, 0, s>>>(xsp, start, skey, n, g, d2, pb.cnt, pb.scan_tmp);
     else if (store)
-      k_pair_count2<T><<<grid_for(n), kBlock, 0, s>>>(xsp, start, skey, n, g, d2, pb.cnt, pb.ent, pb.nent, pb.entcap);
+      k_pair_count2<T><<<grid_for(n), kBlock, 0, s>>>(xsp, start, skey, n, g, d2, pb.cnt, pb.ent, pb.nent, pb.entcap,
+                                                      pb.scan_tmp);
     else
-      k_pair_count<T, 2><<<grid_for(n), kBlock, 0, s>>>(xsp, start, skey, n, g, d2, pb.cnt);
+      k_pair_count<T, 2><<<grid_for(n), kBlock, 0, s>>>(xsp, start, skey, n, g, d2, pb.cnt, pb.scan_tmp);
   };
   if (prec == 32) {
     float d = float(dist);
@@ -583,7 +584,8 @@ void pair_count(const CellGeom& g, int prec, const void* const* xs, const int32_
     run(dist * dist);
   }
   GCL_HIP(hipGetLastError());
-  exclusive_scan_i64(pb.cnt, pb.off, n, pb.scan_tmp, nullptr, s);
+  k_pair_offsets<<<unsigned(scan_tiles(n)), kScanThreads, 0, s>>>(pb.cnt, pb.off, n, pb.scan_tmp);
+  GCL_HIP(hipGetLastError());
 }
 
 namespace {

@@ -2,7 +2,7 @@
 // GPUCellList and by the SPH step's rebuild.
 #pragma once
 
-#include "gclsph_internal.hpp"
+#include "blockscan.hpp"
 
 namespace gclsph {
 
@@ -81,12 +81,12 @@ struct SortBuffers {
   int64_t n = 0, ncells = 0;
   int32_t* key = nullptr;    // cell of each input item
   int32_t* slot = nullptr;   // arrival slot inside its cell (atomic, unordered)
-  int32_t* cnt = nullptr;    // ncells + 1 histogram
+  int32_t* cnt = nullptr;    // ncells histogram: zero before a sort and, its scan clears it, after it
   int32_t* start = nullptr;  // ncells + 1 exclusive scan of cnt
   int32_t* tmp = nullptr;    // n: input index per unordered slot
   int32_t* perm = nullptr;   // n: sorted position -> input index
   int32_t* skey = nullptr;   // n: cell of each sorted position
-  int64_t* scan_tmp = nullptr;
+  uint64_t* scan_tmp = nullptr;  // scan_words(ncells)
   int32_t* maxcell = nullptr;  // 1: max particles per cell of the last binning
   bool sorted = false;         // perm holds a previous binning's order
   void alloc(int64_t n_, int64_t ncells_);
@@ -98,7 +98,7 @@ struct PairBuffers {
   int64_t n = 0;
   int32_t* cnt = nullptr;    // n + 1
   int64_t* off = nullptr;    // n + 1
-  int64_t* scan_tmp = nullptr;
+  uint64_t* scan_tmp = nullptr;  // scan_words(n)
   int32_t* pairs = nullptr;  // 2 * capacity
   int64_t capacity = 0;
   // 2D: the neighbour windows the count pass found, read back by the emit
@@ -189,13 +189,10 @@ __device__ __forceinline__ void row_union(RowUnion& u, const int32_t* start, con
 // into cells, and writes the sorted order (perm, skey, start).  The order
 // inside a cell is by input index, so the result is deterministic.
 // `prec` is 64 or 32; `use_off64` selects the Float64-offset cell map.
-// `x_alt`/`sel` (nullable): a second set of position pointers, chosen on the
-// device when *sel != 0 (the SPH state is double-buffered on the device).
 // `xs` (nullable): D arrays that receive the positions in sorted order (what
 // gather_positions would write), moved by the sort's rank kernel.
 void bin_sort(const CellGeom& g, int prec, const void* const* x, int64_t n, bool use_off64, SortBuffers& sb,
-              const int* flag, hipStream_t s, const void* const* x_alt = nullptr, const int* sel = nullptr,
-              void* const* xs = nullptr);
+              hipStream_t s, void* const* xs = nullptr);
 
 // Gathers x (input order) into xs (sorted order) using perm.
 void gather_positions(int dim, int prec, const void* const* x, void* const* xs, const int32_t* perm, int64_t n,

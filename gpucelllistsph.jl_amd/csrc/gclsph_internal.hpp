@@ -51,11 +51,10 @@ inline unsigned grid_for(int64_t n, int block = kBlock) {
 // end of a `stepsolve` call.
 struct StepCtl {
   int parity;         // which of the ping-pong state buffers is current
-  int rebuild;        // rebuild the cell order at the start of the next step
-  int rebuilt;        // the current step rebuilt (membership uses the current x)
+  int rebuild;        // rebuild the cell order at the start of the next step; within a step
+                      // that does, parity and pparity are those before it until the commit
   int synced;         // half-step state equals the main state (no correction ran)
   int pparity;       // which ptype / id buffer is current (flipped by reorders only)
-  int xrb_cur;       // rebuild positions are the current positions (no step since)
   int iter;          // 1-based iteration inside the running stepsolve call
   int nsteps;        // iterations of the running call
   long long updaten;  // rebuilds in this call
@@ -88,18 +87,5 @@ __device__ inline void atomic_max_nonneg(unsigned long long* slot, double v) {
 }
 
 __device__ inline double bits_to_double(unsigned long long b) { return __longlong_as_double((long long)b); }
-
-// Exclusive scan of n int32 counts into int32 (or int64) offsets; out[n] = total.
-// Implemented in scan.hip.  `flag` (nullable) makes every launch a no-op while
-// *flag == 0, so the scan can sit in a step sequence that only sometimes
-// rebuilds.  Returns nothing; `tmp` must hold scan_tmp_elems(n) elements.
-size_t scan_tmp_elems(int64_t n);
-void exclusive_scan_i32(const int32_t* in, int32_t* out, int64_t n, int64_t* tmp, const int* flag,
-                        hipStream_t s, int32_t* max_out = nullptr);
-void exclusive_scan_i64(const int32_t* in, int64_t* out, int64_t n, int64_t* tmp, const int* flag,
-                        hipStream_t s);
-
-// Fill helpers usable under graph capture (no hipMemsetAsync).
-void fill_i32(int32_t* p, int64_t n, int32_t v, const int* flag, hipStream_t s);
 
 }  // namespace gclsph

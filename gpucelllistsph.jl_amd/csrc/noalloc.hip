@@ -27,10 +27,6 @@ constexpr int64_t kNaMaxPoints = GCLSPH_NOALLOC_MAX_POINTS;
 constexpr int64_t kNaMaxCells = GCLSPH_NOALLOC_MAX_CELLS;
 
 constexpr size_t align256(size_t b) { return (b + 255) / 256 * 256; }
-constexpr size_t scan_elems(int64_t n) {  // scan_tmp_elems() of scan.hip, for the fixed maxima
-  return size_t((n + kTile - 1) / kTile + 2 + ((n + kTile - 1) / kTile + 1) / 2 + 1);
-}
-
 // Layout of the scratch array (each piece 256-byte aligned): the counting
 // sort (key, slot, tmp, perm, skey; cell histogram and starts; scan tiles;
 // max-per-cell), the sorted coordinates (3 components with the padding the
@@ -53,12 +49,12 @@ constexpr Layout make_layout() {
   L.skey = take(4 * size_t(kNaMaxPoints));
   L.cnt = take(4 * size_t(kNaMaxCells + 1));
   L.start = take(4 * size_t(kNaMaxCells + 1));
-  L.sort_scan = take(8 * scan_elems(kNaMaxCells));
+  L.sort_scan = take(8 * size_t(scan_words(kNaMaxCells)));
   L.maxcell = take(16);
   for (int k = 0; k < 3; ++k) L.xs[k] = take(8 * size_t(kNaMaxPoints + kPosPad));
   L.pcnt = take(4 * size_t(kNaMaxPoints + 1));
   L.poff = take(8 * size_t(kNaMaxPoints + 1));
-  L.pair_scan = take(8 * scan_elems(kNaMaxPoints));
+  L.pair_scan = take(8 * size_t(scan_words(kNaMaxPoints)));
   L.total = o;
   return L;
 }
@@ -71,6 +67,9 @@ __device__ __align__(256) unsigned char scratch[kLayout.total];
 
 std::mutex g_mutex;
 std::array<unsigned char*, 64> g_scratch_ptr{};  // device address of `scratch`, per device ordinal
+// Whether a call on the device ended before its sort had cleared the cell
+// histogram again (it is zero when the library is loaded).
+std::array<bool, 64> g_dirty{};
 
 unsigned char* scratch_on_current_device(int dev) {
   GCL_CHECK(dev >= 0 && dev < int(g_scratch_ptr.size()), kErrUnsupported, "device ordinal beyond 63");
@@ -140,14 +139,14 @@ extern "C" int gcl_neighborlist_noalloc(int dim, int64_t n, const double* const*
     sb.skey = reinterpret_cast<int32_t*>(base + kLayout.skey);
     sb.cnt = reinterpret_cast<int32_t*>(base + kLayout.cnt);
     sb.start = reinterpret_cast<int32_t*>(base + kLayout.start);
-    sb.scan_tmp = reinterpret_cast<int64_t*>(base + kLayout.sort_scan);
+    sb.scan_tmp = reinterpret_cast<uint64_t*>(base + kLayout.sort_scan);
     sb.maxcell = reinterpret_cast<int32_t*>(base + kLayout.maxcell);
     sb.sorted = false;  // visit the points in input order (the scratch holds another call's order)
     PairBuffers pb;
     pb.n = n;
     pb.cnt = reinterpret_cast<int32_t*>(base + kLayout.pcnt);
     pb.off = reinterpret_cast<int64_t*>(base + kLayout.poff);
-    pb.scan_tmp = reinterpret_cast<int64_t*>(base + kLayout.pair_scan);
+    pb.scan_tmp = reinterpret_cast<uint64_t*>(base + kLayout.pair_scan);
     pb.pairs = pairs_dev;
     pb.capacity = capacity;
     void* xs[3] = {base + kLayout.xs[0], base + kLayout.xs[1], base + kLayout.xs[2]};
@@ -155,11 +154,14 @@ extern "C" int gcl_neighborlist_noalloc(int dim, int64_t n, const double* const*
 
     // cellmap! + fillcells_naive! with the Float64 MIN, as the constructor
     // bins (src/celllist.jl:55-66), then the pair search (:72-75)
-    bin_sort(g, GCLSPH_F64, x, n, true, sb, nullptr, s, nullptr, nullptr, xs);
+    if (g_dirty[size_t(dev)]) GCL_HIP(hipMemsetAsync(sb.cnt, 0, 4 * size_t(kNaMaxCells), s));
+    g_dirty[size_t(dev)] = true;
+    bin_sort(g, GCLSPH_F64, x, n, true, sb, s, xs);
     pair_count(g, GCLSPH_F64, xs, sb.start, sb.skey, n, dist, pb, s);
     int64_t total = 0;
     GCL_HIP(hipMemcpyAsync(&total, pb.off + n, sizeof(int64_t), hipMemcpyDeviceToHost, s));
     GCL_HIP(hipStreamSynchronize(s));
+    g_dirty[size_t(dev)] = false;
     pair_emit(g, GCLSPH_F64, xs, sb.start, sb.skey, sb.perm, n, dist, total, pb, s);
     GCL_HIP(hipStreamSynchronize(s));
     *pairsn = total;

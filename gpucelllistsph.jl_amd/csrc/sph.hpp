@@ -283,7 +283,7 @@ struct SceneDev {
   StepFlags F;
   // counting-sort buffers of the rebuild
   int32_t *key, *slot, *cnt, *start, *tmp, *perm, *skey, *maxcell;
-  int64_t* scan_tmp;
+  uint64_t* scan_tmp;
   int64_t ncells;
 };
 
@@ -293,7 +293,7 @@ struct SceneDev {
 // pmap512 does the same for the 512-thread blocks of the pass kernels (their
 // 128-thread blocks halve the pmap entries), and qmap for the pair kernels' blocks
 // of 64 particles with a quad of lanes each.
-// Cell kernels run one block per 1024-cell tile; cmap maps a block to (problem,
+// The cell scan runs one block per tile of kTile cells; cmap maps a block to (problem,
 // tile).  Per-problem kernels run one block per problem.
 struct LaunchSet {
   void* scenes = nullptr;  // device SceneDev<R>[count]
@@ -320,6 +320,9 @@ struct LaunchSet {
 // binning, scan, scatter, rank, reorder of the state, commit, membership store.
 template <int D, typename R>
 void launch_rebuild(const LaunchSet& L, hipStream_t s);
+// Commits a rebuild outside a step (in a step k_finalize does).
+template <int D, typename R>
+void launch_commit_rebuild(const LaunchSet& L, hipStream_t s);
 // Pair passes in one of kPassVariants variants that differ only in code
 // generation and launch shape (same results): variant = cg + 4·bs + 12·oc,
 // with cg in [0, 4) the prefetch / occupancy-target choice, bs in [0, 3) the

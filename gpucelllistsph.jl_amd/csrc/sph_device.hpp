@@ -341,6 +341,11 @@ __device__ __forceinline__ float dotf(const float* a, const float* b) {
   return s;
 }
 
+// Buffers of the current state within a step, after the rebuild stage: a
+// rebuild writes the other ones, and the flag is cleared when the step ends.
+__device__ __forceinline__ int cur_parity(const StepCtl* c) { return c->parity ^ c->rebuild; }
+__device__ __forceinline__ int cur_pparity(const StepCtl* c) { return c->pparity ^ c->rebuild; }
+
 // Positions of the pair-list membership test: the current positions when this
 // step rebuilt (or when no later step can skip a rebuild), else the stored
 // rebuild positions.

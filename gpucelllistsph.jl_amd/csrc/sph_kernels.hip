@@ -192,12 +192,12 @@ __global__ __launch_bounds__(256) void k_nmask(SS ss) {
   static_assert(D == 3, "the 2D membership store is part of k_reorder_nmask2");
   GCLSPH_SCENE(ss);
   const StepCtl* ctl = B.ctl;
-  if (!ctl->rebuilt) return;
+  if (!ctl->rebuild) return;
   const int64_t a0 = int64_t(m.y) * kBlock;
   if (a0 >= B.n) return;  // whole block
   const bool active = a < B.n;
   const double dist2 = C.dist2;
-  const int p = ctl->parity;  // the rebuild positions are the current ones
+  const int p = cur_parity(ctl);  // the rebuild positions are the current ones
   const double* XM[3] = {B.X[p][0], B.X[p][1], B.X[p][D == 3 ? 2 : 1]};
   const int cap = B.necap;
   uint64_t* out = B.NE + a;
@@ -315,26 +315,23 @@ __global__ __launch_bounds__(256) void k_nmask(SS ss) {
 }
 
 // ------------------------------------------------------------------ kernels
-// Runs after the (conditional) rebuild kernels: commits the reorder.
+// Commits the rebuild of a problem (one thread per problem): the reordered
+// buffers become the current ones.
+template <typename R>
+__device__ __forceinline__ void commit_rebuild(const SceneDev<R>& sd, StepCtl* ctl) {
+  if (!ctl->rebuild) return;
+  ctl->parity ^= 1;
+  ctl->pparity ^= 1;
+  ctl->updaten += 1;
+  const long long mp = *sd.maxcell;
+  if (mp > ctl->mppcell) ctl->mppcell = (long long)ceil(double(mp) * 1.05 + 1);  // src/celllist.jl:105-106
+  ctl->rebuild = 0;
+}
+
 template <typename R, typename SS>
-__global__ void k_post_rebuild(SS ss) {
-  if (threadIdx.x != 0) return;
+__global__ void k_commit_rebuild(SS ss) {
   const SceneDev<R>& sd = scene_at<R>(ss, blockIdx.x);
-  StepCtl* ctl = sd.B.ctl;
-  const int32_t* maxcell = sd.maxcell;
-  const int write_xrb = sd.F.write_xrb;
-  if (ctl->rebuild) {
-    ctl->parity ^= 1;
-    ctl->pparity ^= 1;
-    ctl->rebuilt = 1;
-    ctl->updaten += 1;
-    long long mp = *maxcell;
-    if (mp > ctl->mppcell) ctl->mppcell = (long long)ceil(double(mp) * 1.05 + 1);  // src/celllist.jl:105-106
-    ctl->rebuild = 0;
-    ctl->xrb_cur = write_xrb ? 0 : 1;
-  } else {
-    ctl->rebuilt = 0;
-  }
+  if (threadIdx.x == 0) commit_rebuild(sd, sd.B.ctl);
 }
 
 // New sorted position s takes the state of old position perm[s] (its
@@ -498,7 +495,7 @@ __global__ __launch_bounds__(256) void k_dpc_sum(SS ss) {
   GCLSPH_SCENE_PAIR(ss, kBlock, Quad);
   if (!F.dpc_on) return;
   const StepCtl* ctl = B.ctl;
-  const int p = ctl->parity, q = p ^ 1, pp = ctl->pparity, rebuilt = ctl->rebuilt;
+  const int p = cur_parity(ctl), q = p ^ 1, pp = cur_pparity(ctl), rebuilt = ctl->rebuild;
   const double dt = ctl->dt;
   if (a >= B.n) return;
   const double* X[3] = {B.X[q][0], B.X[q][1], B.X[q][D == 3 ? 2 : 1]};
@@ -610,7 +607,7 @@ __global__ void k_dpc_apply(SS ss) {
   GCLSPH_SCENE(ss);
   if (!F.dpc_on) return;
   const StepCtl* ctl = B.ctl;
-  const int q = ctl->parity ^ 1, pp = ctl->pparity;
+  const int q = cur_parity(ctl) ^ 1, pp = cur_pparity(ctl);
   const double dt = ctl->dt;
   if (a >= B.n || B.PT[pp][a] <= 1) return;
   double fr[3];
@@ -640,7 +637,7 @@ __global__ void k_xsph_rec(SS ss) {
   GCLSPH_SCENE(ss);
   if (!F.xsph_on) return;
   const StepCtl* ctl = B.ctl;
-  const int p = ctl->parity, q = p ^ 1, pp = ctl->pparity;
+  const int p = cur_parity(ctl), q = p ^ 1, pp = cur_pparity(ctl);
   if (a >= B.n) return;
   typename Records<D, R>::N rec{};
   double fr[3];
@@ -663,7 +660,7 @@ __global__ __launch_bounds__(256) void k_xsph(SS ss) {
   GCLSPH_SCENE_PAIR(ss, kBlock, Quad);
   if (!F.xsph_on) return;
   const StepCtl* ctl = B.ctl;
-  const int p = ctl->parity, q = p ^ 1, pp = ctl->pparity, rebuilt = ctl->rebuilt;
+  const int p = cur_parity(ctl), q = p ^ 1, pp = cur_pparity(ctl), rebuilt = ctl->rebuild;
   const double dt = ctl->dt;
   if (a >= B.n) return;
   const int32_t* PT = B.PT[pp];
@@ -741,7 +738,7 @@ __global__ __launch_bounds__(256) void k_cspm_sum(SS ss) {
   GCLSPH_SCENE_PAIR(ss, kBlock, Quad);
   if (!F.cspm_fire) return;
   const StepCtl* ctl = B.ctl;
-  const int p = ctl->parity, q = p ^ 1, pp = ctl->pparity, rebuilt = ctl->rebuilt;
+  const int p = cur_parity(ctl), q = p ^ 1, pp = cur_pparity(ctl), rebuilt = ctl->rebuild;
   if (a >= B.n) return;
   const int32_t* PT = B.PT[pp];
   const int32_t pta = PT[a];
@@ -807,7 +804,7 @@ __global__ void k_cspm_apply(SS ss) {
   GCLSPH_SCENE(ss);
   if (!F.cspm_fire) return;
   const StepCtl* ctl = B.ctl;
-  const int q = ctl->parity ^ 1, pp = ctl->pparity;
+  const int q = cur_parity(ctl) ^ 1, pp = cur_pparity(ctl);
   if (a >= B.n) return;
   double nr = B.TMP[a];
   if (nr != nr) return;
@@ -854,7 +851,7 @@ __global__ void k_dt_visc(SS ss) {
   GCLSPH_SCENE(ss);
   if (!(F.ts && !F.visc_in_pass2)) return;  // the whole block belongs to one problem
   StepCtl* ctl = B.ctl;
-  const int q = ctl->parity ^ 1;
+  const int q = cur_parity(ctl) ^ 1;
   const bool active = a < B.n;
   double v = 0.0;
   if (active) {
@@ -892,6 +889,7 @@ __global__ void k_finalize(SS ss) {
     tot[k] = wave_max(v);
   }
   if (l != 0) return;
+  commit_rebuild(sd, ctl);
   double cdx = tot[0];
   if (cdx > 0.9 * C.nui) ctl->rebuild = 1;
   ctl->maxcdx_out = jl_max(ctl->maxcdx_out, cdx);
@@ -910,7 +908,6 @@ __global__ void k_finalize(SS ss) {
   ctl->red_visc = 0;
   ctl->parity ^= 1;
   ctl->synced = corr_on ? 0 : 1;
-  ctl->xrb_cur = 0;
   ctl->iter += 1;
 }
 
@@ -958,27 +955,15 @@ __global__ __launch_bounds__(256) void k_diag(SS ss, int xm_mode, int use_masks)
 // which makes the order deterministic.  Every kernel returns at once for a
 // problem whose control block does not ask for a rebuild.
 
-// cnt[0..ncells] = 0 and maxcell = 0 (cell tiles).
-template <typename R, typename SS>
-__global__ void kb_clear_cells(SS ss) {
-  int2 m;
-  const SceneDev<R>& sd = tile_scene<R>(ss, m);
-  if (sd.B.ctl->rebuild == 0) return;
-  const int64_t base = int64_t(m.y) * kTile;
-#pragma unroll
-  for (int k = 0; k < kScanItems; ++k) {
-    const int64_t i = base + int64_t(k) * kScanThreads + threadIdx.x;
-    if (i <= sd.ncells) sd.cnt[i] = 0;
-  }
-  if (m.y == 0 && threadIdx.x == 0) *sd.maxcell = 0;
-}
-
 // Cell of every particle (current positions) and its arrival slot.
 template <int D, typename R, typename SS>
 __global__ void kb_cellmap(SS ss) {
   GCLSPH_SCENE(ss);
   const StepCtl* ctl = B.ctl;
-  if (ctl->rebuild == 0 || a >= B.n) return;
+  if (ctl->rebuild == 0) return;
+  clear_scan_words(sd.scan_tmp, sd.ncells, a, (B.n + kBlock - 1) / kBlock * kBlock);
+  if (a == 0) *sd.maxcell = 0;
+  if (a >= B.n) return;
   const int p = ctl->parity;
   int32_t c[3] = {1, 1, 1};
 #pragma unroll
@@ -989,111 +974,14 @@ __global__ void kb_cellmap(SS ss) {
   sd.slot[a] = wave_aggregated_slot(sd.cnt, key);
 }
 
-// Tile sums (and tile maxima, stored after the sums) of the cell counts.
+// Cell starts from the histogram, which is zero again afterwards;
+// start[ncells] = n.
 template <typename R, typename SS>
-__global__ void kb_tile_sums(SS ss) {
+__global__ __launch_bounds__(kScanThreads) void kb_cell_starts(SS ss) {
   int2 m;
   const SceneDev<R>& sd = tile_scene<R>(ss, m);
   if (sd.B.ctl->rebuild == 0) return;
-  const int64_t n = sd.ncells, nt = (n + kTile - 1) / kTile;
-  if (m.y >= nt) return;
-  const int64_t base = int64_t(m.y) * kTile;
-  int64_t s = 0;
-  int32_t mx = 0;
-#pragma unroll
-  for (int k = 0; k < kScanItems; ++k) {
-    const int64_t i = base + int64_t(k) * kScanThreads + threadIdx.x;
-    if (i < n) {
-      const int32_t v = sd.cnt[i];
-      s += v;
-      mx = v > mx ? v : mx;
-    }
-  }
-  int64_t tot;
-  block_exclusive_scan<int64_t>(s, &tot);
-  if (threadIdx.x == 0) sd.scan_tmp[m.y] = tot;
-  __shared__ int32_t wmx[kScanThreads / 64];
-  for (int o = 32; o > 0; o >>= 1) {
-    const int32_t t = __shfl_xor(mx, o, 64);
-    mx = t > mx ? t : mx;
-  }
-  if ((threadIdx.x & 63) == 0) wmx[threadIdx.x >> 6] = mx;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int32_t v = wmx[0];
-    for (int w = 1; w < kScanThreads / 64; ++w) v = wmx[w] > v ? wmx[w] : v;
-    reinterpret_cast<int32_t*>(sd.scan_tmp + nt + 2)[m.y] = v;
-  }
-}
-
-// One block per problem: exclusive scan of the tile sums in place (total at
-// [nt]) and the maximum cell count.
-template <typename R, typename SS>
-__global__ void kb_scan_tile_sums(SS ss) {
-  const SceneDev<R>& sd = scene_at<R>(ss, blockIdx.x);
-  if (sd.B.ctl->rebuild == 0) return;
-  int64_t* tsum = sd.scan_tmp;
-  const int64_t nt = (sd.ncells + kTile - 1) / kTile;
-  const int32_t* tm = reinterpret_cast<const int32_t*>(tsum + nt + 2);
-  int32_t mx = 0;
-  for (int64_t i = threadIdx.x; i < nt; i += kScanThreads) mx = tm[i] > mx ? tm[i] : mx;
-  for (int o = 32; o > 0; o >>= 1) {
-    const int32_t t = __shfl_xor(mx, o, 64);
-    mx = t > mx ? t : mx;
-  }
-  if ((threadIdx.x & 63) == 0) atomicMax(sd.maxcell, mx);
-  const int64_t per = (nt + kScanThreads - 1) / kScanThreads;
-  const int64_t b = int64_t(threadIdx.x) * per, e = b + per < nt ? b + per : nt;
-  int64_t s = 0;
-  for (int64_t i = b; i < e; ++i) s += tsum[i];
-  int64_t tot;
-  int64_t pre = block_exclusive_scan<int64_t>(s, &tot);
-  for (int64_t i = b; i < e; ++i) {
-    const int64_t v = tsum[i];
-    tsum[i] = pre;
-    pre += v;
-  }
-  if (threadIdx.x == 0) tsum[nt] = tot;
-}
-
-// Cell starts: tile scans plus the tile prefixes; start[ncells] = n.
-template <typename R, typename SS>
-__global__ void kb_tile_scan(SS ss) {
-  int2 m;
-  const SceneDev<R>& sd = tile_scene<R>(ss, m);
-  if (sd.B.ctl->rebuild == 0) return;
-  const int64_t n = sd.ncells, nt = (n + kTile - 1) / kTile;
-  if (m.y >= nt) return;
-  const int64_t base = int64_t(m.y) * kTile + int64_t(threadIdx.x) * kScanItems;
-  static_assert(kScanItems == 4, "one 16-byte word of counts per thread");
-  const bool whole = base + kScanItems <= n;  // the last tile's tail goes element by element
-  int32_t v[kScanItems];
-  if (whole) {
-    const int4 w = *reinterpret_cast<const int4*>(sd.cnt + base);
-    v[0] = w.x, v[1] = w.y, v[2] = w.z, v[3] = w.w;
-  } else {
-#pragma unroll
-    for (int k = 0; k < kScanItems; ++k) v[k] = base + k < n ? sd.cnt[base + k] : 0;
-  }
-  int64_t s = 0;
-#pragma unroll
-  for (int k = 0; k < kScanItems; ++k) s += v[k];
-  int64_t tot;
-  int64_t pre = block_exclusive_scan<int64_t>(s, &tot) + sd.scan_tmp[m.y];
-  int32_t o[kScanItems];
-#pragma unroll
-  for (int k = 0; k < kScanItems; ++k) {
-    o[k] = int32_t(pre);
-    pre += v[k];
-  }
-  if (whole) {
-    *reinterpret_cast<int4*>(sd.start + base) = make_int4(o[0], o[1], o[2], o[3]);
-  } else {
-#pragma unroll
-    for (int k = 0; k < kScanItems; ++k)
-      if (base + k < n) sd.start[base + k] = o[k];
-  }
-  if (m.y == 0 && threadIdx.x == 0) sd.start[n] = int32_t(sd.scan_tmp[nt]);
+  scan_tile<true>(sd.cnt, sd.start, sd.ncells, sd.scan_tmp, sd.maxcell);
 }
 
 // Sort key of an x coordinate: its bit pattern made unsigned-monotone (order
@@ -1189,22 +1077,21 @@ template <int D, typename R>
 void launch_rebuild(const LaunchSet& L, hipStream_t s) {
   with_scenes<R>(L, [&](auto ss) {
     using SS = decltype(ss);
-    kb_clear_cells<R, SS><<<L.ctiles, kScanThreads, 0, s>>>(ss);
     kb_cellmap<D, R, SS><<<L.pblocks, kBlock, 0, s>>>(ss);
-    kb_tile_sums<R, SS><<<L.ctiles, kScanThreads, 0, s>>>(ss);
-    kb_scan_tile_sums<R, SS><<<L.count, kScanThreads, 0, s>>>(ss);
-    kb_tile_scan<R, SS><<<L.ctiles, kScanThreads, 0, s>>>(ss);
+    kb_cell_starts<R, SS><<<L.ctiles, kScanThreads, 0, s>>>(ss);
     kb_scatter<D, R, SS><<<L.pblocks, kBlock, 0, s>>>(ss);
     kb_rank<D, R, SS><<<L.pblocks, kBlock, 0, s>>>(ss);
     if constexpr (D == 2) {
       k_reorder_nmask2<R, SS><<<L.pblocks, kBlock, 0, s>>>(ss);
-      k_post_rebuild<R, SS><<<L.count, 64, 0, s>>>(ss);
     } else {
       k_reorder<D, R, SS><<<L.pblocks, kBlock, 0, s>>>(ss);
-      k_post_rebuild<R, SS><<<L.count, 64, 0, s>>>(ss);
       k_nmask<D, R, SS><<<L.pblocks, kBlock, 0, s>>>(ss);
     }
   });
+}
+template <int D, typename R>
+void launch_commit_rebuild(const LaunchSet& L, hipStream_t s) {
+  with_scenes<R>(L, [&](auto ss) { k_commit_rebuild<R, decltype(ss)><<<L.count, 64, 0, s>>>(ss); });
 }
 template <int D, typename R>
 void launch_init_pn(const LaunchSet& L, hipStream_t s) {
@@ -1251,6 +1138,7 @@ void launch_diag(const LaunchSet& L, int xm_mode, int use_masks, hipStream_t s) 
 
 #define GCLSPH_INSTANTIATE(D, R)                                                         \
   template void launch_rebuild<D, R>(const LaunchSet&, hipStream_t);                     \
+  template void launch_commit_rebuild<D, R>(const LaunchSet&, hipStream_t);              \
   template void launch_init_pn<D, R>(const LaunchSet&, hipStream_t);                     \
   template void launch_dpc<D, R>(const LaunchSet&, hipStream_t);                         \
   template void launch_xsph<D, R>(const LaunchSet&, hipStream_t);                        \

@@ -45,7 +45,7 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W))) void k_
 #pragma clang fp contract(off)
   GCLSPH_SCENE_PAIR(ss, BS, Quad);
   const StepCtl* ctl = B.ctl;
-  const int p = ctl->parity, pp = ctl->pparity, rebuilt = ctl->rebuilt;
+  const int p = cur_parity(ctl), pp = cur_pparity(ctl), rebuilt = ctl->rebuild;
   const double dt = ctl->dt;
   if (a >= B.n) return;
   const double* X[3] = {B.X[p][0], B.X[p][1], B.X[p][D == 3 ? 2 : 1]};
@@ -200,7 +200,7 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W))) void k_
 #pragma clang fp contract(off)
   GCLSPH_SCENE_PAIR(ss, BS, Quad);
   StepCtl* ctl = B.ctl;
-  const int p = ctl->parity, q = p ^ 1, pp = ctl->pparity, rebuilt = ctl->rebuilt;
+  const int p = cur_parity(ctl), q = p ^ 1, pp = cur_pparity(ctl), rebuilt = ctl->rebuild;
   const double dt = ctl->dt;
   const bool active = a < B.n;
   double red_cdx = 0.0, red_acc = 0.0, red_visc = 0.0;

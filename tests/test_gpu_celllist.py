@@ -51,6 +51,26 @@ def test_reference_fixture(G, O, S):
     assert_same_celllist(g, o)
 
 
+@pytest.mark.parametrize("n", [1, 15, 4095, 4096, 4097, 20001])
+@pytest.mark.parametrize("cells", [(1, 1), (64, 64), (4097, 1), (600, 480)])
+def test_scan_tiles(G, O, S, n, cells):
+    """Cell starts and pair offsets are scans in tiles of 4096 items that look
+    back over up to 64 tiles at a time: items and cells at, around and beyond
+    one tile, a row of cells that ends a tile by one, and 288,000 cells (71
+    tiles), most of them empty; a second binning finds the histogram cleared."""
+    x, y = S.uniform01(11, n, 0) * cells[0], S.uniform01(11, n, 1) * cells[1]
+    d = 1.0 if cells != (1, 1) else 0.05 if n > 100 else 1.0
+    kw = dict(MIN=(1e-9, 1e-9), MAX=tuple(float(c) for c in cells))
+    if cells == (1, 1) and n > 5000:
+        kw = dict(MIN=(1e-9, 1e-9), MAX=(0.5, 0.5))  # most points outside: clamped into the edge cells
+    g = G.GPUCellList((x, y), (d, d), d if n < 5000 else d / 4, **kw)
+    o = O.CellList((x, y), (d, d), d if n < 5000 else d / 4, **kw)
+    assert_same_celllist(g, o)
+    G.update_(g)
+    o.update()
+    assert_same_celllist(g, o)
+
+
 def test_config1_update_and_partialupdate(G, O, S):
     """200,000 uniform points, cellsize = dist = 0.016, jittered by N(0, 0.001^2) per step."""
     pts = S.config1_points()
