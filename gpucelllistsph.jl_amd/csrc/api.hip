@@ -16,6 +16,7 @@
 #include <vector>
 
 #include "../../include/gclsph.h"
+#include "readback.hpp"
 #include "sph.hpp"
 
 using namespace gclsph;
@@ -52,6 +53,27 @@ template <typename T>
 __global__ void k_gather(const T* __restrict__ src, T* __restrict__ dst, const int32_t* __restrict__ perm, int64_t n) {
   int64_t s = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (s < n) dst[s] = src[perm[s]];
+}
+// Results in caller order: the sorted slot of each particle, then values
+// [first, first + count) of up to three components of n particles one after the
+// other, widened, written in order (to page-locked host memory).
+__global__ void k_invert(const int32_t* __restrict__ id, int32_t* __restrict__ inv, int64_t n) {
+  const int64_t s = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (s < n) inv[id[s]] = int32_t(s);
+}
+template <typename T>
+struct Fields {
+  const T* c[3];
+};
+template <typename T>
+__global__ void k_export(Fields<T> src, const int32_t* __restrict__ inv, double* __restrict__ out, int64_t first,
+                         int64_t count, int64_t n, double add) {
+  const int64_t j = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (j >= count) return;
+  const int64_t e = first + j;
+  const int c = int(e >= n) + int(e >= 2 * n);
+  const T* v = c == 0 ? src.c[0] : (c == 1 ? src.c[1] : src.c[2]);
+  out[j] = double(v[inv[e - c * n]]) + add;
 }
 template <typename T>
 __global__ void k_scatter_by(const T* __restrict__ src, T* __restrict__ dst, const int32_t* __restrict__ id,
@@ -129,6 +151,7 @@ struct sph_s;
 
 // --------------------------------------------------------------------- gcl_s
 struct gcl_s {
+  HostSlots::Ref slots;
   int dim = 2, prec = 64;
   int64_t n = 0;
   double dist = 0;
@@ -217,6 +240,7 @@ struct gcl_s {
 
 // --------------------------------------------------------------------- sph_s
 struct sph_s {
+  HostSlots::Ref slots;
   gcl_s* sys = nullptr;
   int dim = 2, prec = GCLSPH_F64;
   int64_t n = 0;
@@ -527,6 +551,32 @@ struct sph_s {
 
   template <typename R>
   SphBufs<R>& bufs();
+
+  // Current sorted slot of every particle, in scratch memory of the problem
+  // (TMP, which the kernels use within a step only).
+  const int32_t* slots_by_id() {
+    int32_t* inv = reinterpret_cast<int32_t*>(split() ? Bf.TMP : Bd.TMP);
+    k_invert<<<grid_for(n), kBlock, 0, stream>>>(idcur(), inv, n);
+    GCL_HIP(hipGetLastError());
+    return inv;
+  }
+  // comps components of a sorted field to out (comps blocks of n) in caller order.
+  template <typename T>
+  void export_fields(const T* const* src, int comps, double add, double* out) {
+    const int32_t* inv = slots_by_id();
+    const Fields<T> f{{src[0], src[comps > 1 ? 1 : 0], src[comps > 2 ? 2 : 0]}};
+    HostSlots::copy_out(out, sizeof(double) * size_t(n) * size_t(comps), stream,
+                        [&](void* slot, size_t off, size_t len) {
+                          const int64_t first = int64_t(off / sizeof(double)), count = int64_t(len / sizeof(double));
+                          k_export<T><<<grid_for(count), kBlock, 0, stream>>>(f, inv, static_cast<double*>(slot), first,
+                                                                             count, n, add);
+                          GCL_HIP(hipGetLastError());
+                        });
+  }
+  template <typename T>
+  void export_field(const T* src, double add, double* out) {
+    export_fields<T>(&src, 1, add, out);
+  }
 
   // Per-call switches of this problem (the per-step ones follow on the device).
   StepFlags call_flags(bool ts) const {
@@ -1044,17 +1094,11 @@ struct sph_batch_s {
 
 namespace {
 
-// Host copy of a sorted device array, returned in caller order.
-template <typename T>
-std::vector<double> unsort(const T* dev, const int32_t* id_dev, int64_t n, hipStream_t s, double add = 0.0) {
-  std::vector<T> v(static_cast<size_t>(n));
-  std::vector<int32_t> id(static_cast<size_t>(n));
-  GCL_HIP(hipMemcpyAsync(v.data(), dev, sizeof(T) * size_t(n), hipMemcpyDeviceToHost, s));
-  GCL_HIP(hipMemcpyAsync(id.data(), id_dev, 4 * size_t(n), hipMemcpyDeviceToHost, s));
-  GCL_HIP(hipStreamSynchronize(s));
-  std::vector<double> out(static_cast<size_t>(n));
-  for (int64_t i = 0; i < n; ++i) out[size_t(id[size_t(i)])] = double(v[size_t(i)]) + add;
-  return out;
+// bytes of device memory to the caller's.
+void copy_out(void* out, const void* src, size_t bytes, hipStream_t st) {
+  HostSlots::copy_out(out, bytes, st, [&](void* slot, size_t off, size_t len) {
+    GCL_HIP(hipMemcpyAsync(slot, static_cast<const char*>(src) + off, len, hipMemcpyDeviceToHost, st));
+  });
 }
 
 // Lazily (re)builds the pair list of a cell list owned by an SPH problem:
@@ -1062,7 +1106,6 @@ std::vector<double> unsort(const T* dev, const int32_t* id_dev, int64_t n, hipSt
 void ensure_pairs(gcl_s* g) {
   if (!g->attached || g->pairs_valid) return;
   sph_s* P = g->attached;
-  P->read_ctl();
   const void* xm[3] = {P->membership(0), P->membership(1), P->membership(g->dim == 3 ? 2 : 1)};
   int64_t total = 0;
   pair_count(P->G, 64, xm, P->sb.start, P->sb.skey, g->n, g->dist, g->pb, P->stream);
@@ -1214,7 +1257,6 @@ int gcl_partialupdate(gcl_t h, int fillzero) {
     GCL_CHECK(h != nullptr, kErrArgument, "NULL handle");
     if (h->attached) {
       sph_s* P = h->attached;
-      P->read_ctl();
       const void* xc[3] = {P->xcur(0), P->xcur(1), P->xcur(h->dim == 3 ? 2 : 1)};
       pair_count(P->G, 64, xc, P->sb.start, P->sb.skey, h->n, h->dist, h->pb, P->stream);
       int64_t total = 0;
@@ -1236,7 +1278,6 @@ int gcl_set_points(gcl_t h, const double* const* pts) {
     GCL_CHECK(h != nullptr && pts != nullptr, kErrArgument, "NULL argument");
     if (h->attached) {
       sph_s* P = h->attached;
-      P->read_ctl();
       P->flush_diag();
       P->materialize_halfstep();
       double* tmp = nullptr;
@@ -1259,11 +1300,7 @@ int gcl_get_points(gcl_t h, double* const* out) {
     GCL_CHECK(h != nullptr && out != nullptr, kErrArgument, "NULL argument");
     if (h->attached) {
       sph_s* P = h->attached;
-      P->read_ctl();
-      for (int k = 0; k < h->dim; ++k) {
-        std::vector<double> v = unsort<double>(P->xcur(k), P->idcur(), h->n, P->stream);
-        std::memcpy(out[k], v.data(), 8 * size_t(h->n));
-      }
+      for (int k = 0; k < h->dim; ++k) P->export_field<double>(P->xcur(k), 0.0, out[k]);
     } else {
       for (int k = 0; k < h->dim; ++k) {
         if (h->prec == 32) {
@@ -1271,7 +1308,7 @@ int gcl_get_points(gcl_t h, double* const* out) {
           GCL_HIP(hipMemcpy(v.data(), h->xo[k], 4 * size_t(h->n), hipMemcpyDeviceToHost));
           for (int64_t i = 0; i < h->n; ++i) out[k][i] = v[size_t(i)];
         } else {
-          GCL_HIP(hipMemcpy(out[k], h->xo[k], 8 * size_t(h->n), hipMemcpyDeviceToHost));
+          copy_out(out[k], h->xo[k], 8 * size_t(h->n), h->stream);
         }
       }
     }
@@ -1300,8 +1337,7 @@ int gcl_get_pairs(gcl_t h, int32_t* ij, int64_t cap, int64_t* written) {
     ensure_pairs(h);
     int64_t c = std::min<int64_t>(cap, h->pb.capacity);
     hipStream_t s = h->attached ? h->attached->stream : h->stream;
-    if (c > 0) GCL_HIP(hipMemcpyAsync(ij, h->pb.pairs, 8 * size_t(c), hipMemcpyDeviceToHost, s));
-    GCL_HIP(hipStreamSynchronize(s));
+    if (c > 0) copy_out(ij, h->pb.pairs, 8 * size_t(c), s);
     if (written) *written = c;
   });
 }
@@ -1310,7 +1346,6 @@ int gcl_info(gcl_t h, gcl_info_t* out) {
   return guard([&] {
     GCL_CHECK(h != nullptr && out != nullptr, kErrArgument, "NULL argument");
     if (h->attached) {
-      h->attached->read_ctl();
       h->mppcell = h->attached->hctl.mppcell;
     }
     std::memset(out, 0, sizeof(*out));
@@ -1345,7 +1380,6 @@ int gcl_get_pcell(gcl_t h, int32_t* out) {
     GCL_CHECK(h != nullptr && out != nullptr, kErrArgument, "NULL argument");
     SortBuffers& sb = h->attached ? h->attached->sb : h->sb;
     hipStream_t s = h->attached ? h->attached->stream : h->stream;
-    if (h->attached) h->attached->read_ctl();
     const int32_t* id = h->attached ? h->attached->idcur() : sb.perm;
     std::vector<int32_t> skey(size_t(h->n)), idh(size_t(h->n));
     GCL_HIP(hipMemcpyAsync(skey.data(), sb.skey, 4 * size_t(h->n), hipMemcpyDeviceToHost, s));
@@ -1484,11 +1518,9 @@ int sph_destroy(sph_t h) {
     GCL_CHECK(h->batches == 0, kErrState, "problem belongs to a batch (destroy the batch first)");
     // hand the current points back to the cell list (caller order)
     gcl_s* g = h->sys;
-    h->read_ctl();
-    for (int k = 0; k < g->dim; ++k) {
-      std::vector<double> v = unsort<double>(h->xcur(k), h->idcur(), g->n, h->stream);
-      GCL_HIP(hipMemcpy(g->xo[k], v.data(), 8 * size_t(g->n), hipMemcpyHostToDevice));
-    }
+    const int32_t* inv = h->slots_by_id();
+    for (int k = 0; k < g->dim; ++k) gather<double>(h->xcur(k), static_cast<double*>(g->xo[k]), inv, g->n, h->stream);
+    GCL_HIP(hipStreamSynchronize(h->stream));
     g->attached = nullptr;
     delete h;
     g->update(true);
@@ -1527,58 +1559,57 @@ int sph_stepsolve(sph_t h, int64_t n, int timestepping, double tl0, double tl1, 
 int sph_get_field(sph_t h, int field, double* out) {
   return guard([&] {
     GCL_CHECK(h != nullptr && out != nullptr, kErrArgument, "NULL argument");
-    h->read_ctl();
     const int64_t n = h->n;
-    const int32_t* id = h->idcur();
     const int p = h->hctl.parity;
     const double rho0 = h->par[SPH_RHO0];
-    auto put = [&](const std::vector<double>& v, int k) { std::memcpy(out + size_t(k) * size_t(n), v.data(), 8 * size_t(n)); };
-    auto vec_r = [&](auto* const* a, double add) {
-      for (int k = 0; k < h->dim; ++k) put(unsort(a[k], id, n, h->stream, add), k);
+    auto vec = [&](auto* const* a) {
+      using T = std::remove_const_t<std::remove_pointer_t<std::remove_reference_t<decltype(a[0])>>>;
+      const T* c[3] = {a[0], a[1], a[h->dim - 1]};
+      h->export_fields<T>(c, h->dim, 0.0, out);
     };
     bool sp = h->split();
     switch (field) {
       case SPH_FIELD_X:
-        for (int k = 0; k < h->dim; ++k) put(unsort<double>(h->xcur(k), id, n, h->stream), 0 + k);
+        vec(sp ? h->Bf.X[p] : h->Bd.X[p]);
         break;
       case SPH_FIELD_V:
-        if (sp) vec_r(h->Bf.V[p], 0.0);
-        else vec_r(h->Bd.V[p], 0.0);
+        if (sp) vec(h->Bf.V[p]);
+        else vec(h->Bd.V[p]);
         break;
       case SPH_FIELD_RHO:
-        if (sp) put(unsort<float>(h->Bf.RHO[p], id, n, h->stream, rho0), 0);
-        else put(unsort<double>(h->Bd.RHO[p], id, n, h->stream), 0);
+        if (sp) h->export_field<float>(h->Bf.RHO[p], rho0, out);
+        else h->export_field<double>(h->Bd.RHO[p], 0.0, out);
         break;
       case SPH_FIELD_P:  // the last pressure! call: pass 2's half-step EOS, or EOS(ρ) before DPC
-        if (sp) put(unsort<float>(h->p_from_dpc ? h->Bf.PBUF : h->Bf.PH, id, n, h->stream), 0);
-        else put(unsort<double>(h->p_from_dpc ? h->Bd.PBUF : h->Bd.PH, id, n, h->stream), 0);
+        if (sp) h->export_field<float>(h->p_from_dpc ? h->Bf.PBUF : h->Bf.PH, 0.0, out);
+        else h->export_field<double>(h->p_from_dpc ? h->Bd.PBUF : h->Bd.PH, 0.0, out);
         break;
       case SPH_FIELD_ACC:
-        if (sp) vec_r(h->Bf.ACC, 0.0);
-        else vec_r(h->Bd.ACC, 0.0);
+        if (sp) vec(h->Bf.ACC);
+        else vec(h->Bd.ACC);
         break;
       case SPH_FIELD_SUMW:
         h->flush_diag();
-        put(unsort<double>(sp ? h->Bf.SUMW : h->Bd.SUMW, id, n, h->stream), 0);
+        h->export_field<double>(sp ? h->Bf.SUMW : h->Bd.SUMW, 0.0, out);
         break;
       case SPH_FIELD_SUMGRADW:
         h->flush_diag();
-        vec_r(sp ? h->Bf.SUMGW : h->Bd.SUMGW, 0.0);
+        vec(sp ? h->Bf.SUMGW : h->Bd.SUMGW);
         break;
       case SPH_FIELD_DRHO:
-        if (sp) put(unsort<float>(h->Bf.DRHO, id, n, h->stream), 0);
-        else put(unsort<double>(h->Bd.DRHO, id, n, h->stream), 0);
+        if (sp) h->export_field<float>(h->Bf.DRHO, 0.0, out);
+        else h->export_field<double>(h->Bd.DRHO, 0.0, out);
         break;
       case SPH_FIELD_PTYPE:
-        put(unsort<int32_t>(h->ptcur(), id, n, h->stream), 0);
+        h->export_field<int32_t>(h->ptcur(), 0.0, out);
         break;
       case SPH_FIELD_DPC:  // Δv_dpc of the last step's dpcreg!; zero when the last call ran without DPC
         if (!h->p_from_dpc) {
           std::memset(out, 0, sizeof(double) * size_t(n) * size_t(h->dim));
         } else if (sp) {
-          vec_r(h->Bf.DV, 0.0);
+          vec(h->Bf.DV);
         } else {
-          vec_r(h->Bd.DV, 0.0);
+          vec(h->Bd.DV);
         }
         break;
       default:

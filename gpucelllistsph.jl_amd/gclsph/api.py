@@ -187,14 +187,18 @@ def partialupdate_(c: GPUCellList, fillzero: bool = True) -> None:
     check(lib().gcl_partialupdate(c._h, int(bool(fillzero))))
 
 
+def _pairs(c: GPUCellList, n: int) -> np.ndarray:
+    """The first n entries of the pair buffer (n <= capacity)."""
+    out = np.empty((n, 2), dtype=np.int32)
+    w = C.c_int64()
+    if n > 0:
+        check(lib().gcl_get_pairs(c._h, out.ctypes.data_as(C.POINTER(C.c_int32)), n, C.byref(w)))
+    return out
+
+
 def neighborlist(c: GPUCellList) -> np.ndarray:
     """neighborlist(c) — the whole pair buffer (capacity x 2, int32, 1-based, zero padded)."""
-    cap = c.capacity
-    out = np.zeros((max(cap, 0), 2), dtype=np.int32)
-    w = C.c_int64()
-    if cap > 0:
-        check(lib().gcl_get_pairs(c._h, out.ctypes.data_as(C.POINTER(C.c_int32)), cap, C.byref(w)))
-    return out
+    return _pairs(c, max(c.capacity, 0))
 
 
 NOALLOC_MAX_POINTS = 524288
@@ -229,7 +233,7 @@ def neighborlistview(c: GPUCellList) -> np.ndarray:
     cap = c.capacity
     if n > cap:
         raise IndexError(f"attempt to access {cap}-element pair list at index [1:{n}]")
-    return neighborlist(c)[:n]
+    return _pairs(c, n)
 
 
 # --------------------------------------------------------------------------

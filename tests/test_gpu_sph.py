@@ -341,6 +341,37 @@ def test_f64_hydrostatic_term_ranges(G, O, S, c0):
         assert rel_err(got[f], ref.get(f)) < TOL64[f], f
 
 
+@pytest.mark.parametrize("prec", ["f64", "f32split"])
+@pytest.mark.parametrize("n", [1, 65535, 65536, 65537, 131073, 700001])
+def test_fields_come_back_in_caller_order(G, S, prec, n):
+    """Getters reorder on the device and copy in chunks of 1 MiB (131,072
+    values; two components of 65,536) moved by up to four threads: counts at,
+    around and well beyond a chunk, read by two host threads at once."""
+    import threading
+
+    p, dist = S.standard_params(0.02, 2)
+    x, y = S.uniform01(3, n, 0) * 20, S.uniform01(3, n, 1) * 20
+    v = (np.float32(S.uniform01(3, n, 2)).astype(np.float64), -np.arange(n, dtype=np.float64))
+    rho = p.rho0 + np.arange(n) % 512 / 512
+    pt = (np.arange(n) % 3).astype(np.int32)
+    probs = []
+    for _ in range(2):
+        cl = G.GPUCellList((x, y), (0.1, 0.1), 0.05)
+        probs.append(G.SPHProblem.from_params(cl, p, rho, pt, v=v, precision=prec))
+    wrong = []
+
+    def read(prob):
+        got = (*G.get_points(prob), *G.get_velocity(prob), G.get_density(prob), G.get_ptype(prob), *prob.system.points)
+        wrong.extend(k for k, (a, b) in enumerate(zip(got, (x, y, *v, rho, pt, x, y))) if not np.array_equal(a, b))
+
+    threads = [threading.Thread(target=read, args=(q,)) for q in probs]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert wrong == []
+
+
 def test_argument_errors(G, S):
     sc = S.dam_break_2d(0.05, 0.5, 1.0, 2.0, 1.5)
     cl = G.GPUCellList(sc.points, sc.cellsize, sc.dist)
