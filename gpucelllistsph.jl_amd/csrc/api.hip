@@ -762,12 +762,17 @@ void LaunchSet::build(const int64_t* n, const int64_t* ncells, unsigned cnt, int
   };
   int64_t total = 0;
   for (unsigned i = 0; i < cnt; ++i) total += n[i];
+  for (scan_rows = 4; scan_rows < 16; scan_rows *= 2) {
+    int64_t tiles = 0;
+    for (unsigned i = 0; i < cnt; ++i) tiles += scan_tiles(ncells[i], scan_rows);
+    if (tiles <= kScanInOrder) break;
+  }
   quad = pair_quads(total, dim, split);
   for (unsigned i = 0; i < cnt; ++i) {
     blocks(pm, i, n[i], kBlock);
     blocks(pm512, i, n[i], 512);  // the pass kernels' 512-thread blocks
     if (quad) blocks(qm, i, n[i], 64);
-    blocks(cm, i, ncells[i], kTile);
+    blocks(cm, i, ncells[i], int64_t(scan_rows) * kScanRow);
   }
   for (auto* v : {&pm, &pm512, &qm})
     if (v->empty()) v->push_back(make_int2(0, 0));  // a no-op block (a >= n everywhere)

@@ -2,18 +2,25 @@
 // launch (used by the cell list, the pair list and the SPH step's rebuild).
 #pragma once
 
+#include <type_traits>
+
 #include "gclsph_internal.hpp"
 
 namespace gclsph {
 
 constexpr int kScanThreads = 256;
-constexpr int kScanItems = 16;
-constexpr int kTile = kScanThreads * kScanItems;  // 4096
+constexpr int kScanRow = 4 * kScanThreads;  // items of one 16-byte load per thread
 
-constexpr int64_t scan_tiles(int64_t n) { return (n + kTile - 1) / kTile; }
+// A device-wide scan runs in tiles of 4, 8 or 16 rows, a block each: as many
+// rows as keep it within kScanInOrder blocks (scan_tile below), fewest first.
+constexpr int kScanInOrder = 512;
+constexpr int64_t scan_tiles(int64_t n, int rows) { return (n + rows * kScanRow - 1) / (rows * kScanRow); }
+constexpr int scan_rows(int64_t n) {
+  return scan_tiles(n, 4) <= kScanInOrder ? 4 : (scan_tiles(n, 8) <= kScanInOrder ? 8 : 16);
+}
 // Words of the scratch array of a device-wide scan: a ticket counter, then one
 // status word per tile.
-constexpr int64_t scan_words(int64_t n) { return 1 + scan_tiles(n); }
+constexpr int64_t scan_words(int64_t n) { return 1 + scan_tiles(n, 4); }
 
 template <typename T>
 __device__ inline T wave_inclusive_scan(T v, int lane) {
@@ -25,148 +32,161 @@ __device__ inline T wave_inclusive_scan(T v, int lane) {
   return v;
 }
 
-// Exclusive block scan over kScanThreads values; returns the thread's exclusive
-// prefix and writes the block total to *total.
-template <typename T>
-__device__ inline T block_exclusive_scan(T v, T* total) {
-  __shared__ T wsum[kScanThreads / 64];
-  int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  T inc = wave_inclusive_scan(v, lane);
-  if (lane == 63) wsum[w] = inc;
-  __syncthreads();
-  T pre = 0, tot = 0;
-#pragma unroll
-  for (int k = 0; k < kScanThreads / 64; ++k) {
-    if (k < w) pre += wsum[k];
-    tot += wsum[k];
-  }
-  __syncthreads();
-  *total = tot;
-  return pre + inc - v;
-}
-
 // Clears the scratch words of the scan of n items; called by every thread (of
 // `threads` in all, this one the i-th) of a kernel before the scan's.
 __device__ __forceinline__ void clear_scan_words(uint64_t* words, int64_t n, int64_t i, int64_t threads) {
   for (; i < scan_words(n); i += threads) words[i] = 0;
 }
 
-// Exclusive scan of in[0..n) into out[0..n], out[n] = total, by scan_tiles(n)
-// blocks of kScanThreads threads in one launch (decoupled look-back).  A block
-// takes its tile from a ticket counter, publishes the tile's sum, adds up the
-// sums before it, and publishes its prefix; it waits only for tiles of earlier
-// tickets, whose blocks run and publish their sums before they wait, so every
-// wait ends whatever the order and number of blocks the chip holds.  A status
-// word holds its state and its value, so one atomic store publishes both.
-// max_out (nullable): atomic maximum of the items.  Clear: the items are zero
-// afterwards.  in and out are 16-byte aligned.
+// Exclusive scan of in[0..n) into out[0..n], out[n] = total, by
+// scan_tiles(n, Rows) blocks of kScanThreads threads in one launch (decoupled
+// look-back).  A block publishes its tile's sum, adds up the sums before it,
+// 256 tiles at a time, and publishes its prefix.  A status word holds its state
+// and its value, so one atomic store publishes both.  max_out (nullable): atomic
+// maximum of the items.  Clear: the items are zero afterwards.  in and out are
+// 16-byte aligned.
+//
+// A block waits only for tiles before its own, so every wait ends if those
+// blocks run.  In a launch of at most kScanInOrder blocks `tile` is the block's
+// place in the grid: all of them fit the chip at once (it holds 2048 such
+// blocks, an eighth of them on each XCD, and four launches can run at a time),
+// whatever else it runs.  Beyond that (tile < 0) blocks take tiles from a
+// counter, so a tile before one's own is a running block's; the counter costs
+// ~24 ns a block, one after the other.
 //
 // One launch instead of three (tile sums, their scan, the tiles again): each
 // launch of a step costs 4.4 us however small, and the items are read once.
-template <bool Clear, typename O>
+template <int Rows, bool Clear, typename O>
 __device__ __forceinline__ void scan_tile(int32_t* __restrict__ in, O* __restrict__ out, int64_t n,
-                                          uint64_t* __restrict__ words, int32_t* max_out) {
+                                          uint64_t* __restrict__ words, int32_t* max_out, int64_t tile) {
   constexpr uint64_t kSum = uint64_t(1) << 62, kPrefix = uint64_t(2) << 62, kValue = kSum - 1;
-  __shared__ uint64_t ticket, before;
-  __shared__ int32_t wmax[kScanThreads / 64];
-  if (threadIdx.x == 0) ticket = atomicAdd(reinterpret_cast<unsigned long long*>(words), 1ull);
-  __syncthreads();
-  const int64_t tile = int64_t(ticket);
-  const int64_t base = tile * kTile + int64_t(threadIdx.x) * kScanItems;
-  const bool whole = base + kScanItems <= n;  // the last tile's tail goes item by item
-  int32_t v[kScanItems];
-  if (whole) {
-    int4* p = reinterpret_cast<int4*>(in + base);
+  constexpr int kWaves = kScanThreads / 64;
+  __shared__ uint64_t ticket, wadd[kWaves];
+  __shared__ O wsum[Rows][kWaves];
+  __shared__ int32_t wmax[kWaves], wfull[kWaves];
+  if (tile < 0) {  // uniform
+    if (threadIdx.x == 0) ticket = atomicAdd(reinterpret_cast<unsigned long long*>(words), 1ull);
+    __syncthreads();
+    tile = int64_t(ticket);
+  }
+  const int lane = int(threadIdx.x & 63), wave = int(threadIdx.x >> 6);
+  const int64_t base = tile * (Rows * kScanRow) + 4 * int64_t(threadIdx.x);
+  int32_t v[Rows][4];
 #pragma unroll
-    for (int k = 0; k < kScanItems / 4; ++k) {
-      const int4 w = p[k];
-      v[4 * k] = w.x, v[4 * k + 1] = w.y, v[4 * k + 2] = w.z, v[4 * k + 3] = w.w;
-    }
-    if constexpr (Clear) {
+  for (int r = 0; r < Rows; ++r) {
+    const int64_t i = base + r * kScanRow;
+    if (i + 4 <= n) {
+      const int4 w = *reinterpret_cast<const int4*>(in + i);
+      v[r][0] = w.x, v[r][1] = w.y, v[r][2] = w.z, v[r][3] = w.w;
+      if (Clear) *reinterpret_cast<int4*>(in + i) = make_int4(0, 0, 0, 0);
+    } else {  // the end of the last tile goes item by item
 #pragma unroll
-      for (int k = 0; k < kScanItems / 4; ++k) p[k] = make_int4(0, 0, 0, 0);
-    }
-  } else {
-#pragma unroll
-    for (int k = 0; k < kScanItems; ++k) {
-      v[k] = base + k < n ? in[base + k] : 0;
-      if (Clear && base + k < n) in[base + k] = 0;
+      for (int k = 0; k < 4; ++k) {
+        v[r][k] = i + k < n ? in[i + k] : 0;
+        if (Clear && i + k < n) in[i + k] = 0;
+      }
     }
   }
-  O s = 0;
   int32_t mx = 0;
+  O pre[Rows];  // the thread's prefix in its wave's part of each row
 #pragma unroll
-  for (int k = 0; k < kScanItems; ++k) {
-    s += v[k];
-    mx = v[k] > mx ? v[k] : mx;
+  for (int r = 0; r < Rows; ++r) {
+    O s = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      s += v[r][k];
+      mx = v[r][k] > mx ? v[r][k] : mx;
+    }
+    const O inc = wave_inclusive_scan<O>(s, lane);
+    pre[r] = inc - s;
+    if (lane == 63) wsum[r][wave] = inc;
   }
   if (max_out) {
     for (int o = 32; o > 0; o >>= 1) {
       const int32_t t = __shfl_xor(mx, o, 64);
       mx = t > mx ? t : mx;
     }
-    if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = mx;
-  }
-  O total;
-  const O mine = block_exclusive_scan<O>(s, &total);
-  uint64_t* status = words + 1;
-  if (threadIdx.x < 64) {
-    const int lane = int(threadIdx.x);
-    if (lane == 0) {
-      __hip_atomic_store(status + tile, (tile == 0 ? kPrefix : kSum) | uint64_t(total), __ATOMIC_RELAXED,
-                         __HIP_MEMORY_SCOPE_AGENT);
-      if (max_out) {
-        for (int k = 1; k < kScanThreads / 64; ++k) mx = wmax[k] > mx ? wmax[k] : mx;
-        if (mx > 0) atomicMax(max_out, mx);
-      }
-    }
-    uint64_t pre = 0;
-    for (int64_t j = tile - 1; j >= 0; j -= 64) {  // 64 tiles at a time, nearest first
-      const int64_t i = j - lane;
-      uint64_t w;
-      for (;;) {
-        w = i >= 0 ? __hip_atomic_load(status + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : kPrefix;
-        if (!__any((w >> 62) == 0)) break;
-        __builtin_amdgcn_s_sleep(1);
-      }
-      const uint64_t full = __ballot((w >> 62) == 2);
-      const int last = full ? __builtin_ctzll(full) : 63;  // the nearest tile with its prefix ends the walk
-      uint64_t add = lane <= last ? w & kValue : 0;
-      for (int o = 32; o > 0; o >>= 1) add += __shfl_xor(add, o, 64);
-      pre += add;
-      if (full) break;
-    }
-    if (lane == 0) {
-      if (tile > 0)
-        __hip_atomic_store(status + tile, kPrefix | (pre + uint64_t(total)), __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
-      before = pre;
-    }
+    if (lane == 0) wmax[wave] = mx;
   }
   __syncthreads();
-  O pre = O(before) + mine;
-  if (whole) {
-    O o[kScanItems];
+  O total = 0;
 #pragma unroll
-    for (int k = 0; k < kScanItems; ++k) {
-      o[k] = pre;
-      pre += v[k];
-    }
-    int4* p = reinterpret_cast<int4*>(out + base);
+  for (int r = 0; r < Rows; ++r) {
 #pragma unroll
-    for (int k = 0; k < int(kScanItems * sizeof(O) / 16); ++k) {
-      int4 w;
-      __builtin_memcpy(&w, reinterpret_cast<const char*>(o) + 16 * k, 16);
-      p[k] = w;
-    }
-  } else {
-#pragma unroll
-    for (int k = 0; k < kScanItems; ++k) {
-      if (base + k < n) out[base + k] = pre;
-      pre += v[k];
+    for (int w = 0; w < kWaves; ++w) {
+      if (w == wave) pre[r] += total;
+      total += wsum[r][w];
     }
   }
-  if (tile == scan_tiles(n) - 1 && threadIdx.x == 0) out[n] = O(before) + total;
+  uint64_t* status = words + 1;
+  if (threadIdx.x == 0) {
+    __hip_atomic_store(status + tile, (tile == 0 ? kPrefix : kSum) | uint64_t(total), __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+    if (max_out) {
+      for (int w = 1; w < kWaves; ++w) mx = wmax[w] > mx ? wmax[w] : mx;
+      if (mx > 0) atomicMax(max_out, mx);
+    }
+  }
+  uint64_t before = 0;
+  for (int64_t j = tile - 1; j >= 0; j -= kScanThreads) {  // nearest first; uniform over the block
+    const int64_t i = j - threadIdx.x;
+    uint64_t w;
+    for (;;) {
+      w = i >= 0 ? __hip_atomic_load(status + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : kPrefix;
+      if (!__any((w >> 62) == 0)) break;
+      __builtin_amdgcn_s_sleep(1);
+    }
+    const uint64_t full = __ballot((w >> 62) == 2);
+    const int last = full ? __builtin_ctzll(full) : 63;  // the nearest tile with its prefix ends the walk
+    uint64_t add = lane <= last ? w & kValue : 0;
+    for (int o = 32; o > 0; o >>= 1) add += __shfl_xor(add, o, 64);
+    if (lane == 0) {
+      wadd[wave] = add;
+      wfull[wave] = full != 0;
+    }
+    __syncthreads();
+    bool found = false;
+#pragma unroll
+    for (int k = 0; k < kWaves; ++k) {
+      before += found ? 0 : wadd[k];
+      found |= wfull[k] != 0;
+    }
+    __syncthreads();
+    if (found) break;
+  }
+  if (threadIdx.x == 0 && tile > 0)
+    __hip_atomic_store(status + tile, kPrefix | (before + uint64_t(total)), __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+  for (int r = 0; r < Rows; ++r) {
+    const int64_t i = base + r * kScanRow;
+    O o[4];
+    o[0] = O(before) + pre[r];
+#pragma unroll
+    for (int k = 1; k < 4; ++k) o[k] = o[k - 1] + v[r][k - 1];
+    if (i + 4 <= n) {
+      int4* p = reinterpret_cast<int4*>(out + i);
+#pragma unroll
+      for (int k = 0; k < int(4 * sizeof(O) / 16); ++k) {
+        int4 w;
+        __builtin_memcpy(&w, reinterpret_cast<const char*>(o) + 16 * k, 16);
+        p[k] = w;
+      }
+    } else {
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        if (i + k < n) out[i + k] = o[k];
+    }
+  }
+  if (threadIdx.x == 0 && tile == scan_tiles(n, Rows) - 1) out[n] = O(before) + total;
+}
+
+// Calls f with the rows per tile as a constant.
+template <typename F>
+inline void with_scan_rows(int rows, F&& f) {
+  if (rows == 4) f(std::integral_constant<int, 4>());
+  else if (rows == 8) f(std::integral_constant<int, 8>());
+  else f(std::integral_constant<int, 16>());
 }
 
 }  // namespace gclsph

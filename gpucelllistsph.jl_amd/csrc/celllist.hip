@@ -66,15 +66,19 @@ __global__ void k_cellmap(XPtrs src, int64_t n, CellGeom g, int use_off64, int32
 }
 
 // Cell starts from the histogram, which is zero again afterwards.
+template <int Rows>
 __global__ __launch_bounds__(kScanThreads) void k_cell_starts(int32_t* cnt, int32_t* start, int64_t ncells,
                                                               uint64_t* words, int32_t* maxcell) {
-  scan_tile<true>(cnt, start, ncells, words, maxcell);
+  scan_tile<Rows, true>(cnt, start, ncells, words, maxcell,
+                        gridDim.x <= kScanInOrder ? int64_t(blockIdx.x) : int64_t(-1));
 }
 
 // Offsets of the pairs from their counts.
+template <int Rows>
 __global__ __launch_bounds__(kScanThreads) void k_pair_offsets(int32_t* cnt, int64_t* off, int64_t n,
                                                                uint64_t* words) {
-  scan_tile<false>(cnt, off, n, words, nullptr);
+  scan_tile<Rows, false>(cnt, off, n, words, nullptr,
+                         gridDim.x <= kScanInOrder ? int64_t(blockIdx.x) : int64_t(-1));
 }
 
 // Item visited t-th (order as in k_cellmap) to its arrival slot: tmp holds
@@ -458,7 +462,10 @@ void bin_sort_t(const CellGeom& g, const void* const* x, int64_t n, bool use_off
   k_cellmap<T, D><<<grid_for(n), kBlock, 0, s>>>(xp, n, g, use_off64 ? 1 : 0, sb.key, sb.slot, sb.cnt, order,
                                                  sb.scan_tmp, sb.maxcell);
   GCL_HIP(hipGetLastError());
-  k_cell_starts<<<unsigned(scan_tiles(nc)), kScanThreads, 0, s>>>(sb.cnt, sb.start, nc, sb.scan_tmp, sb.maxcell);
+  with_scan_rows(scan_rows(nc), [&](auto rows) {
+    k_cell_starts<rows()><<<unsigned(scan_tiles(nc, rows)), kScanThreads, 0, s>>>(sb.cnt, sb.start, nc, sb.scan_tmp,
+                                                                                  sb.maxcell);
+  });
   GCL_HIP(hipGetLastError());
   k_scatter<<<grid_for(n), kBlock, 0, s>>>(sb.key, sb.slot, sb.start, sb.tmp, sb.skey, order, n);
   GCL_HIP(hipGetLastError());
@@ -584,7 +591,9 @@ void pair_count(const CellGeom& g, int prec, const void* const* xs, const int32_
     run(dist * dist);
   }
   GCL_HIP(hipGetLastError());
-  k_pair_offsets<<<unsigned(scan_tiles(n)), kScanThreads, 0, s>>>(pb.cnt, pb.off, n, pb.scan_tmp);
+  with_scan_rows(scan_rows(n), [&](auto rows) {
+    k_pair_offsets<rows()><<<unsigned(scan_tiles(n, rows)), kScanThreads, 0, s>>>(pb.cnt, pb.off, n, pb.scan_tmp);
+  });
   GCL_HIP(hipGetLastError());
 }
 

@@ -293,7 +293,7 @@ struct SceneDev {
 // pmap512 does the same for the 512-thread blocks of the pass kernels (their
 // 128-thread blocks halve the pmap entries), and qmap for the pair kernels' blocks
 // of 64 particles with a quad of lanes each.
-// The cell scan runs one block per tile of kTile cells; cmap maps a block to (problem,
+// The cell scan runs one block per tile of scan_rows rows of cells; cmap maps a block to (problem,
 // tile).  Per-problem kernels run one block per problem.
 struct LaunchSet {
   void* scenes = nullptr;  // device SceneDev<R>[count]
@@ -303,6 +303,7 @@ struct LaunchSet {
   int2* pmap512 = nullptr;
   int2* qmap = nullptr;
   unsigned pblocks = 0, ctiles = 0, count = 0, pblocks512 = 0, qblocks = 0;
+  int scan_rows = 4;  // rows per tile of the cell scan
   bool quad = false;  // the pair kernels run a quad of lanes per particle
   bool gamma7 = true;  // γ = 7 in every problem (the FP64 passes have kernels for it)
   size_t scene_bytes = 0;

@@ -976,12 +976,13 @@ __global__ void kb_cellmap(SS ss) {
 
 // Cell starts from the histogram, which is zero again afterwards;
 // start[ncells] = n.
-template <typename R, typename SS>
+template <int Rows, typename R, typename SS>
 __global__ __launch_bounds__(kScanThreads) void kb_cell_starts(SS ss) {
   int2 m;
   const SceneDev<R>& sd = tile_scene<R>(ss, m);
   if (sd.B.ctl->rebuild == 0) return;
-  scan_tile<true>(sd.cnt, sd.start, sd.ncells, sd.scan_tmp, sd.maxcell);
+  scan_tile<Rows, true>(sd.cnt, sd.start, sd.ncells, sd.scan_tmp, sd.maxcell,
+                        gridDim.x <= kScanInOrder ? int64_t(m.y) : int64_t(-1));
 }
 
 // Sort key of an x coordinate: its bit pattern made unsigned-monotone (order
@@ -1078,7 +1079,9 @@ void launch_rebuild(const LaunchSet& L, hipStream_t s) {
   with_scenes<R>(L, [&](auto ss) {
     using SS = decltype(ss);
     kb_cellmap<D, R, SS><<<L.pblocks, kBlock, 0, s>>>(ss);
-    kb_cell_starts<R, SS><<<L.ctiles, kScanThreads, 0, s>>>(ss);
+    with_scan_rows(L.scan_rows, [&](auto rows) {
+      kb_cell_starts<rows(), R, SS><<<L.ctiles, kScanThreads, 0, s>>>(ss);
+    });
     kb_scatter<D, R, SS><<<L.pblocks, kBlock, 0, s>>>(ss);
     kb_rank<D, R, SS><<<L.pblocks, kBlock, 0, s>>>(ss);
     if constexpr (D == 2) {

@@ -52,12 +52,13 @@ def test_reference_fixture(G, O, S):
 
 
 @pytest.mark.parametrize("n", [1, 15, 4095, 4096, 4097, 20001])
-@pytest.mark.parametrize("cells", [(1, 1), (64, 64), (4097, 1), (600, 480)])
+@pytest.mark.parametrize("cells", [(1, 1), (64, 64), (4097, 1), (600, 480), (1200, 1000), (2100, 1024), (3001, 3000)])
 def test_scan_tiles(G, O, S, n, cells):
-    """Cell starts and pair offsets are scans in tiles of 4096 items that look
-    back over up to 64 tiles at a time: items and cells at, around and beyond
-    one tile, a row of cells that ends a tile by one, and 288,000 cells (71
-    tiles), most of them empty; a second binning finds the histogram cleared."""
+    """Cell starts and pair offsets are scans in tiles of 4096 items (8192 or
+    16384 beyond 2 M and 4 M, and with a ticket counter beyond 8 M) that look
+    back over 256 tiles at a time: items and cells at, around and beyond a tile,
+    a row of cells that ends a tile by one, and grids of 288,000 to 9 M cells,
+    most of them empty; a second binning finds the histogram cleared."""
     x, y = S.uniform01(11, n, 0) * cells[0], S.uniform01(11, n, 1) * cells[1]
     d = 1.0 if cells != (1, 1) else 0.05 if n > 100 else 1.0
     kw = dict(MIN=(1e-9, 1e-9), MAX=tuple(float(c) for c in cells))
