@@ -163,6 +163,7 @@ struct SphBufs {
 // y (set_pt / rec_pt).
 template <int D>
 struct alignas(16) PartnerN {
+  static constexpr size_t kPosBytes = sizeof(double) * D;
   double x[D];
   float v[D];
   float rho;  // ρ - ρ0
@@ -170,6 +171,7 @@ struct alignas(16) PartnerN {
 };
 template <>
 struct alignas(16) PartnerN<3> {
+  static constexpr size_t kPosBytes = sizeof(float) * 3;
   float xo[3];  // x - cell frame
   float v[3];
   float rho;
@@ -205,6 +207,7 @@ static_assert(sizeof(PartnerHX<2>) == 48 && sizeof(PartnerHX<3>) == 48, "partner
 // room (all but the 3D half-step record, which a seventh word would widen).
 template <int D>
 struct alignas(16) PartnerN64 {
+  static constexpr size_t kPosBytes = sizeof(double) * D;
   double x[D];
   double v[D];
   double rho;

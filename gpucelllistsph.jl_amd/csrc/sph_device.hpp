@@ -586,6 +586,20 @@ __device__ __forceinline__ T ld_rec(const void* base, uint32_t b, int64_t n) {
   return r;
 }
 
+// The words of record b that hold its position (the other fields read as zero).
+template <typename T>
+__device__ __forceinline__ T ld_pos(const void* base, uint32_t b, int64_t n) {
+  constexpr int kW = int(sizeof(T) / 16), kHead = int((T::kPosBytes + 15) / 16);
+  constexpr bool apart = RecordWords<T>::value;
+  const uint4* p = reinterpret_cast<const uint4*>(base) + (apart ? uint64_t(b) : uint64_t(b) * kW);
+  uint4 w[kW] = {};
+#pragma unroll
+  for (int i = 0; i < kHead; ++i) w[i] = p[apart ? i * n : i];
+  T r;
+  __builtin_memcpy(&r, w, sizeof(T));
+  return r;
+}
+
 template <typename T>
 __device__ __forceinline__ void st_rec(void* base, int64_t a, const T& r, int64_t n) {
   constexpr int kW = int(sizeof(T) / 16);
