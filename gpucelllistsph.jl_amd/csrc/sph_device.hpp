@@ -1031,7 +1031,6 @@ struct Own {
   R drho;  // what the records hold: ρ_a, or δρ_a in FP32-split
   R P;
   R mPi;   // -m0/ρ_a, of the pressure term
-  R kd;    // FP64: 2hδc0 of the δ-SPH term, which acts on ptype > 1 only
   int32_t pt;
 };
 template <typename R>
@@ -1043,7 +1042,6 @@ __device__ __forceinline__ Own<R> own_of(R drho, R P, int32_t pt, const SphConst
   o.pt = pt;
   if constexpr (std::is_same<R, double>::value) {
     o.rho = drho;
-    o.kd = pt > 1 ? C.DDTkh : 0.0;
     o.mPi = -C.m0 * (1.0 / drho);
   } else {
     o.rho = C.f_rho0 + drho;
@@ -1073,10 +1071,11 @@ __device__ __forceinline__ void pair_terms(const SphConst& C, const StepFlags& F
   const double dvdg = Same ? dvdx : dotm<D>(dv, dg);
   const Inv3<double> iv = pair_inv(q, rb, o.rho + rb, r2 + C.eta2);
   const bool both = o.pt > 0 && ptb > 0;
-  {  // ∂ρ/∂t: m0 dwr (dv·dg - kd (ρb - ρa - hydrostatic) (dx·dg) / (ρb (r² + η²)))
-    const double e = o.kd * ((rb - o.rho) - hydro_drho_d<G7>(C.DDTgz * dx[1], C)) * iv.den * dxdg;
-    const double s = C.m0 * dwr * fma_(-e, iv.rhob, dvdg);
-    t.v[D] = both ? s : 0.0;
+  {  // ∂ρ/∂t: m0 dwr (dv·dg - 2hδc0 (ρb - ρa - hydrostatic) (dx·dg) / (ρb (r² + η²))), diffusion for ptype > 1 only
+    const double e = C.DDTkh * ((rb - o.rho) - hydro_drho_d<G7>(C.DDTgz * dx[1], C)) * iv.den * dxdg;
+    // selected, not scaled by 0: a partner's NaN or infinite density stops here
+    const double w = o.pt > 1 ? fma_(-e, iv.rhob, dvdg) : dvdg;
+    t.v[D] = both ? C.m0 * dwr * w : 0.0;
   }
   double f = (o.P + Pb) * iv.rhob * o.mPi;             // pressure
   const double av = C.av * fmin(dvdx, 0.0) * iv.den;  // artificial viscosity, approaching pairs

@@ -227,6 +227,29 @@ def test_membership_with_candidates_exactly_at_dist(G, S, monkeypatch, prec, dim
         assert np.array_equal(a, b)
 
 
+@pytest.mark.parametrize("dim", [2, 3])
+def test_nan_reaches_the_same_densities_in_both_precisions(G, S, dim):
+    """The δ-SPH diffusion term acts on ptype > 1 only and is selected, not
+    scaled by zero: after one step with NaN velocities the FP64 densities are
+    NaN where the FP32-split ones are, wall particles (ptype 1) included."""
+    n = 1500
+    u = [S.uniform01(11, n, k) for k in range(6)]
+    p, dist = S.standard_params(0.02, dim)
+    pts = tuple(0.1 + (5.0 if dim == 3 else 18.0) * dist * u[k] for k in range(dim))
+    v = [0.1 * (c - 0.5) for c in u[3 : 3 + dim]]
+    for c in v:
+        c[::97] = np.nan
+    rho = np.full(n, p.rho0) * (1 + 1e-3 * u[0])
+    nans = {}
+    for prec in ("f64", "f32split"):
+        cl = G.GPUCellList(pts, (dist,) * dim, dist)
+        prob = G.SPHProblem.from_params(cl, p, rho, np.where(np.arange(n) % 9 == 4, 1, 2), v=tuple(v), precision=prec)
+        G.stepsolve_(prob, 1, timestepping=False)
+        nans[prec] = np.isnan(np.asarray(G.get_density(prob)))
+    assert 0 < np.count_nonzero(nans["f64"]) < n
+    assert np.array_equal(nans["f64"], nans["f32split"])
+
+
 @pytest.mark.parametrize("prec", ["f64", "f32split"])
 @pytest.mark.parametrize("case", ["dam2d", "dam2d_allphys", "dam3d_allphys"])
 def test_ptype_values_act_by_class(G, prec, case):
