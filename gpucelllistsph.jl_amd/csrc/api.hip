@@ -356,17 +356,19 @@ struct sph_s {
     B.PRH = dalloc<uint8_t>(int64_t(rh) * n);
   }
 
-  // Entry store of the membership: a particle needs at most one entry per
-  // window, 32-candidate windows of its 3^(D-1) stencil rows (each holding at
-  // most 3 * mppcell candidates), or in 3D FP32-split kWin3-candidate windows
-  // of its 27 stencil cells.  GCLSPH_NMASK_CAP lowers the capacity (particles
+  // Entry store of the membership.  Its windows are cut from 64 candidates of
+  // a stencil row at a time (Windows), a row holding at most 3 * mppcell: two
+  // windows of 32 in each 64, or in 3D FP32-split, whose windows are of kWin3
+  // candidates of one of the 27 cells, one more than the cells' own for every
+  // 64 that end inside a cell.  GCLSPH_NMASK_CAP lowers the capacity (particles
   // beyond it scan their stencil instead).  Reallocation drops the stored
   // membership.
   template <typename R>
   void ensure_nmask(SphBufs<R>& B) {
     const int64_t mpp = std::max<int64_t>({hctl.mppcell, sys->mppcell, 1});
     const bool cells = dim == 3 && std::is_same<R, float>::value;  // cell_windows<3, R>()
-    int64_t need = cells ? 27 * ((mpp + kWin3 - 1) / kWin3) : (dim == 2 ? 3 : 9) * ((3 * mpp + 31) / 32);
+    const int64_t runs = (3 * mpp + 63) / 64;                      // of 64 candidates in a row
+    int64_t need = cells ? 27 * ((mpp + kWin3 - 1) / kWin3) + 9 * (runs - 1) : (dim == 2 ? 3 : 9) * 2 * runs;
     if (const char* env = std::getenv("GCLSPH_NMASK_CAP")) {
       const long v = std::strtol(env, nullptr, 10);
       if (v >= 0 && v < need) need = v;

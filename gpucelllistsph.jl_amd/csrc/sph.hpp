@@ -113,7 +113,7 @@ struct SphBufs {
   StepCtl* ctl;
   double* RED;  // per-block partial maxima: [|cdx|, |a|, visc] x nblk
   int nblk;
-  // neighbour-list membership of the last rebuild (k_nmask): entry e of
+  // neighbour-list membership of the last rebuild (written with the reorder): entry e of
   // particle a at NE[e * n + a] = (window base << 32) | member bits; NC[a]
   // entries, or -1 when more than necap were needed
   uint64_t* NE;

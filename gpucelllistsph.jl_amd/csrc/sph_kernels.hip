@@ -36,7 +36,7 @@ __device__ __forceinline__ uint32_t window_mask(uint32_t acc, int32_t len, int64
   const int32_t nc = (len + 3) & ~3;
   uint32_t mk = __builtin_bitreverse32(acc << (32 - nc));
   if (len < 32) mk &= (1u << len) - 1u;
-  const int64_t self = a - lo;
+  const int32_t self = int32_t(a) - lo;
   if (self >= 0 && self < len) mk &= ~(1u << self);
   return mk;
 }
@@ -64,26 +64,25 @@ __device__ __forceinline__ uint32_t window_bits_lds(const double2* lp, double xa
   return window_mask(acc, len, a, lo);
 }
 
-// 3D: the same over positions staged as three arrays (x, y, z).
-__device__ __forceinline__ uint32_t window_bits_lds3(const double* lx, const double* ly, const double* lz, double xa0,
-                                                     double xa1, double xa2, int64_t a, int32_t lo, int32_t hi,
-                                                     double dist2) {
+// 3D: the same over positions staged as (x, y) pairs and z.
+__device__ __forceinline__ uint32_t window_bits_lds3(const double2* lp, const double* lz, double xa0, double xa1,
+                                                     double xa2, int64_t a, int32_t lo, int32_t hi, double dist2) {
 #pragma clang fp contract(off)
   const int32_t len = hi - lo;
   uint32_t acc = 0;
   for (int32_t j = 0; j < len; j += 4) {
-    double c0[4], c1[4], c2[4];
+    double2 c[4];
+    double c2[4];
     double r[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      c0[u] = lx[j + u];
-      c1[u] = ly[j + u];
+      c[u] = lp[j + u];
       c2[u] = lz[j + u];
     }
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      const double d0 = xa0 - c0[u];
-      const double d1 = xa1 - c1[u];
+      const double d0 = xa0 - c[u].x;
+      const double d1 = xa1 - c[u].y;
       const double d2 = xa2 - c2[u];
       double r2 = d0 * d0 + d1 * d1;
       r[u] = r2 + d2 * d2;
@@ -95,224 +94,106 @@ __device__ __forceinline__ uint32_t window_bits_lds3(const double* lx, const dou
 
 // The candidates of a stencil row that can pass the membership test, where
 // the rank orders every cell by x (so a row, three consecutive cells of one
-// y and z, is in x order): [lo, hi) narrowed by bisection over the staged
-// x (lx[b] of candidate b) to the first b with xa - x_b < dist and, from
-// there, the first b with xa - x_b <= -dist.  Every candidate outside has
-// |fl(xa - x_b)| >= dist, the same FP64 difference the test squares, so its
-// r^2 rounds to at least fl(dist^2) = dist2 and the test fails.  A NaN
-// coordinate (never a member: its r^2 is NaN) compares false both ways; the
-// bisection still only drops candidates whose real x lies beyond an x it
-// found outside the range, since the real x are in order.
-__device__ __forceinline__ void x_range(const double* lx, double xa, double dist, int32_t& lo, int32_t& hi) {
-  int32_t n = hi - lo;
-  while (n > 0) {
-    const int32_t h = n >> 1;
-    if (xa - lx[lo + h] >= dist) {
-      lo += h + 1;
-      n -= h + 1;
-    } else {
-      n = h;
-    }
+// y and z, is in x order): [lo, hi) (at most 256) narrowed by bisection over the
+// staged x (lp[b].x of candidate b) to the first b with xa - x_b < dist and, from
+// there, the first b with xa - x_b <= -dist; the two searches go in step, their
+// loads in flight together.  Every candidate outside has |fl(xa - x_b)| >=
+// dist, the same FP64 difference the test squares, so its r^2 rounds to at
+// least fl(dist^2) = dist2 and the test fails.  A NaN coordinate (never a
+// member: its r^2 is NaN) compares false both ways; the bisection still only
+// drops candidates whose real x lies beyond an x it found outside the range,
+// since the real x are in order.
+__device__ __forceinline__ void x_range(const double2* lp, double xa, double dist, int32_t& lo, int32_t& hi) {
+  if (lo >= hi) return;
+  int32_t l = lo, u = lo;
+#pragma unroll
+  for (int32_t step = 128; step > 0; step >>= 1) {
+    const int32_t pl = l + step, pu = u + step;
+    const double dl = xa - lp[(pl < hi ? pl : hi) - 1].x, du = xa - lp[(pu < hi ? pu : hi) - 1].x;
+    l = pl <= hi && dl >= dist ? pl : l;
+    u = pu <= hi && !(du <= -dist) ? pu : u;
   }
-  int32_t b = lo;
-  n = hi - lo;
-  while (n > 0) {
-    const int32_t h = n >> 1;
-    if (xa - lx[b + h] <= -dist) {
-      n = h;
-    } else {
-      b += h + 1;
-      n -= h + 1;
-    }
-  }
-  hi = b;
+  // 255 of 256 reached
+  if (l < hi && xa - lp[l].x >= dist) ++l;
+  if (u < hi && !(xa - lp[u].x <= -dist)) ++u;
+  lo = l;
+  hi = u;
 }
 
-// Row windows as stored: up to 32 candidates from a first member, the member
-// bits of the consecutive test windows of one row merged into the pending
-// window while they fall inside it (fewer, fuller windows for the pair
-// loops).  add() in row order, flush() at the end of the row.
-struct RowWindows {
+// Least real distance along one axis from coordinate x in cell i (0-based) to
+// any point binned into cell i + o, o in {-1, 0, 1}, less a margin for the
+// rounding of the binning; edge cells, which also hold what lies outside the
+// grid, reach outward only.  0 for NaN.
+__device__ __forceinline__ double axis_gap(double x, double off, double cs, int64_t i, int o) {
+  if (o == 0) return 0.0;
+  const double u = x - off, edge = double(o > 0 ? i + 1 : i) * cs;
+  const double gap = o > 0 ? edge - u : u - edge;
+  return fmax(gap - 1e-13 * (fabs(u) + fabs(edge) + cs), 0.0);
+}
+
+// The stored windows of a particle: each starts at a member and holds the
+// members among the next 32 candidates (row) or the next kWin3 of its cell
+// (cells), from the member bits of up to 64 candidates of a row at a time.
+struct Windows {
   uint64_t* out;
   int64_t n;
   int cap;
-  int& cnt;
-  int32_t pb = 0;
-  uint32_t pm = 0;
-  __device__ __forceinline__ void flush() {
-    if (pm != 0) {
-      if (cnt < cap) out[int64_t(cnt) * n] = (uint64_t(uint32_t(pb)) << 32) | pm;
-      ++cnt;
-      pm = 0;
+  int cnt = 0;
+  __device__ __forceinline__ void put(int32_t base, uint32_t bits) {
+    if (cnt < cap) out[int64_t(cnt) * n] = (uint64_t(uint32_t(base)) << 32) | bits;
+    ++cnt;
+  }
+  // bit t: candidate b + t
+  __device__ __forceinline__ void row(int32_t b, uint64_t bits) {
+    while (bits != 0) {
+      const int t0 = __builtin_ctzll(bits);
+      b += t0;
+      bits >>= t0;
+      put(b, uint32_t(bits));
+      b += 32;
+      bits >>= 32;
     }
   }
-  __device__ __forceinline__ void add(int32_t w0, uint32_t mk) {
-    uint64_t rest = mk;
-    while (rest != 0) {
-      const int t0 = __builtin_ctzll(rest);
-      const int32_t b0 = w0 + t0;
-      if (pm == 0 || b0 >= pb + 32) {
-        flush();
-        pb = b0;
+  // the same of the row's three cells, cell ox = j - 1 being [sb[j], sb[j + 1])
+  __device__ __forceinline__ void cells(int32_t b, uint64_t bits, const int32_t* sb, int oy, int oz) {
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      const int32_t e = sb[j + 1] - b;  // candidates left in the cell
+      if (e <= 0) continue;
+      uint64_t in = bits;
+      int32_t c = b;
+      if (e < 64) {
+        in &= (uint64_t(1) << e) - 1u;
+        bits >>= e;
+        b += e;
+      } else {
+        bits = 0;
       }
-      const uint64_t lm = (uint64_t(1) << (pb + 32 - b0)) - 1u;  // 1..32 bits
-      pm |= uint32_t(((rest >> t0) & lm) << (b0 - pb));
-      rest &= ~(lm << t0);
+      while (in != 0) {
+        const int t0 = __builtin_ctzll(in);
+        c += t0;
+        in >>= t0;
+        put(c, (win_code3(j - 1, oy, oz) << kWin3) | (uint32_t(in) & kWinMask3));
+        c += kWin3;
+        in >>= kWin3;
+      }
     }
   }
 };
-
-// Candidates staged in LDS: 2D 400 positions per wave (the union of a wave's
-// three stencil rows holds ~300 on a uniform lattice), 26 KiB per block, six
-// blocks per CU; 3D 1280 per block and plane of three stencil rows, 32 KiB.
-constexpr int kNmaskWave = 400;
-constexpr int kNmaskPlane = 1280;
-
-// Neighbour-list membership of the last rebuild, stored per particle as
-// (mask, base) entries: one window of candidates [base, base + len) with its
-// member bits in the low word.  Windows of up to 32 candidates of one
-// stencil row, or in 3D FP32-split of up to kWin3 candidates inside one
-// stencil cell with the cell's offset coded above the member bits
-// (win_code3), which is what the cell frames of its partner records need.
-// Each window starts at a member (the first one not covered by the window
-// before it), so with the rows in x order a particle's partners fill few
-// windows; stored in stencil order.  Entry e of particle a is NE[e * n + a]; NC[a]
-// is the entry count, or -1 when the particle needs more than necap entries
-// (its partners are then found by scanning the stencil).
-//
-// k_nmask is the 3D store (the 2D one runs inside k_reorder_nmask2 below):
-// the block stages the candidates' positions plane by plane (three stencil
-// rows at a time, ~1000 candidates per particle in all) and every lane tests
-// there the candidates of each row within dist of it in x (x_range, ~46 % of
-// them); a block whose union exceeds the LDS budget reads the whole rows from
-// global memory.  The tests are the same expression in every path, so the
-// bits are the same.
-template <int D, typename R, typename SS>
-__global__ __launch_bounds__(256) void k_nmask(SS ss) {
-  static_assert(D == 3, "the 2D membership store is part of k_reorder_nmask2");
-  GCLSPH_SCENE(ss);
-  const StepCtl* ctl = B.ctl;
-  if (!ctl->rebuild) return;
-  const int64_t a0 = int64_t(m.y) * kBlock;
-  if (a0 >= B.n) return;  // whole block
-  const bool active = a < B.n;
-  const double dist2 = C.dist2;
-  const int p = cur_parity(ctl);  // the rebuild positions are the current ones
-  const double* XM[3] = {B.X[p][0], B.X[p][1], B.X[p][D == 3 ? 2 : 1]};
-  const int cap = B.necap;
-  uint64_t* out = B.NE + a;
-  __shared__ double lx[kNmaskPlane + 4], ly[kNmaskPlane + 4], lz[kNmaskPlane + 4];  // +4: window reads run up to 3 past a row's end
-  __shared__ RowUnion u;
-  double xa0 = 0.0, xa1 = 0.0, xa2 = 0.0;
-  int64_t ix = 0, iy = 0, iz = 0;
-  if (active) {
-    xa0 = XM[0][a];
-    xa1 = XM[1][a];
-    xa2 = XM[2][a];
-    cell_xyz<3>(G, B.skey[a], ix, iy, iz);
-  }
-  const int64_t gx = G.grid[0], gy = G.grid[1], gz = G.grid[2], nce = G.ncells();
-  int cnt = 0;
-#pragma unroll
-  for (int pl = 0; pl < 3; ++pl) {  // rows 3·pl .. 3·pl+2 lie in the plane dz = pl - 1
-    // the cell boundaries of the particle's three rows in this plane, loaded
-    // together before the staging: cell ox = j - 1 of row kk is [sb[kk][j],
-    // sb[kk][j + 1]) when it lies in the grid (indices clamped for the load)
-    const int64_t z = iz + pl - 1;
-    int32_t sb[3][4];
-#pragma unroll
-    for (int kk = 0; kk < 3; ++kk) {
-      const int64_t y = iy + kk - 1;
-      const int64_t row = gx * (y + gy * z);
-      const bool in = active && y >= 0 && y < gy && z >= 0 && z < gz;
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        int64_t i = row + ix - 1 + t;
-        i = i < 0 ? 0 : (i > nce ? nce : i);
-        sb[kk][t] = in ? B.start[i] : 0;
-      }
-    }
-    if (threadIdx.x == 0) row_union(u, B.start, B.skey, G, B.n, a0, pl - 1);
-    __syncthreads();
-    const int32_t total = u.uo[3];
-    const bool staged = total <= kNmaskPlane;  // uniform over the block
-    if (staged) {
-      for (int32_t i = threadIdx.x; i < total; i += kBlock) {
-        const int k = (i >= u.uo[1]) + (i >= u.uo[2]);
-        const int32_t b = u.ub[k] + (i - u.uo[k]);
-        lx[i] = XM[0][b];
-        ly[i] = XM[1][b];
-        lz[i] = XM[2][b];
-      }
-    }
-    __syncthreads();
-    if (active) {
-#pragma unroll
-      for (int kk = 0; kk < 3; ++kk) {
-        const int64_t y = iy + kk - 1;
-        if (y < 0 || y >= gy || z < 0 || z >= gz) continue;
-        const int32_t off = u.uo[kk] - u.ub[kk];  // candidate b at l?[b + off]
-        auto test = [&](int32_t w0, int32_t hi) {
-          return staged ? window_bits_lds3(lx + (w0 + off), ly + (w0 + off), lz + (w0 + off), xa0, xa1, xa2, a, w0, hi,
-                                           dist2)
-                        : window_bits<D>(XM[0], XM[1], XM[2], xa0, xa1, xa2, a, w0, hi, dist2);
-        };
-        // the row's candidates in the grid, narrowed to |x_a - x_b| < dist
-        // where they are staged, tested in 32-candidate windows (one trip
-        // count for every lane of the wave, whatever its x in its cell)
-        int32_t rb = ix >= 1 ? sb[kk][0] : sb[kk][1];
-        int32_t re = ix + 1 < gx ? sb[kk][3] : sb[kk][2];
-        if (staged) x_range(lx + off, xa0, C.dist, rb, re);
-        // in 3D FP32-split the member bits are stored as windows of one cell
-        // (the cell frames of the records need it), merged across the test
-        // windows: from a first member, up to kWin3 candidates of its cell
-        // (ox = pj - 1); pm holds the pending window's bits
-        int32_t pb = 0;
-        int pj = 0;
-        uint32_t pm = 0;
-        RowWindows rw{out, B.n, cap, cnt};  // FP64: 32-candidate row windows
-        auto flush = [&]() {
-          if (pm != 0) {
-            const uint64_t code = uint64_t(win_code3(pj - 1, kk - 1, pl - 1)) << kWin3;
-            if (cnt < cap) out[int64_t(cnt) * B.n] = (uint64_t(uint32_t(pb)) << 32) | code | pm;
-            ++cnt;
-            pm = 0;
-          }
-        };
-        for (int32_t w0 = rb; w0 < re; w0 += 32) {
-          const int32_t hi = re < w0 + 32 ? re : w0 + 32;
-          const uint32_t mk = test(w0, hi);
-          if constexpr (cell_windows<D, R>()) {
-            uint64_t rest = mk;
-            while (rest != 0) {
-              const int t0 = __builtin_ctzll(rest);
-              const int32_t b0 = w0 + t0;
-              const int j = (b0 >= sb[kk][1]) + (b0 >= sb[kk][2]);
-              if (pm == 0 || j != pj || b0 >= pb + int32_t(kWin3)) {
-                flush();
-                pb = b0;
-                pj = j;
-              }
-              // this test window's bits from b0 to the end of the pending
-              // window or of the cell, whichever comes first (1..kWin3 of them)
-              const int32_t ce = sb[kk][j + 1], we = pb + int32_t(kWin3);
-              const uint64_t lm = (uint64_t(1) << ((ce < we ? ce : we) - b0)) - 1u;
-              pm |= uint32_t(((rest >> t0) & lm) << (b0 - pb));
-              rest &= ~(lm << t0);
-            }
-          } else {
-            rw.add(w0, mk);
-          }
-        }
-        if constexpr (cell_windows<D, R>()) flush();
-        else rw.flush();
-      }
-    }
-    __syncthreads();  // the next plane overwrites the staged positions
-  }
-  if (active) B.NC[a] = cnt <= cap ? cnt : -1;
-  return;
+// test(lo, hi): member bits of up to 32 candidates; of up to 64 here.
+template <typename Test>
+__device__ __forceinline__ uint64_t bits64(int32_t lo, int32_t hi, const Test& test) {
+  const int32_t mid = hi < lo + 32 ? hi : lo + 32;
+  uint64_t bits = test(lo, mid);
+  if (mid < hi) bits |= uint64_t(test(mid, hi)) << 32;
+  return bits;
 }
+
+// Candidates staged in LDS per wave: 2D 400 positions (the union of a wave's
+// three stencil rows holds ~300 on a uniform lattice), 26 KiB per block, six
+// blocks per CU; 3D one row at a time, 256 positions (~180), 25 KiB.
+constexpr int kNmaskWave = 400;
+constexpr int kNmaskRow = 256;
 
 // ------------------------------------------------------------------ kernels
 // Commits the rebuild of a problem (one thread per problem): the reordered
@@ -387,20 +268,126 @@ __device__ __forceinline__ void reorder_one(const SphBufs<R>& B, const SphConst&
   B.ID[pq][s] = B.ID[pp][src];
 }
 
-template <int D, typename R, typename SS>
-__global__ void k_reorder(SS ss) {
-  GCLSPH_SCENE(ss);
-  const StepCtl* ctl = B.ctl;
-  if (ctl->rebuild == 0) return;
-  if (a >= B.n) return;
-  double xs[3];
-  reorder_one<D, R>(B, C, G, F, ctl, a, xs);
+// Neighbour-list membership of the last rebuild, stored per particle as
+// (mask, base) entries: one window of candidates [base, base + len) with its
+// member bits in the low word.  Windows of up to 32 candidates of one
+// stencil row, or in 3D FP32-split of up to kWin3 candidates inside one
+// stencil cell with the cell's offset coded above the member bits
+// (win_code3), which is what the cell frames of its partner records need.
+// Each window starts at a member (the first one not covered by the window
+// before it), so with the rows in x order a particle's partners fill few
+// windows; stored in stencil order.  Entry e of particle a is NE[e * n + a]; NC[a]
+// is the entry count, or -1 when the particle needs more than necap entries
+// (its partners are then found by scanning the stencil).
+//
+// It runs in the kernel that reorders the state, from the rebuild positions in
+// the new order, which the rank kernel wrote (the other fields move in this
+// kernel, which needs no other block's writes).  xa: a's rebuild position.
+// Wave-level only (no block barrier).
+//
+// 3D: a wave takes its 9 stencil rows one after the other: it stages the
+// candidates of a row of all its particles in its LDS slice, the next row's
+// loads in flight, and every lane tests its own row there: the candidates whose
+// x lies within the half width that the row's distance in y and z leaves of
+// the sphere (~330 of the ~1050 candidates of a particle).  A row beyond the
+// slice is tested whole from global memory: same expression, same bits.  Bound
+// by the LDS reads of the tests (24 B each, lanes at different places).
+// 883,376 particles: 0.50 ms staged by the block, a plane at a time behind two
+// barriers, narrowed to |x_a - x_b| < dist only, and in a launch of its own (its
+// reorder 36 us more); with the reorder 0.45 ms here.  31,962: 95 + 7 -> 84 us.
+template <typename R>
+__device__ __forceinline__ void nmask3_new(const SphBufs<R>& B, const SphConst& C, const CellGeom& G,
+                                           const StepCtl* ctl, int64_t a, int64_t a0, const double* xa,
+                                           double2 (*lds_xy)[kNmaskRow + 4], double (*lds_z)[kNmaskRow + 4]) {
+  const bool active = a < B.n;
+  const double dist2 = C.dist2;
+  const int q = ctl->parity ^ 1;  // the new order (committed after this kernel)
+  const double* XN[3] = {B.X[q][0], B.X[q][1], B.X[q][2]};
+  Windows win{B.NE + a, B.n, B.necap};
+  const int w = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+  const int lane = int(threadIdx.x & 63);
+  const int64_t aw = a0 + 64 * w;
+  if (aw >= B.n) return;  // whole wave
+  double2* lxy = lds_xy[w];
+  double* lz = lds_z[w];
+  const int64_t gx = G.grid[0], gy = G.grid[1], gz = G.grid[2], nce = G.ncells();
+  // the wave's candidates of row r: one contiguous range [ub, ue)
+  const int64_t c0 = B.skey[aw], c1 = B.skey[aw + 63 < B.n ? aw + 63 : B.n - 1];
+  auto row_offset = [&](int r) { return gx * (r % 3 - 1) + gx * gy * (r / 3 - 1); };
+  auto bound_of = [&](int64_t c) { return B.start[c < 0 ? 0 : (c > nce ? nce : c)]; };
+  constexpr int kSlots = kNmaskRow / 64;
+  double v[kSlots][3];
+  int32_t ub, ue;
+  auto prefetch = [&](int r) {
+    ub = bound_of(c0 + row_offset(r) - 1);
+    ue = bound_of(c1 + row_offset(r) + 2);
+    if (ue - ub > kNmaskRow) return;
+#pragma unroll
+    for (int t = 0; t < kSlots; ++t) {
+      const int32_t b = ub + lane + 64 * t;
+      if (b < ue) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) v[t][k] = XN[k][b];
+      }
+    }
+  };
+  int64_t ix = 0, iy = 0, iz = 0;
+  cell_xyz<3>(G, B.skey[active ? a : aw], ix, iy, iz);
+  double cs[3];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) cs[k] = 1.0 / G.hinv64[k];
+  prefetch(0);
+#pragma unroll 1
+  for (int r = 0; r < 9; ++r) {
+    const int oy = r % 3 - 1, oz = r / 3 - 1;
+    const int32_t wb = ub;
+    const bool staged = ue - ub <= kNmaskRow;  // uniform over the wave
+    if (staged) {
+#pragma unroll
+      for (int t = 0; t < kSlots; ++t) {
+        if (ub + lane + 64 * t < ue) {
+          lxy[lane + 64 * t] = make_double2(v[t][0], v[t][1]);
+          lz[lane + 64 * t] = v[t][2];
+        }
+      }
+    }
+    // the cell boundaries of the particle's row: cell ox = j - 1 is
+    // [sb[j], sb[j + 1]) when it lies in the grid
+    const int64_t y = iy + oy, z = iz + oz;
+    const bool in = active && y >= 0 && y < gy && z >= 0 && z < gz;
+    int32_t sb[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) sb[t] = in ? bound_of(gx * (y + gy * z) + ix - 1 + t) : 0;
+    if (r < 8) prefetch(r + 1);
+    // the wave's LDS operations complete in issue order; the fence keeps the
+    // compiler from moving the reads below ahead of these writes
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    const double gap_y = axis_gap(xa[1], G.off64[1], cs[1], iy, oy), gap_z = axis_gap(xa[2], G.off64[2], cs[2], iz, oz);
+    const double h2 = dist2 * (1.0 + 1e-12) - (gap_y * gap_y + gap_z * gap_z);
+    if (in && !(h2 < 0.0)) {
+      int32_t rb = ix >= 1 ? sb[0] : sb[1];
+      int32_t re = ix + 1 < gx ? sb[3] : sb[2];
+      const double2* lp = lxy - wb;  // candidate b at lp[b]
+      const double* lq = lz - wb;
+      if (staged) x_range(lp, xa[0], fmin(C.dist, sqrt(h2) * (1.0 + 1e-12)), rb, re);
+      auto test = [&](int32_t lo, int32_t hi) {
+        return staged ? window_bits_lds3(lp + lo, lq + lo, xa[0], xa[1], xa[2], a, lo, hi, dist2)
+                      : window_bits<3>(XN[0], XN[1], XN[2], xa[0], xa[1], xa[2], a, lo, hi, dist2);
+      };
+      for (int32_t w0 = rb; w0 < re; w0 += 64) {
+        const uint64_t bits = bits64(w0, re < w0 + 64 ? re : w0 + 64, test);
+        // FP32-split: windows of one cell (the cell frames of the records need it)
+        if constexpr (cell_windows<3, R>()) win.cells(w0, bits, sb, oy, oz);
+        else win.row(w0, bits);
+      }
+    }
+    __builtin_amdgcn_wave_barrier();  // the next row overwrites the staged positions
+  }
+  if (active) B.NC[a] = win.cnt <= win.cap ? win.cnt : -1;
 }
 
-// Membership store (k_nmask's 2D path) of particle a, from the rebuild
-// positions in the new order, which the rank kernel wrote (the other fields
-// move in this kernel, which needs no other block's writes).  xa: a's
-// rebuild position.  Wave-level only (no block barrier).
+// 2D: the wave stages the union of its three rows at once.
 template <typename R>
 __device__ __forceinline__ void nmask2_new(const SphBufs<R>& B, const SphConst& C, const CellGeom& G,
                                            const StepCtl* ctl, int64_t a, int64_t a0, const double* xa,
@@ -409,8 +396,7 @@ __device__ __forceinline__ void nmask2_new(const SphBufs<R>& B, const SphConst& 
   const double dist2 = C.dist2;
   const int q = ctl->parity ^ 1;  // the new order (committed after this kernel)
   const double* XN[2] = {B.X[q][0], B.X[q][1]};
-  const int cap = B.necap;
-  uint64_t* out = B.NE + a;
+  Windows win{B.NE + a, B.n, B.necap};
   const int w = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
   const int lane = int(threadIdx.x & 63);
   const int64_t aw = a0 + 64 * w;
@@ -418,7 +404,6 @@ __device__ __forceinline__ void nmask2_new(const SphBufs<R>& B, const SphConst& 
   RowUnion u;
   row_union(u, B.start, B.skey, G, B.n, aw, 0, 64);
   const int32_t total = u.uo[3];
-  int cnt = 0;
   if (total <= kNmaskWave) {  // uniform over the wave
     double2* wl = lds[w];
     const int32_t d0 = u.ub[0] - u.uo[0], d1 = u.ub[1] - u.uo[1], d2 = u.ub[2] - u.uo[2];
@@ -447,33 +432,30 @@ __device__ __forceinline__ void nmask2_new(const SphBufs<R>& B, const SphConst& 
         const double2* lrow = wl + (u.uo[k] - u.ub[k]);  // candidate b at lrow[b]
         // (a row of ~35 candidates: bounding it to |x_a - x_b| < dist by
         // bisection, as in 3D, costs more than the tests it saves)
-        RowWindows rw{out, B.n, cap, cnt};
-        for (int32_t w0 = rows.b[k]; w0 < rows.e[k]; w0 += 32) {
-          const int32_t hi = rows.e[k] < w0 + 32 ? rows.e[k] : w0 + 32;
-          rw.add(w0, window_bits_lds(lrow + w0, xa[0], xa[1], a, w0, hi, dist2));
-        }
-        rw.flush();
+        auto test = [&](int32_t lo, int32_t hi) {
+          return window_bits_lds(lrow + lo, xa[0], xa[1], a, lo, hi, dist2);
+        };
+        for (int32_t w0 = rows.b[k]; w0 < rows.e[k]; w0 += 64)
+          win.row(w0, bits64(w0, rows.e[k] < w0 + 64 ? rows.e[k] : w0 + 64, test));
       }
     }
   } else if (active) {
     const Rows<2> rows = stencil_rows<2>(G, B.start, B.skey[a]);
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-      RowWindows rw{out, B.n, cap, cnt};
-      for (int32_t w0 = rows.b[k]; w0 < rows.e[k]; w0 += 32) {
-        const int32_t hi = rows.e[k] < w0 + 32 ? rows.e[k] : w0 + 32;
-        rw.add(w0, window_bits<2>(XN[0], XN[1], XN[1], xa[0], xa[1], 0.0, a, w0, hi, dist2));
-      }
-      rw.flush();
+      auto test = [&](int32_t lo, int32_t hi) {
+        return window_bits<2>(XN[0], XN[1], XN[1], xa[0], xa[1], 0.0, a, lo, hi, dist2);
+      };
+      for (int32_t w0 = rows.b[k]; w0 < rows.e[k]; w0 += 64)
+        win.row(w0, bits64(w0, rows.e[k] < w0 + 64 ? rows.e[k] : w0 + 64, test));
     }
   }
-  if (active) B.NC[a] = cnt <= cap ? cnt : -1;
+  if (active) B.NC[a] = win.cnt <= win.cap ? win.cnt : -1;
 }
 
-// 2D rebuild tail in one kernel: the reorder of the state and the membership
+// Rebuild tail in one kernel: the reorder of the state and the membership
 // store of the same particles, which are independent of each other (one
-// launch instead of two; both parts are bound by vector-memory traffic, so
-// they add up rather than overlap).  Same tests, same bits as k_nmask.
+// launch instead of two).
 template <typename R, typename SS>
 __global__ __launch_bounds__(256) void k_reorder_nmask2(SS ss) {
   GCLSPH_SCENE(ss);
@@ -485,6 +467,20 @@ __global__ __launch_bounds__(256) void k_reorder_nmask2(SS ss) {
   double xa[3] = {0.0, 0.0, 0.0};
   if (a < B.n) reorder_one<2, R>(B, C, G, F, ctl, a, xa);
   nmask2_new<R>(B, C, G, ctl, a, a0, xa, lds);
+}
+
+template <typename R, typename SS>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_reorder_nmask3(SS ss) {
+  GCLSPH_SCENE(ss);
+  const StepCtl* ctl = B.ctl;
+  if (ctl->rebuild == 0) return;
+  const int64_t a0 = int64_t(m.y) * kBlock;
+  if (a0 >= B.n) return;  // whole block
+  __shared__ double2 lds_xy[kBlock / 64][kNmaskRow + 4];  // +4: window reads run up to 3 past a row's end
+  __shared__ double lds_z[kBlock / 64][kNmaskRow + 4];
+  double xa[3] = {0.0, 0.0, 0.0};
+  if (a < B.n) reorder_one<3, R>(B, C, G, F, ctl, a, xa);
+  nmask3_new<R>(B, C, G, ctl, a, a0, xa, lds_xy, lds_z);
 }
 
 // ---- corrections after the update (src/sphproblem.jl:303-322) --------------
@@ -1099,12 +1095,8 @@ void launch_rebuild(const LaunchSet& L, hipStream_t s) {
     });
     kb_scatter<D, R, SS><<<L.pblocks, kBlock, 0, s>>>(ss);
     kb_rank<D, R, SS><<<L.pblocks, kBlock, 0, s>>>(ss);
-    if constexpr (D == 2) {
-      k_reorder_nmask2<R, SS><<<L.pblocks, kBlock, 0, s>>>(ss);
-    } else {
-      k_reorder<D, R, SS><<<L.pblocks, kBlock, 0, s>>>(ss);
-      k_nmask<D, R, SS><<<L.pblocks, kBlock, 0, s>>>(ss);
-    }
+    if constexpr (D == 2) k_reorder_nmask2<R, SS><<<L.pblocks, kBlock, 0, s>>>(ss);
+    else k_reorder_nmask3<R, SS><<<L.pblocks, kBlock, 0, s>>>(ss);
   });
 }
 template <int D, typename R>

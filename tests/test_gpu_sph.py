@@ -251,6 +251,40 @@ def test_nan_reaches_the_same_densities_in_both_precisions(G, S, dim):
 
 
 @pytest.mark.parametrize("prec", ["f64", "f32split"])
+@pytest.mark.parametrize("kind", ["dense", "wide", "outside"])
+def test_membership_3d_rows(G, S, monkeypatch, prec, kind):
+    """The 3D membership store narrows a stencil row by its distance from the
+    particle and tests it from a 256-entry slice: rows longer than the slice and
+    than one mask of 64 (dense), cells wider than dist (wide), particles far
+    outside the grid, binned into its edge cells (outside), give the steps of the full stencil scan (GCLSPH_NMASK_CAP=0) bit for bit."""
+    n = 1500
+    u = [S.uniform01(11, n, k) for k in range(6)]
+    p, dist = S.standard_params(0.02, 3)
+    side = 2.2 * dist if kind == "dense" else 5.0 * dist
+    cell = (1.37 if kind == "wide" else 1.0) * dist
+    pts = tuple(0.1 + side * u[k] for k in range(3))
+    v = np.stack([0.1 * (c - 0.5) for c in u[3:]])
+    if kind == "outside":
+        v[:, ::5] *= 20.0 * 3.0 * dist / p.dt  # up to 3 dist along an axis in a step
+    rho = np.full(n, p.rho0) * (1 + 1e-3 * u[0])
+
+    def run(cap):
+        if cap is None:
+            monkeypatch.delenv("GCLSPH_NMASK_CAP", raising=False)
+        else:
+            monkeypatch.setenv("GCLSPH_NMASK_CAP", str(cap))
+        cl = G.GPUCellList(pts, (cell,) * 3, dist)
+        prob = G.SPHProblem.from_params(cl, p, rho, np.where(np.arange(n) % 9 == 4, 1, 2), v=tuple(v), precision=prec)
+        G.stepsolve_(prob, 3, timestepping=False)
+        return [np.asarray(gpu_fields(G, prob)[f]) for f in FIELDS]
+
+    ref = run(0)
+    for cap in (None, 3):
+        for a, b in zip(run(cap), ref):
+            assert np.array_equal(a, b, equal_nan=True)
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32split"])
 @pytest.mark.parametrize("case", ["dam2d", "dam2d_allphys", "dam3d_allphys"])
 def test_ptype_values_act_by_class(G, prec, case):
     """The pair terms ask of a particle type only whether it is > 0, > 1, < 0 or
