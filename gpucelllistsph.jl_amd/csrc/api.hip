@@ -378,7 +378,8 @@ struct sph_s {
     GCL_HIP(hipStreamSynchronize(stream));
     if (ne_buf) GCL_HIP(hipFree(ne_buf));
     ne_buf = nullptr;
-    GCL_HIP(hipMalloc(&ne_buf, sizeof(uint64_t) * size_t(std::max<int64_t>(need, 1)) * size_t(n)));
+    // a row more than is filled: the reader asks for the entry after the last (Stored)
+    GCL_HIP(hipMalloc(&ne_buf, sizeof(uint64_t) * size_t(need + 1) * size_t(n)));
     necap = int(need);
     B.NE = ne_buf;
     B.necap = necap;
@@ -851,14 +852,10 @@ void run_steps(sph_s* const* P, unsigned count, LaunchSet& L, hipStream_t st, in
   // timing, else the fastest measured on the dam-break scenes per dimension
   // and precision until it has been tuned.
   int pv[2];
-  if (std::is_same<R, float>::value) {
-    pv[0] = 2;  // prefetch, >= 3 waves per SIMD
-    pv[1] = 0;  // prefetch, compiler's occupancy
-  } else if (D == 2) {
-    pv[0] = pv[1] = 0;
-  } else {  // no prefetch, 128 threads: 284 + 345 us for 191,232 particles, 347 + 410 prefetching
-    pv[0] = pv[1] = 5;
-  }
+  // 3D: prefetch, three waves per SIMD (191,232 particles FP64 299 + 320 us,
+  // 303 + 376 without prefetch); 2D: prefetch
+  pv[0] = D == 3 || std::is_same<R, float>::value ? 2 : 0;
+  pv[1] = D == 3 ? 2 : 0;
   bool forced = false;
   if (const char* env = std::getenv("GCLSPH_PASS_VARIANT")) {
     int v1 = -1, v2 = -1;
@@ -955,7 +952,7 @@ void run_steps(sph_s* const* P, unsigned count, LaunchSet& L, hipStream_t st, in
     int k = 0;
     for (; k < warm; ++k) launch_step(cspm_at(k + 1), pv[0], pv[1], nullptr);
     for (int v = 0; v < nocap; ++v) {
-      // FP64 held to five waves per SIMD spills and is 1.3 to 5 times slower
+      // in FP64 3 is 1 (pass1_cg)
       if (std::is_same<R, double>::value && v % kPassCodegen == 3) continue;
       time_step(k, v, v);
     }

@@ -115,7 +115,7 @@ struct SphBufs {
   int nblk;
   // neighbour-list membership of the last rebuild (written with the reorder): entry e of
   // particle a at NE[e * n + a] = (window base << 32) | member bits; NC[a]
-  // entries, or -1 when more than necap were needed
+  // entries, or -1 when more than necap were needed; NE has necap + 1 rows
   uint64_t* NE;
   int32_t* NC;
   int necap;

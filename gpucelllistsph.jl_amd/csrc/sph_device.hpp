@@ -8,6 +8,8 @@
 #include "blockscan.hpp"
 #include "sph.hpp"
 
+#define GCLSPH_INLINE __attribute__((always_inline))  // of a lambda
+
 namespace gclsph {
 
 // ---------------------------------------------------------------- math helpers
@@ -766,63 +768,36 @@ __device__ __forceinline__ FrameK3 particle_k(const SphBufs<R>& B, const SphCons
 
 // Neighbour-list partners b of particle a in a fixed order (stencil rows in
 // order, ascending sorted index inside a row; in 3D each row visited cell by
-// cell, which is the same order).  nc >= 0: the nc stored entries of the
-// membership store, read one ahead so the next load overlaps the current
-// window's pair bodies.  nc < 0: the windows are computed here from the
-// membership positions XM.  Each lane runs its own sequence, so all lanes of a
-// wave execute the (long) pair body together.  Fr (3D only): the iterator also
-// keeps the current window's separation constants from the particle's FrameK3.
-template <int D, typename R, bool Fr = false>
-struct Partners {
-  static_assert(!Fr || cell_windows<D, R>(), "cell frames come with cell windows");
-  const SphBufs<R>& B;
-  const CellGeom& G;
-  const double* const xm0;  // membership positions, held by value
-  const double* const xm1;
-  const double* const xm2;
-  const double dist2;
-  const int64_t a;
-  const int nc;
-  const uint64_t* pe;
-  uint64_t nxt;
-  int e = 1, k = -1;
-  int32_t w0 = 0, re = 0, cb = 0;
-  uint32_t c = 0;
-  FrameK3 kt;        // Fr: the particle's separation constants
-  float wk[3];       // Fr: constants of the current window
-  int j = 3;         // 3D scan (nc < 0): cell of row k, 0..2 for ox = -1..1
+// cell, which is the same order), a window of candidates with its member bits at
+// a time: from the membership store (Stored), or, for a particle that needs more
+// entries than the store holds (nc < 0), computed from the membership positions
+// (Scanned).  Each lane runs its own sequence, so all lanes of a wave execute the
+// (long) pair body together.  The two are separate loops: one that could do both
+// carried the scan's state through every trip (XSPH in 3D FP32-split: 86
+// registers instead of 67), and its store path waited for the entry that it had
+// just asked for.  A call of 31,962 particles in 3D FP64 with all corrections:
+// 3.27 -> 3.09 ms.
+// Fr (3D only): also the current window's separation constants, from the
+// particle's FrameK3.
+template <bool Fr>
+struct Window {
+  uint32_t c = 0;  // members not yet taken; bit t: candidate cb + t
+  int32_t cb = 0;
+  FrameK3 kt;   // Fr: the particle's separation constants
+  float wk[3];  // Fr: constants of the current window
 
-  __device__ __forceinline__ Partners(const SphBufs<R>& B_, int64_t a_, int nc_, const CellGeom& G_,
-                                      const double* const* XM_, double dist2_, const FrameK3* kt_ = nullptr)
-      : B(B_),
-        G(G_),
-        xm0(XM_[0]),
-        xm1(XM_[1]),
-        xm2(XM_[2]),
-        dist2(dist2_),
-        a(a_),
-        nc(nc_),
-        pe(B_.NE + a_),
-        nxt(nc_ > 0 ? *pe : 0ull) {
-    if constexpr (Fr) kt = *kt_;
-    fill();
-  }
-
-  // Another partner is waiting (the iterator always stands on the next one).
+  // Another partner is waiting in the window.
   __device__ __forceinline__ bool has() const { return c != 0; }
 
-  // The waiting partner; moves on to the one after it.
+  // The window's next partner.
   __device__ __forceinline__ int32_t take() {
     const int32_t b = cb + __builtin_ctz(c);
     c &= c - 1;
-    if (c == 0) fill();
     return b;
   }
-  // As take(), with the separation constants of the partner's window.
+  // As take(), with the separation constants of the window.
   __device__ __forceinline__ int32_t take(Win3& w) {
-    w.k[0] = wk[0];
-    w.k[1] = wk[1];
-    w.k[2] = wk[2];
+    constants(w);
     return take();
   }
   __device__ __forceinline__ int32_t take(NoWin&) { return take(); }
@@ -832,23 +807,22 @@ struct Partners {
   template <typename W>
   __device__ __forceinline__ int32_t take_quad(bool& on, const int32_t none, W& w) {
     const uint32_t i = threadIdx.x & 3u;
-    const bool had = c != 0;
     uint32_t m = c;
     m = i > 0 ? m & (m - 1) : m;
     m = i > 1 ? m & (m - 1) : m;
     m = i > 2 ? m & (m - 1) : m;
     on = m != 0;
     const int32_t b = on ? cb + __builtin_ctz(m) : none;
-    if constexpr (Fr) {
-      w.k[0] = wk[0];
-      w.k[1] = wk[1];
-      w.k[2] = wk[2];
-    }
+    if constexpr (Fr) constants(w);
     c = quad_lane<3>(m & (m - 1));
-    if (had && c == 0) fill();
     return b;
   }
 
+  __device__ __forceinline__ void constants(Win3& w) const {
+    w.k[0] = wk[0];
+    w.k[1] = wk[1];
+    w.k[2] = wk[2];
+  }
   __device__ __forceinline__ void set_window(uint32_t code) {
     if constexpr (Fr) {
       // base-3 digits of code < 27: q / 3 = (q · 11) >> 5 for q < 27
@@ -858,30 +832,76 @@ struct Partners {
       for (int d = 0; d < 3; ++d) wk[d] = fmaf(float(o1[d]), -kt.cf[d], kt.km[d]);
     }
   }
+};
 
-  // c == 0: loads the next window that has members (c stays 0 at the end).
-  __device__ __forceinline__ void fill() {
-    if (nc >= 0) {
-      if (nxt == 0) return;  // stored entries always have member bits
+// The halves of a stored entry, in registers of their own: shared with the
+// entry's, they would leave the load of the next one no place but a second pair,
+// copied (and so waited for) at once.
+__device__ __forceinline__ void split_entry(uint64_t e, uint32_t& bits, uint32_t& base) {
+  asm("v_mov_b32 %0, %1" : "=&v"(bits) : "v"(uint32_t(e)));
+  asm("v_mov_b32 %0, %1" : "=&v"(base) : "v"(uint32_t(e >> 32)));
+}
+
+// The nc stored entries, read one ahead: the entry asked for when a window
+// begins is first needed when it is empty.  The load has no condition (the store
+// has a row more than entries may fill, and what the last load reads is not
+// used), so its result needs no second register and no wait at the load.
+template <int D, typename R, bool Fr = false>
+struct Stored : Window<Fr> {
+  static_assert(!Fr || cell_windows<D, R>(), "cell frames come with cell windows");
+  const int64_t n;
+  const uint64_t* pe;
+  uint64_t nxt;
+  int left;  // entries not yet begun
+
+  __device__ __forceinline__ Stored(const SphBufs<R>& B, int64_t a, int nc, const FrameK3* kt_ = nullptr)
+      : n(B.n), pe(B.NE + a), nxt(*pe), left(nc) {
+    if constexpr (Fr) this->kt = *kt_;
+  }
+  // An empty window gives way to the next one (entries have member bits).
+  __device__ __forceinline__ void refill() {
+    if (this->c == 0 && left > 0) {
+      uint32_t bits, base;
+      split_entry(nxt, bits, base);
       if constexpr (cell_windows<D, R>()) {
-        c = uint32_t(nxt) & kWinMask3;
-        set_window(uint32_t(nxt) >> kWin3);
-      } else {
-        c = uint32_t(nxt);
+        this->set_window(bits >> kWin3);
+        bits &= kWinMask3;
       }
-      cb = int32_t(nxt >> 32);
-      pe += B.n;
-      nxt = e < nc ? *pe : 0ull;
-      ++e;
-      return;
+      this->c = bits;
+      this->cb = int32_t(base);
+      --left;
+      pe += n;
+      nxt = *pe;
     }
+  }
+};
+
+template <int D, typename R, bool Fr = false>
+struct Scanned : Window<Fr> {
+  const SphBufs<R>& B;
+  const CellGeom& G;
+  const double* const xm0;  // membership positions, held by value
+  const double* const xm1;
+  const double* const xm2;
+  const double dist2;
+  const int64_t a;
+  int k = -1;
+  int32_t w0 = 0, re = 0;
+  int j = 3;  // 3D: cell of row k, 0..2 for ox = -1..1
+
+  __device__ __forceinline__ Scanned(const SphBufs<R>& B_, int64_t a_, const CellGeom& G_, const double* const* XM_,
+                                     double dist2_, const FrameK3* kt_ = nullptr)
+      : B(B_), G(G_), xm0(XM_[0]), xm1(XM_[1]), xm2(XM_[2]), dist2(dist2_), a(a_) {
+    if constexpr (Fr) this->kt = *kt_;
+  }
+  __device__ __forceinline__ void refill() {
     if constexpr (cell_windows<D, R>()) {
       // stencil cell by cell, windows of kWin3 candidates inside a cell
-      while (c == 0) {
+      while (this->c == 0) {
         if (w0 >= re) {
           if (++j > 2) {
             j = 0;
-            if (++k >= Rows<3>::N) return;
+            if (++k >= Rows<3>::N) break;
           }
           int64_t cx, cy, cz;
           cell_xyz<3>(G, B.skey[a], cx, cy, cz);
@@ -890,24 +910,24 @@ struct Partners {
           const int64_t cell = x + G.grid[0] * (y + G.grid[1] * z);
           w0 = in ? B.start[cell] : 0;
           re = in ? B.start[cell + 1] : 0;
-          set_window(win_code3(j - 1, (k % 3) - 1, (k / 3) - 1));
+          this->set_window(win_code3(j - 1, (k % 3) - 1, (k / 3) - 1));
           continue;
         }
         const int32_t hi = re < w0 + kWin3 ? re : w0 + kWin3;
-        c = window_bits_lean<3>(xm0, xm1, xm2, xm0[a], xm1[a], xm2[a], a, w0, hi, dist2);
-        cb = w0;
+        this->c = window_bits_lean<3>(xm0, xm1, xm2, xm0[a], xm1[a], xm2[a], a, w0, hi, dist2);
+        this->cb = w0;
         w0 = hi;
       }
     } else {
-      while (c == 0) {
+      while (this->c == 0) {
         if (w0 >= re) {
-          if (++k >= Rows<D>::N) return;
+          if (++k >= Rows<D>::N) break;
           row_range<D>(G, B.start, B.skey[a], k, w0, re);
           continue;
         }
         const int32_t hi = re < w0 + 32 ? re : w0 + 32;
-        c = window_bits_lean<D>(xm0, xm1, xm2, xm0[a], xm1[a], D == 3 ? xm2[a] : 0.0, a, w0, hi, dist2);
-        cb = w0;
+        this->c = window_bits_lean<D>(xm0, xm1, xm2, xm0[a], xm1[a], D == 3 ? xm2[a] : 0.0, a, w0, hi, dist2);
+        this->cb = w0;
         w0 = hi;
       }
     }
@@ -921,12 +941,16 @@ struct Partners {
 template <int D, typename R, typename F>
 __device__ __forceinline__ void for_each_partner(const SphBufs<R>& B, int64_t a, int nc, const CellGeom& G,
                                                  const double* const* XM, double dist2, F&& body) {
-  Partners<D, R> it(B, a, nc, G, XM, dist2);
-  for (;;) {
-    const bool m = it.has();
-    if (!__any(m)) break;
-    if (m) body(it.take());
-  }
+  const auto loop = [&](auto&& it) GCLSPH_INLINE {
+    for (;;) {
+      it.refill();
+      const bool m = it.has();
+      if (!__any(m)) break;
+      if (m) body(it.take());
+    }
+  };
+  loop(Stored<D, R>(B, a, nc));
+  if (nc < 0) loop(Scanned<D, R>(B, a, G, XM, dist2));
 }
 
 // As for_each_partner, with the partner data split off: fetch(b) loads what
@@ -950,9 +974,8 @@ __device__ __forceinline__ Sums<N, R> sum_partners(const SphBufs<R>& B, int64_t 
                                                    const FrameK3* kt = nullptr) {
   constexpr bool Fr = Frames && D == 3 && std::is_same<R, float>::value;
   using W = typename std::conditional<Fr, Win3, NoWin>::type;
-  Partners<D, R, Fr> it(B, a, nc, G, XM, dist2, kt);
   Sums<N, R> sum;
-  auto run = [&](const bool on, const auto& f, const W& w) {
+  auto run = [&](const bool on, const auto& f, const W& w) GCLSPH_INLINE {
     if constexpr (Quad) {
       Terms<N, R> t;
       if (on) {
@@ -967,47 +990,58 @@ __device__ __forceinline__ Sums<N, R> sum_partners(const SphBufs<R>& B, int64_t 
       sum.add(t);
     }
   };
-  // this lane's next partner; `none` (a valid index) and on = false without one
-  auto take = [&](bool& on, const int32_t none, W& w) {
-    if constexpr (Quad) {
-      return it.take_quad(on, none, w);
-    } else {
-      on = it.has();
-      return on ? it.take(w) : none;
+  auto one_by_one = [&](auto&& it) GCLSPH_INLINE {
+    for (;;) {
+      it.refill();
+      if (!__any(it.has())) break;
+      W w{};
+      if constexpr (Quad) {
+        bool on;
+        const int32_t b = it.take_quad(on, int32_t(a), w);
+        run(on, fetch(b), w);
+      } else if (it.has()) {
+        run(true, fetch(it.take(w)), w);
+      }
     }
   };
   if constexpr (!Pipe) {
-    while (__any(it.has())) {
-      W w{};
-      bool on;
-      const int32_t b = take(on, int32_t(a), w);
+    one_by_one(Stored<D, R, Fr>(B, a, nc, kt));
+  } else {
+    // two partners in flight, alternating between two sets of registers; a lane
+    // without a next partner fetches a valid address again and skips the body
+    Stored<D, R, Fr> it(B, a, nc, kt);
+    // this lane's next partner; `none` (a valid index) and on = false without one
+    auto take = [&](bool& on, const int32_t none, W& w) GCLSPH_INLINE {
       if constexpr (Quad) {
-        run(on, fetch(b), w);
-      } else if (on) {
-        run(true, fetch(b), w);
+        return it.take_quad(on, none, w);
+      } else {
+        on = it.has();
+        return on ? it.take(w) : none;
+      }
+    };
+    it.refill();
+    if (__any(it.has())) {
+      W w0{}, w1{};
+      bool m0, m1;
+      int32_t b0 = take(m0, int32_t(a), w0);
+      auto f0 = fetch(b0);
+      for (;;) {
+        it.refill();
+        bool more = __any(it.has());
+        const int32_t b1 = take(m1, b0, w1);
+        auto f1 = fetch(b1);
+        run(m0, f0, w0);
+        if (!more) break;
+        it.refill();
+        more = __any(it.has());
+        b0 = take(m0, b1, w0);
+        f0 = fetch(b0);
+        run(m1, f1, w1);
+        if (!more) break;
       }
     }
-    return sum;
   }
-  // two partners in flight, alternating between two sets of registers; a lane
-  // without a next partner fetches a valid address again and skips the body
-  if (!__any(it.has())) return sum;
-  W w0{}, w1{};
-  bool m0, m1;
-  int32_t b0 = take(m0, int32_t(a), w0);
-  auto f0 = fetch(b0);
-  for (;;) {
-    bool more = __any(it.has());
-    const int32_t b1 = take(m1, b0, w1);
-    auto f1 = fetch(b1);
-    run(m0, f0, w0);
-    if (!more) break;
-    more = __any(it.has());
-    b0 = take(m0, b1, w0);
-    f0 = fetch(b0);
-    run(m1, f1, w1);
-    if (!more) break;
-  }
+  if (nc < 0) one_by_one(Scanned<D, R, Fr>(B, a, G, XM, dist2, kt));
   return sum;
 }
 

@@ -665,8 +665,11 @@ __global__ void k_xsph_rec(SS ss) {
 }
 
 // xsphcorr! + update_xsphcorr! (src/gpukernels_sph.jl:1757-1838): W at xⁿ.
+// At most four waves per SIMD: with the seven that its registers allow, their
+// partners' records displace each other in the CU's L1 (883,376 particles in 3D
+// FP32-split: 565 us at seven, 530 at five, 496 at four).
 template <int D, typename R, bool Quad, typename SS>
-__global__ __launch_bounds__(256) void k_xsph(SS ss) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 4))) void k_xsph(SS ss) {
 #pragma clang fp contract(off)
   GCLSPH_SCENE_PAIR(ss, kBlock, Quad);
   if (!F.xsph_on) return;

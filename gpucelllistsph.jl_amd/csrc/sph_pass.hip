@@ -36,12 +36,14 @@ namespace gclsph {
 // launch shape (so their results are bit-identical: one thread computes one
 // particle whatever the block): Pipe fetches the next partner's data before the
 // current pair body (two register sets), W asks the compiler for at least W
-// waves per SIMD (fewer registers), BS is the block size.  The step driver
+// waves per SIMD (fewer registers; W = 3 in 3D for exactly three, which in
+// FP32-split keeps pass 2's partner records in L1: 848 us for 883,376
+// particles, 930 with four), BS is the block size.  The step driver
 // picks one per pass by timing them on live steps.
 //
 // ---- pass 1 ---------------------------------------------------------------
 template <int D, typename R, typename SS, bool Pipe, int W, int BS, bool G7, bool Quad>
-__global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W))) void k_pass1(SS ss) {
+__global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W, D == 3 && W == 3 ? 3 : 8))) void k_pass1(SS ss) {
 #pragma clang fp contract(off)
   GCLSPH_SCENE_PAIR(ss, BS, Quad);
   const StepCtl* ctl = B.ctl;
@@ -196,7 +198,7 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W))) void k_
 
 // ---- pass 2 + symplectic update ------------------------------------------
 template <int D, typename R, typename SS, bool Pipe, int W, int BS, bool G7, bool Quad>
-__global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W))) void k_pass2(SS ss) {
+__global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W, D == 3 && W == 3 ? 3 : 8))) void k_pass2(SS ss) {
 #pragma clang fp contract(off)
   GCLSPH_SCENE_PAIR(ss, BS, Quad);
   StepCtl* ctl = B.ctl;
@@ -442,13 +444,14 @@ size_t cap_lds(int bs) {
   return blocks * lds <= cu && lds <= blk ? lds : 0;
 }
 // code generation cg: 0 pipelined; 1 not pipelined; 2 pipelined, >= 3
-// waves/SIMD; 3 not pipelined, >= 5 waves/SIMD
+// waves/SIMD (3D: exactly 3); 3 (FP32-split) not pipelined, >= 5 waves/SIMD,
+// which makes FP64 spill: there it is 1
 template <int D, typename R, int BS>
 void pass1_cg(const LaunchSet& L, hipStream_t s, int cg, size_t lds) {
   switch (cg) {
     case 1: pass1_as<D, R, false, 1, BS>(L, s, lds); break;
     case 2: pass1_as<D, R, true, 3, BS>(L, s, lds); break;
-    case 3: pass1_as<D, R, false, 5, BS>(L, s, lds); break;
+    case 3: pass1_as<D, R, false, sizeof(R) == 8 ? 1 : 5, BS>(L, s, lds); break;
     default: pass1_as<D, R, true, 1, BS>(L, s, lds); break;
   }
 }
@@ -457,7 +460,7 @@ void pass2_cg(const LaunchSet& L, hipStream_t s, int cg, size_t lds) {
   switch (cg) {
     case 1: pass2_as<D, R, false, 1, BS>(L, s, lds); break;
     case 2: pass2_as<D, R, true, 3, BS>(L, s, lds); break;
-    case 3: pass2_as<D, R, false, 5, BS>(L, s, lds); break;
+    case 3: pass2_as<D, R, false, sizeof(R) == 8 ? 1 : 5, BS>(L, s, lds); break;
     default: pass2_as<D, R, true, 1, BS>(L, s, lds); break;
   }
 }
