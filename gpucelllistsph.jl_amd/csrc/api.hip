@@ -853,9 +853,8 @@ void run_steps(sph_s* const* P, unsigned count, LaunchSet& L, hipStream_t st, in
   // and precision until it has been tuned.
   int pv[2];
   // 3D: prefetch, three waves per SIMD (191,232 particles FP64 299 + 320 us,
-  // 303 + 376 without prefetch); 2D: prefetch
-  pv[0] = D == 3 || std::is_same<R, float>::value ? 2 : 0;
-  pv[1] = D == 3 ? 2 : 0;
+  // 303 + 376 without prefetch); 2D has block sizes only
+  pv[0] = pv[1] = D == 3 ? 2 : 0;
   bool forced = false;
   if (const char* env = std::getenv("GCLSPH_PASS_VARIANT")) {
     int v1 = -1, v2 = -1;
@@ -952,13 +951,14 @@ void run_steps(sph_s* const* P, unsigned count, LaunchSet& L, hipStream_t st, in
     int k = 0;
     for (; k < warm; ++k) launch_step(cspm_at(k + 1), pv[0], pv[1], nullptr);
     for (int v = 0; v < nocap; ++v) {
-      // in FP64 3 is 1 (pass1_cg)
-      if (std::is_same<R, double>::value && v % kPassCodegen == 3) continue;
+      // those that differ (pass1_cg): the block sizes in 2D, no 3 in 3D FP64
+      const int cg = v % kPassCodegen;
+      if (D == 2 ? cg != 0 : std::is_same<R, double>::value && cg == 3) continue;
       time_step(k, v, v);
     }
     read_stage();
     const int r0[2] = {ranked(0, 0), ranked(1, 0)}, r1[2] = {ranked(0, 1), ranked(1, 1)};
-    time_step(k, r0[0] % nocap + nocap, r0[1] % nocap + nocap);
+    if (D == 3) time_step(k, r0[0] % nocap + nocap, r0[1] % nocap + nocap);
     time_step(k, r0[0], r0[1]);
     time_step(k, r1[0], r1[1]);
     read_stage();

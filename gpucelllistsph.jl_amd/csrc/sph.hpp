@@ -331,7 +331,8 @@ void launch_commit_rebuild(const LaunchSet& L, hipStream_t s);
 // generation and launch shape (same results): variant = cg + 4·bs + 12·oc,
 // with cg in [0, 4) the prefetch / occupancy-target choice, bs in [0, 3) the
 // block size (256, 128, 512 threads) and oc in [0, 2) an occupancy cap (1: at
-// most kPassCapWaves waves per SIMD, by launching with unused LDS).
+// most kPassCapWaves waves per SIMD, by launching with unused LDS); in 2D the
+// block size alone tells variants apart.
 constexpr int kPassCodegen = 4;
 constexpr int kPassBlockSizes = 3;
 constexpr int kPassCaps = 2;

@@ -613,6 +613,90 @@ __device__ __forceinline__ void st_rec(void* base, int64_t a, const T& r, int64_
   for (int i = 0; i < kW; ++i) p[apart ? i * n : i] = w[i];
 }
 
+// ---- 2D partner records staged in LDS
+// The pair passes with one lane per particle read a partner's record ~36 times
+// for each particle, at 64 places per load, and were bound by the CU's L1 (FP64:
+// an access each cycle; FP32-split: 0.93, with the VALU at 0.9).  A block's
+// particles are consecutive cells, so their partners lie in three ranges of
+// sorted indices (~3.4 BS records), which the block copies to LDS once, by
+// coalesced loads.  Two of a record's 16-byte words are staged: all of an
+// FP32-split one, half of an FP64 one; the other FP64 words stay with the L1.
+// Three words staged left LDS for three waves per SIMD instead of four (1.02 M
+// particles FP64: 52 KiB a block).  FP32-split passes are then bound by VALU
+// issue (1.0 per CU and cycle).  3.95 M particles FP32-split: passes 414 + 481
+// -> 380 + 433 us; 1.02 M FP64: 189 + 259 -> 180 + 230 us.
+constexpr int kStagedWords = 2;
+// Records staged at most.  The rows above and below a block's cells hold up to
+// 4/3 of its particles where the cell size is 3.6 lattice spacings, and each row
+// the cells beside its ends.  Short of this many (3 BS + 160) a half of the
+// blocks of a lattice fell back to global memory.
+template <int BS>
+constexpr int kStageCap = 15 * BS / 4 + 128;
+
+// Where the records of the block's stencil rows are staged: record b of row r at
+// b + d[r].  The row of a window is taken to be the last one that begins at or
+// before it: where ranges overlap, that one reaches at least as far.
+struct RowMap {
+  int32_t s1, s2;
+  int32_t d0, d1, d2;
+  __device__ __forceinline__ int32_t at(int32_t b) const {
+    const int32_t v0 = d0, v1 = d1, v2 = d2;  // values: a choice between members would keep them in memory
+    int32_t d = b >= s1 ? v1 : v0;
+    d = b >= s2 ? v2 : d;
+    return d;
+  }
+};
+
+// Stages the first Words words of the records of the three stencil rows around
+// the block's particles [a0, a0 + BS): row r is one range of sorted indices,
+// from the cell before the first particle's to the one after the last's (more
+// than the particles need where the block goes over a row end; in a narrow grid
+// the ranges overlap).  False when they don't fit or some particle has no stored
+// membership (nc < 0): the block then reads global memory.  Called by the whole
+// block.
+template <int BS, int Words, typename R>
+__device__ __forceinline__ bool stage_rows(uint4 (*lds)[kStageCap<BS>], const void* base, const SphBufs<R>& B,
+                                           const CellGeom& G, int64_t a0, int nc, RowMap& map) {
+  const int64_t last = (a0 + BS < B.n ? a0 + BS : B.n) - 1, gx = G.grid[0], nce = G.ncells();
+  const int64_t c0 = B.skey[a0], c1 = B.skey[last];
+  int32_t s[3], e[3];
+#pragma unroll
+  for (int r = 0; r < 3; ++r) {
+    const int64_t lo = c0 + gx * (r - 1) - 1, hi = c1 + gx * (r - 1) + 2;
+    s[r] = __builtin_amdgcn_readfirstlane(B.start[lo < 0 ? 0 : (lo > nce ? nce : lo)]);
+    e[r] = __builtin_amdgcn_readfirstlane(B.start[hi < 0 ? 0 : (hi > nce ? nce : hi)]);
+  }
+  const int32_t n0 = e[0] - s[0], n1 = n0 + (e[1] - s[1]), n2 = n1 + (e[2] - s[2]);
+  if (!__syncthreads_and(n2 <= kStageCap<BS> && nc >= 0)) return false;
+  map = {s[1], s[2], -s[0], n0 - s[1], n1 - s[2]};
+  const uint4* p = reinterpret_cast<const uint4*>(base);
+  for (int32_t i = threadIdx.x; i < n2; i += BS) {
+    const int32_t b = i - (i < n0 ? map.d0 : i < n1 ? map.d1 : map.d2);
+#pragma unroll
+    for (int w = 0; w < Words; ++w) lds[w][i] = p[w * B.n + b];
+  }
+  __syncthreads();
+  return true;
+}
+
+// Record b, staged at place i; its words beyond Words come from global memory.
+template <typename T, int Words, int Cap>
+__device__ __forceinline__ T ld_staged(const uint4 (*lds)[Cap], int32_t i, const void* base, uint32_t b,
+                                       int64_t n) {
+  constexpr int kW = int(sizeof(T) / 16);
+  uint4 w[kW];
+#pragma unroll
+  for (int k = 0; k < Words; ++k) w[k] = lds[k][i];
+  if constexpr (Words < kW) {
+    const uint4* p = reinterpret_cast<const uint4*>(base) + b;
+#pragma unroll
+    for (int k = Words; k < kW; ++k) w[k] = p[k * n];
+  }
+  T r;
+  __builtin_memcpy(&r, w, sizeof(T));
+  return r;
+}
+
 // ---- 3D cell frames and per-cell membership windows
 // 3D membership entries hold one window of at most kWin3 candidates inside
 // one stencil cell: the member bits in the low kWin3 bits of the low word and
@@ -1043,6 +1127,39 @@ __device__ __forceinline__ Sums<N, R> sum_partners(const SphBufs<R>& B, int64_t 
   }
   if (nc < 0) one_by_one(Scanned<D, R, Fr>(B, a, G, XM, dist2, kt));
   return sum;
+}
+
+// The same over records staged in LDS (2D, one lane a particle, stored windows
+// only): fetch(b, i) reads record b, staged at place i.
+template <int N, typename R, typename Fetch, typename F>
+__device__ __forceinline__ Sums<N, R> sum_staged(const SphBufs<R>& B, int64_t a, int nc, const RowMap& map,
+                                                 Fetch&& fetch, F&& body) {
+  Sums<N, R> sum;
+  const uint64_t* pe = B.NE + a;
+  uint64_t nxt = *pe;
+  int left = nc;
+  uint32_t c = 0;
+  int32_t cb = 0, at = 0;
+  for (;;) {
+    if (c == 0 && left > 0) {
+      uint32_t base;
+      split_entry(nxt, c, base);
+      cb = int32_t(base);
+      at = cb + map.at(cb);
+      --left;
+      pe += B.n;
+      nxt = *pe;
+    }
+    if (!__any(c != 0)) return sum;
+    if (c != 0) {
+      const int32_t k = __builtin_ctz(c);
+      const auto f = fetch(cb + k, at + k);
+      c &= c - 1;
+      Terms<N, R> t;
+      body(f, t);
+      sum.add(t);
+    }
+  }
 }
 
 // ---------------------------------------------------------------- the pair

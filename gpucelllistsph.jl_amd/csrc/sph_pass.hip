@@ -21,9 +21,9 @@
 // operation order with FMA contraction off, so they see the same values as the
 // reference would.  The pair terms are the reference's to a few ulp: their ten
 // divisions, square roots and powfancy7th are the arithmetic of sph_device.hpp
-// (~85 VALU instructions per pair, ~330 as written; the passes are bound by
-// VALU issue).  1.02 M particles in 2D: a step 0.77 -> 0.50 ms; 191 k in 3D:
-// 1.45x per call.
+// (~85 VALU instructions per pair, ~330 as written, when VALU issue bound the
+// passes).  1.02 M particles in 2D: a step 0.77 -> 0.50 ms; 191 k in 3D: 1.45x
+// per call.
 // R = float: the FP32-split path (density stored as ρ-ρ0, FP32 pair terms
 // summed in FP64, Float64 positions and Δt).
 #include <atomic>
@@ -36,20 +36,35 @@ namespace gclsph {
 // launch shape (so their results are bit-identical: one thread computes one
 // particle whatever the block): Pipe fetches the next partner's data before the
 // current pair body (two register sets), W asks the compiler for at least W
-// waves per SIMD (fewer registers; W = 3 in 3D for exactly three, which in
+// waves per SIMD (fewer registers; W = 3 for exactly three, which in 3D
 // FP32-split keeps pass 2's partner records in L1: 848 us for 883,376
 // particles, 930 with four), BS is the block size.  The step driver
 // picks one per pass by timing them on live steps.
 //
 // ---- pass 1 ---------------------------------------------------------------
 template <int D, typename R, typename SS, bool Pipe, int W, int BS, bool G7, bool Quad>
-__global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W, D == 3 && W == 3 ? 3 : 8))) void k_pass1(SS ss) {
+__global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W, W == 3 ? 3 : 8))) void k_pass1(SS ss) {
 #pragma clang fp contract(off)
   GCLSPH_SCENE_PAIR(ss, BS, Quad);
   const StepCtl* ctl = B.ctl;
   const int p = cur_parity(ctl), pp = cur_pparity(ctl), rebuilt = ctl->rebuild;
   const double dt = ctl->dt;
-  if (a >= B.n) return;
+  constexpr bool kStage = D == 2 && !Quad;  // a quad's block has 64 particles: as much to stage for a quarter of the use
+  bool staged = false;
+  RowMap map{};
+  int nc = 0;
+  using Nb = typename Records<D, R>::N;
+  __shared__ uint4 lds[kStage ? kStagedWords : 1][kStage ? kStageCap<BS> : 1];
+  if constexpr (kStage) {
+    const int64_t a0 = int64_t(m.y) * BS;
+    if (a0 >= B.n) return;  // whole block
+    nc = a < B.n ? B.NC[a] : 0;
+    staged = stage_rows<BS, kStagedWords>(lds, B.PRN, B, G, a0, nc, map);
+    if (a >= B.n) return;
+  } else {
+    if (a >= B.n) return;
+    nc = B.NC[a];
+  }
   const double* X[3] = {B.X[p][0], B.X[p][1], B.X[p][D == 3 ? 2 : 1]};
   const R* V[3] = {B.V[p][0], B.V[p][1], B.V[p][D == 3 ? 2 : 1]};
   const R* RHO = B.RHO[p];
@@ -68,12 +83,13 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W, D == 3 &&
   const int32_t pta = PT[a];
   constexpr int kDrho = D;  // sums: D accelerations, ∂ρ/∂t
 
-  const int nc = B.NC[a];
+  auto fetch = [&](const int32_t b, const auto... at) GCLSPH_INLINE {
+    if constexpr (sizeof...(at) > 0) return ld_staged<Nb, kStagedWords>(lds, at..., B.PRN, b, B.n);
+    else return ld_rec<Nb>(B.PRN, b, B.n);
+  };
   if constexpr (std::is_same<R, double>::value) {
     const Own<R> own = own_of<R>(sa, B.PN[a], pta, C);
-    using Nb = PartnerN64<D>;
-    auto fetch = [&](const int32_t b) { return ld_rec<Nb>(B.PRN, b, B.n); };
-    const auto sum = sum_partners<Pipe, Quad, D, D + 1, R>(B, a, nc, G, XM, C.dist2, fetch, [&](const Nb& q, auto& t) {
+    auto pair = [&](const Nb& q, auto& t) GCLSPH_INLINE {
       double dx[3], dv[3];
 #pragma unroll
       for (int d = 0; d < D; ++d) {
@@ -82,7 +98,14 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W, D == 3 &&
       }
       const double r2 = dist2_of<D>(dx);
       pair_terms<D, G7, true>(C, F, own, q, q.rho, q.pt, q.P, dx, dv, dx, r2, root_of(r2), 0, t);
-    });
+    };
+    Sums<D + 1, R> sum;
+    if constexpr (kStage) {
+      if (staged) sum = sum_staged<D + 1, R>(B, a, nc, map, fetch, pair);
+      else sum = sum_partners<Pipe, Quad, D, D + 1, R>(B, a, nc, G, XM, C.dist2, fetch, pair);
+    } else {
+      sum = sum_partners<Pipe, Quad, D, D + 1, R>(B, a, nc, G, XM, C.dist2, fetch, pair);
+    }
     // ∂v∂t_addgrav!, then the half-step updates (:270-274)
     double av[3];
 #pragma unroll
@@ -132,11 +155,8 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W, D == 3 &&
   } else {
     // ---------------- FP32-split
     const Own<R> own = own_of<R>(sa, B.PN[a], pta, C);
-    using Nb = PartnerN<D>;
-    auto fetch = [&](const int32_t b) { return ld_rec<Nb>(B.PRN, b, B.n); };
     const FrameK3 kt = particle_k<D, R>(B, C, G, a, xa);
-    const auto sum = sum_partners<Pipe, Quad, D, D + 1, R, true>(B, a, nc, G, XM, C.dist2, fetch,
-                                                                 [&](const Nb& q, auto& t, const auto&... win) {
+    auto pair = [&](const Nb& q, auto& t, const auto&... win) GCLSPH_INLINE {
       float dx[3], dv[3];
 #pragma unroll
       for (int d = 0; d < D; ++d) {
@@ -145,7 +165,14 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W, D == 3 &&
       }
       const float r2 = dist2_of<D>(dx);
       pair_terms<D, G7, true>(C, F, own, q, q.rho, rec_pt(q), rec_P(q, C), dx, dv, dx, r2, root_of(r2), 0, t);
-    }, &kt);
+    };
+    Sums<D + 1, R> sum;
+    if constexpr (kStage) {
+      if (staged) sum = sum_staged<D + 1, R>(B, a, nc, map, fetch, pair);
+      else sum = sum_partners<Pipe, Quad, D, D + 1, R, true>(B, a, nc, G, XM, C.dist2, fetch, pair, &kt);
+    } else {
+      sum = sum_partners<Pipe, Quad, D, D + 1, R, true>(B, a, nc, G, XM, C.dist2, fetch, pair, &kt);
+    }
     float av[3];
 #pragma unroll
     for (int d = 0; d < D; ++d) av[d] = sum.get(d);
@@ -198,7 +225,7 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W, D == 3 &&
 
 // ---- pass 2 + symplectic update ------------------------------------------
 template <int D, typename R, typename SS, bool Pipe, int W, int BS, bool G7, bool Quad>
-__global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W, D == 3 && W == 3 ? 3 : 8))) void k_pass2(SS ss) {
+__global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W, W == 3 ? 3 : 8))) void k_pass2(SS ss) {
 #pragma clang fp contract(off)
   GCLSPH_SCENE_PAIR(ss, BS, Quad);
   StepCtl* ctl = B.ctl;
@@ -206,6 +233,15 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W, D == 3 &&
   const double dt = ctl->dt;
   const bool active = a < B.n;
   double red_cdx = 0.0, red_acc = 0.0, red_visc = 0.0;
+  constexpr bool kStage = D == 2 && !Quad;
+  bool staged = false;
+  RowMap map{};
+  const int nc = active ? B.NC[a] : 0;
+  __shared__ uint4 lds[kStage ? kStagedWords : 1][kStage ? kStageCap<BS> : 1];
+  if constexpr (kStage) {
+    const int64_t a0 = int64_t(m.y) * BS;
+    if (a0 < B.n) staged = stage_rows<BS, kStagedWords>(lds, B.PRH, B, G, a0, nc, map);
+  }
   if (active) {
     const double* X[3] = {B.X[p][0], B.X[p][1], B.X[p][D == 3 ? 2 : 1]};
     const double* XH[3] = {B.XH[0], B.XH[1], B.XH[D == 3 ? 2 : 1]};
@@ -225,7 +261,6 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W, D == 3 &&
     const R sha = RH[a];
     const int32_t pta = PT[a];
     constexpr int kDrho = D;  // sums: D accelerations, ∂ρ/∂t
-    const int nc = B.NC[a];
     R av[3];
     R Pha, drho_v;
     if constexpr (std::is_same<R, double>::value) {
@@ -233,9 +268,11 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W, D == 3 &&
       Pha = B.PH[a];
       const Own<R> own = own_of<R>(sha, Pha, pta, C);
       using Nb = PartnerH64<D>;
-      auto fetch = [&](const int32_t b) { return ld_rec<Nb>(B.PRH, b, B.n); };
-      const auto sum = sum_partners<Pipe, Quad, D, D + 1, R>(B, a, nc, G, XM, C.dist2, fetch,
-                                                             [&](const Nb& q, auto& t) {
+      auto fetch = [&](const int32_t b, const auto... at) GCLSPH_INLINE {
+        if constexpr (sizeof...(at) > 0) return ld_staged<Nb, kStagedWords>(lds, at..., B.PRH, b, B.n);
+        else return ld_rec<Nb>(B.PRH, b, B.n);
+      };
+      auto pair = [&](const Nb& q, auto& t) GCLSPH_INLINE {
         double dxn[3], dx[3], dv[3];
 #pragma unroll
         for (int d = 0; d < D; ++d) {
@@ -247,7 +284,14 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W, D == 3 &&
         // force at xⁿ with (bound_D, bound_l) (:295)
         const double r2n = dist2_of<D>(dxn);
         pair_terms<D, G7, false>(C, F, own, q, q.rh, q.pt, q.P, dx, dv, dxn, r2n, root_of(r2n), 1, t);
-      });
+      };
+      Sums<D + 1, R> sum;
+      if constexpr (kStage) {
+        if (staged) sum = sum_staged<D + 1, R>(B, a, nc, map, fetch, pair);
+        else sum = sum_partners<Pipe, Quad, D, D + 1, R>(B, a, nc, G, XM, C.dist2, fetch, pair);
+      } else {
+        sum = sum_partners<Pipe, Quad, D, D + 1, R>(B, a, nc, G, XM, C.dist2, fetch, pair);
+      }
 #pragma unroll
       for (int d = 0; d < D; ++d) av[d] = sum.get(d);
       av[1] = av[1] - C.g;
@@ -312,12 +356,14 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W, D == 3 &&
 #pragma unroll
       for (int d = 0; d < D; ++d) dna[d] = float(xha[d] - xa[d]);
       const FrameK3 kt = particle_k<D, R>(B, C, G, a, xha);
-      auto gather = [&](auto derive_c) {
+      auto gather = [&](auto derive_c) GCLSPH_INLINE {
       constexpr bool derive = decltype(derive_c)::value;
       using Nb = std::conditional_t<derive, PartnerH<D>, PartnerHX<D>>;
-      auto fetch = [&](const int32_t b) { return ld_rec<Nb>(B.PRH, b, B.n); };
-      return sum_partners<Pipe, Quad, D, D + 1, R, true>(B, a, nc, G, XM, C.dist2, fetch,
-                                                         [&](const Nb& r, auto& t, const auto&... win) {
+      auto fetch = [&](const int32_t b, const auto... at) GCLSPH_INLINE {
+        if constexpr (sizeof...(at) > 0) return ld_staged<Nb, kStagedWords>(lds, at..., B.PRH, b, B.n);
+        else return ld_rec<Nb>(B.PRH, b, B.n);
+      };
+      auto pair = [&](const Nb& r, auto& t, const auto&... win) GCLSPH_INLINE {
         const PartnerH<D>* qp;
         if constexpr (derive) qp = &r;
         else qp = &r.h;
@@ -332,7 +378,11 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W, D == 3 &&
         }
         const float r2n = dist2_of<D>(dxn);
         pair_terms<D, G7, false>(C, F, own, q, q.rh, rec_pt(q), rec_P(q, C), dx, dv, dxn, r2n, root_of(r2n), 1, t);
-      }, &kt);
+      };
+      if constexpr (kStage) {
+        if (staged) return sum_staged<D + 1, R>(B, a, nc, map, fetch, pair);
+      }
+      return sum_partners<Pipe, Quad, D, D + 1, R, true>(B, a, nc, G, XM, C.dist2, fetch, pair, &kt);
       };
       const auto sum = F.synced_prev ? gather(std::true_type{}) : gather(std::false_type{});
 #pragma unroll
@@ -443,25 +493,37 @@ size_t cap_lds(int bs) {
   const size_t lds = cu / (blocks + 1) + 1024;  // the static LDS of a pass block is below 1 KiB
   return blocks * lds <= cu && lds <= blk ? lds : 0;
 }
-// code generation cg: 0 pipelined; 1 not pipelined; 2 pipelined, >= 3
-// waves/SIMD (3D: exactly 3); 3 (FP32-split) not pipelined, >= 5 waves/SIMD,
-// which makes FP64 spill: there it is 1
+// Code generation cg, 3D: 0 pipelined; 1 not pipelined; 2 pipelined, three waves
+// per SIMD; 3 (FP32-split) not pipelined, >= 5 waves/SIMD, which makes FP64
+// spill: there it is 1.  2D, where the records are staged, has one: four waves
+// per SIMD, as the staged records allow (FP64 pass 2 by itself would take the
+// registers of three: 246 us, 230 so, 1.02 M particles).
 template <int D, typename R, int BS>
 void pass1_cg(const LaunchSet& L, hipStream_t s, int cg, size_t lds) {
-  switch (cg) {
-    case 1: pass1_as<D, R, false, 1, BS>(L, s, lds); break;
-    case 2: pass1_as<D, R, true, 3, BS>(L, s, lds); break;
-    case 3: pass1_as<D, R, false, sizeof(R) == 8 ? 1 : 5, BS>(L, s, lds); break;
-    default: pass1_as<D, R, true, 1, BS>(L, s, lds); break;
+  if constexpr (D == 2) {
+    pass1_as<D, R, false, 4, BS>(L, s, 0);
+  } else {
+    constexpr bool f32 = std::is_same<R, float>::value;
+    switch (cg) {
+      case 0: pass1_as<D, R, true, 1, BS>(L, s, lds); break;
+      case 2: pass1_as<D, R, true, 3, BS>(L, s, lds); break;
+      case 3: pass1_as<D, R, false, f32 ? 5 : 1, BS>(L, s, lds); break;
+      default: pass1_as<D, R, false, 1, BS>(L, s, lds); break;
+    }
   }
 }
 template <int D, typename R, int BS>
 void pass2_cg(const LaunchSet& L, hipStream_t s, int cg, size_t lds) {
-  switch (cg) {
-    case 1: pass2_as<D, R, false, 1, BS>(L, s, lds); break;
-    case 2: pass2_as<D, R, true, 3, BS>(L, s, lds); break;
-    case 3: pass2_as<D, R, false, sizeof(R) == 8 ? 1 : 5, BS>(L, s, lds); break;
-    default: pass2_as<D, R, true, 1, BS>(L, s, lds); break;
+  if constexpr (D == 2) {
+    pass2_as<D, R, false, 4, BS>(L, s, 0);
+  } else {
+    constexpr bool f32 = std::is_same<R, float>::value;
+    switch (cg) {
+      case 0: pass2_as<D, R, true, 1, BS>(L, s, lds); break;
+      case 2: pass2_as<D, R, true, 3, BS>(L, s, lds); break;
+      case 3: pass2_as<D, R, false, f32 ? 5 : 1, BS>(L, s, lds); break;
+      default: pass2_as<D, R, false, 1, BS>(L, s, lds); break;
+    }
   }
 }
 }  // namespace

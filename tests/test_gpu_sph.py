@@ -639,6 +639,46 @@ def test_pair_quads_equal_one_lane(G, S, monkeypatch, prec, case):
             assert np.array_equal(np.asarray(a), np.asarray(b), equal_nan=True)
 
 
+@pytest.mark.parametrize("variant", ["0,0", "4,4", "8,8"])
+@pytest.mark.parametrize("prec", ["f64", "f32split"])
+@pytest.mark.parametrize("kind", ["narrow", "rows", "dense", "mixed"])
+def test_staged_rows_2d(G, S, monkeypatch, prec, kind, variant):
+    """The 2D passes stage the records of a block's three stencil rows in LDS.
+    Grids of one and two cells across, whose rows overlap (narrow), blocks that
+    go over row ends and a last block part-empty (rows), more records than the
+    LDS holds (dense) and a block with one particle beyond the membership store
+    (mixed, GCLSPH_NMASK_CAP) give the steps of the scan over global memory
+    (GCLSPH_NMASK_CAP=0) bit for bit, at each block size."""
+    n = 1000
+    u = [S.uniform01(13, n, k) for k in range(4)]
+    p, dist = S.standard_params(0.02, 2)
+    p.xsph_eps, p.cspmn = 0.5, 2
+    width = {"narrow": 1.4, "rows": 9.0, "dense": 2.0, "mixed": 9.0}[kind] * dist
+    height = {"narrow": 60.0, "rows": 9.0, "dense": 2.0, "mixed": 9.0}[kind] * dist
+    x, y = 0.1 + width * u[0], 0.1 + height * u[1]
+    if kind == "mixed":
+        x[:40], y[:40] = 0.1 + width * 0.5 + 0.2 * dist * u[0][:40], 0.1 + height * 0.5 + 0.2 * dist * u[1][:40]
+    v = (0.1 * (u[2] - 0.5), 0.1 * (u[3] - 0.5))
+    rho = np.full(n, p.rho0) * (1 + 1e-3 * u[2])
+    monkeypatch.setenv("GCLSPH_PAIR_LANES", "1")
+    monkeypatch.setenv("GCLSPH_PASS_VARIANT", variant)
+
+    def run(cap):
+        if cap is None:
+            monkeypatch.delenv("GCLSPH_NMASK_CAP", raising=False)
+        else:
+            monkeypatch.setenv("GCLSPH_NMASK_CAP", str(cap))
+        cl = G.GPUCellList((x, y), (dist, dist), dist)
+        prob = G.SPHProblem.from_params(cl, p, rho, np.where(np.arange(n) % 9 == 4, 1, 2), v=v, precision=prec)
+        out = [G.stepsolve_(prob, k, timestepping=False) for k in (1, 3)]
+        return out + [np.asarray(gpu_fields(G, prob)[f]) for f in FIELDS]
+
+    ref = run(0)
+    for cap in (None, 4) if kind == "mixed" else (None,):
+        for a, b in zip(run(cap), ref):
+            assert np.array_equal(np.asarray(a), np.asarray(b), equal_nan=True)
+
+
 @pytest.mark.parametrize("n", [1, 2, 63, 65, 257, 1000])
 def test_tiny_and_ragged_problems(G, O, S, n):
     """Problems of 1 and 2 particles and counts that leave the last wave or
