@@ -128,17 +128,20 @@ double sqrt_threshold(double r) {
 
 // Whether a set of n particles in all is stepped with a quad of lanes per
 // particle (same results): up to about where one lane per particle begins to
-// fill the chip.  Step time of one lane / of a quad: 2D FP32-split 1.35 at 1 k
-// to 14 k particles, 1.27 at 28 k, 1.13 at 54 k, 0.97 at 106 k; 2D FP64 1.38,
-// 1.27, 1.01, 0.91; 3D FP64 1.54 at 19 k, 1.17 at 54 k, 1.04 at 91 k, 0.96 at
-// 155 k; 3D FP32-split with every term 1.81, 1.33, 1.17, 0.99.
+// fill the chip.  Step time of one lane / of a quad: 2D FP32-split 1.52 at 14 k
+// particles, 1.22 at 54 k, 1.04 at 106 k, 0.99 at 118 k; 2D FP64 1.50, 1.11, 0.99
+// at 106 k; 3D FP32-split with every term 1.13 at 91 k, 1.00 at 155 k, 0.94 at
+// 219 k.  In 3D FP64 the passes are bound by the L1, not by the VALU that a quad
+// costs, and the four lanes of a particle ask for records that lie together: 1.05
+// at 91 k, 1.09 at 219 k, 1.04 at 488 k, 1.05 at 709 k, 1.02 at 1.16 M (with every
+// term 1.12 at 155 k, 1.06 at 488 k).
 // GCLSPH_PAIR_LANES=1|4 forces one of them.
 bool pair_quads(int64_t n, int dim, bool split) {
   if (const char* env = std::getenv("GCLSPH_PAIR_LANES")) {
     if (std::strcmp(env, "1") == 0) return false;
     if (std::strcmp(env, "4") == 0) return true;
   }
-  return n <= (dim == 2 ? (split ? 80000 : 50000) : (split ? 140000 : 110000));
+  return n <= (dim == 2 ? (split ? 110000 : 95000) : (split ? 140000 : 700000));
 }
 
 int64_t ceil_div08(int64_t v) { return int64_t(std::ceil(double(v) / 0.8)); }
