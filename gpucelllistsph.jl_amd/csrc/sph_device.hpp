@@ -623,7 +623,7 @@ __device__ __forceinline__ void st_rec(void* base, int64_t a, const T& r, int64_
 // FP32-split one, half of an FP64 one; the other FP64 words stay with the L1.
 // Three words staged left LDS for three waves per SIMD instead of four (1.02 M
 // particles FP64: 52 KiB a block).  FP32-split passes are then bound by VALU
-// issue (1.0 per CU and cycle).  3.95 M particles FP32-split: passes 414 + 481
+// issue (1.0 per CU and cycle).  4.05 M particles FP32-split: passes 414 + 481
 // -> 380 + 433 us; 1.02 M FP64: 189 + 259 -> 180 + 230 us.
 constexpr int kStagedWords = 2;
 // Records staged at most.  The rows above and below a block's cells hold up to
