@@ -771,7 +771,7 @@ void LaunchSet::build(const int64_t* n, const int64_t* ncells, unsigned cnt, int
   for (scan_rows = 4; scan_rows < 16; scan_rows *= 2) {
     int64_t tiles = 0;
     for (unsigned i = 0; i < cnt; ++i) tiles += scan_tiles(ncells[i], scan_rows);
-    if (tiles <= kScanInOrder) break;
+    if (tiles <= kScanTiles) break;
   }
   quad = pair_quads(total, dim, split);
   for (unsigned i = 0; i < cnt; ++i) {

@@ -12,11 +12,14 @@ constexpr int kScanThreads = 256;
 constexpr int kScanRow = 4 * kScanThreads;  // items of one 16-byte load per thread
 
 // A device-wide scan runs in tiles of 4, 8 or 16 rows, a block each: as many
-// rows as keep it within kScanInOrder blocks (scan_tile below), fewest first.
-constexpr int kScanInOrder = 512;
+// rows as keep it within kScanTiles blocks, fewest first: a block costs its turn
+// at the tile counter (scan_tile below), a long tile its own time.  Limits of
+// 256 / 512: 700,000 cells 9.1 / 9.0 us (4 rows both), 2.8 M cells 16.3 (16 rows) /
+// 16.5 us (8), the cells of 64 problems, each with a counter, 10.1 (8) / 8.4 us (4).
+constexpr int kScanTiles = 512;
 constexpr int64_t scan_tiles(int64_t n, int rows) { return (n + rows * kScanRow - 1) / (rows * kScanRow); }
 constexpr int scan_rows(int64_t n) {
-  return scan_tiles(n, 4) <= kScanInOrder ? 4 : (scan_tiles(n, 8) <= kScanInOrder ? 8 : 16);
+  return scan_tiles(n, 4) <= kScanTiles ? 4 : (scan_tiles(n, 8) <= kScanTiles ? 8 : 16);
 }
 // Words of the scratch array of a device-wide scan: a ticket counter, then one
 // status word per tile.
@@ -46,25 +49,26 @@ __device__ __forceinline__ void clear_scan_words(uint64_t* words, int64_t n, int
 // maximum of the items.  Clear: the items are zero afterwards.  in and out are
 // 16-byte aligned.
 //
-// A block waits only for tiles before its own, so every wait ends if those
-// blocks run.  In a launch of at most kScanInOrder blocks `tile` is the block's
-// place in the grid: all of them fit the chip at once (it holds 2048 such
-// blocks, an eighth of them on each XCD, and four launches can run at a time),
-// whatever else it runs.  Beyond that (tile < 0) blocks take tiles from a
-// counter, so a tile before one's own is a running block's; the counter costs
-// ~24 ns a block, one after the other.
+// A block waits only for tiles before its own, and takes its tile from a counter
+// when it starts: those tiles are then with blocks that run already, whatever
+// else the chip runs, so every wait ends.  (A block's place in the grid as its
+// tile promises that only while all blocks of all scans in flight fit the chip:
+// of 16 rows of 64-bit sums one block fits a CU, 256 the chip.)  A scan of one
+// tile needs no counter.  Time with the counter / with places in the grid: 6,000
+// and 60,000 cells 2.1 / 2.1 and 4.8 / 4.8 us, 700,000 9.0 / 8.5, 2.8 M 16.5 / 14.8.
 //
 // One launch instead of three (tile sums, their scan, the tiles again): each
 // launch of a step costs 4.4 us however small, and the items are read once.
 template <int Rows, bool Clear, typename O>
 __device__ __forceinline__ void scan_tile(int32_t* __restrict__ in, O* __restrict__ out, int64_t n,
-                                          uint64_t* __restrict__ words, int32_t* max_out, int64_t tile) {
+                                          uint64_t* __restrict__ words, int32_t* max_out) {
   constexpr uint64_t kSum = uint64_t(1) << 62, kPrefix = uint64_t(2) << 62, kValue = kSum - 1;
   constexpr int kWaves = kScanThreads / 64;
   __shared__ uint64_t ticket, wadd[kWaves];
   __shared__ O wsum[Rows][kWaves];
   __shared__ int32_t wmax[kWaves], wfull[kWaves];
-  if (tile < 0) {  // uniform
+  int64_t tile = 0;
+  if (scan_tiles(n, Rows) > 1) {  // uniform
     if (threadIdx.x == 0) ticket = atomicAdd(reinterpret_cast<unsigned long long*>(words), 1ull);
     __syncthreads();
     tile = int64_t(ticket);

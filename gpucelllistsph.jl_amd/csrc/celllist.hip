@@ -69,16 +69,14 @@ __global__ void k_cellmap(XPtrs src, int64_t n, CellGeom g, int use_off64, int32
 template <int Rows>
 __global__ __launch_bounds__(kScanThreads) void k_cell_starts(int32_t* cnt, int32_t* start, int64_t ncells,
                                                               uint64_t* words, int32_t* maxcell) {
-  scan_tile<Rows, true>(cnt, start, ncells, words, maxcell,
-                        gridDim.x <= kScanInOrder ? int64_t(blockIdx.x) : int64_t(-1));
+  scan_tile<Rows, true>(cnt, start, ncells, words, maxcell);
 }
 
 // Offsets of the pairs from their counts.
 template <int Rows>
 __global__ __launch_bounds__(kScanThreads) void k_pair_offsets(int32_t* cnt, int64_t* off, int64_t n,
                                                                uint64_t* words) {
-  scan_tile<Rows, false>(cnt, off, n, words, nullptr,
-                         gridDim.x <= kScanInOrder ? int64_t(blockIdx.x) : int64_t(-1));
+  scan_tile<Rows, false>(cnt, off, n, words, nullptr);
 }
 
 // Item visited t-th (order as in k_cellmap) to its arrival slot: tmp holds

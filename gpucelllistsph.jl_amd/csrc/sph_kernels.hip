@@ -995,8 +995,7 @@ __global__ __launch_bounds__(kScanThreads) void kb_cell_starts(SS ss) {
   int2 m;
   const SceneDev<R>& sd = tile_scene<R>(ss, m);
   if (sd.B.ctl->rebuild == 0) return;
-  scan_tile<Rows, true>(sd.cnt, sd.start, sd.ncells, sd.scan_tmp, sd.maxcell,
-                        gridDim.x <= kScanInOrder ? int64_t(m.y) : int64_t(-1));
+  scan_tile<Rows, true>(sd.cnt, sd.start, sd.ncells, sd.scan_tmp, sd.maxcell);
 }
 
 // Sort key of an x coordinate: its bit pattern made unsigned-monotone (order

@@ -1,6 +1,8 @@
 """Batched ensemble: problems stepped together (one launch per stage for all of
 them) end bit-identical to the same problems stepped one by one, each keeping
 its own Δt, rebuild schedule, time and corrections."""
+import math
+
 import numpy as np
 import pytest
 from cases import golden_cases
@@ -87,6 +89,32 @@ def test_batch_of_uneven_gamma_matches_one_by_one(G, S):
             G.stepsolve_(p, n, timestepping=True)
         G.batch_stepsolve_(batch, n, timestepping=True)
     for a, b in zip(alone, probs):
+        fa, fb = fields(G, a), fields(G, b)
+        for name in fa:
+            assert np.array_equal(fa[name], fb[name]), name
+
+
+@pytest.mark.parametrize("cells", [(1400, 1000), (2600, 1200), (3100, 2900)])
+def test_batch_with_many_cells(G, S, cells):
+    """The cell scan of a batch: problems whose grids reach far beyond their
+    points, two together 8 rows a tile, 16, and beyond 512 tiles of 16, end as on
+    tight grids, bit for bit."""
+    scs = [golden_cases()["dam2d"][0], S.dam_break_2d(0.05, 0.5, 1.0, 2.0, 1.5)]
+
+    def problem(sc, wide):
+        mn = tuple(float(a.min()) - 0.01 for a in sc.points)
+        far = cells if wide else tuple(math.ceil((a.max() - b) / c) + 1 for a, b, c in zip(sc.points, mn, sc.cellsize))
+        mx = tuple(b + k * c for b, k, c in zip(mn, far, sc.cellsize))
+        cl = G.GPUCellList(sc.points, sc.cellsize, sc.dist, MIN=mn, MAX=mx)
+        return G.SPHProblem.from_params(cl, sc.params, sc.rho, sc.ptype, v=sc.v, precision="f64")
+
+    tight, wide = ([problem(sc, w) for sc in scs] for w in (False, True))
+    batch = G.SPHBatch(wide)
+    for n in (1, 3):
+        for p in tight:
+            G.stepsolve_(p, n, timestepping=True)
+        G.batch_stepsolve_(batch, n, timestepping=True)
+    for a, b in zip(tight, wide):
         fa, fb = fields(G, a), fields(G, b)
         for name in fa:
             assert np.array_equal(fa[name], fb[name]), name

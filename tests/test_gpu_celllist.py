@@ -72,6 +72,46 @@ def test_scan_tiles(G, O, S, n, cells):
     assert_same_celllist(g, o)
 
 
+@pytest.mark.parametrize("cells", [(2050, 1024), (2600, 2000), (2900, 2890)])
+def test_scan_tiles_of_8_and_16_rows(G, O, S, cells):
+    """Cell starts of 2.1 M cells (8 rows a tile), 5.2 M and 8.4 M (16 rows, 318
+    and 512 tiles)."""
+    n = 20001
+    x, y = S.uniform01(11, n, 0) * cells[0], S.uniform01(11, n, 1) * cells[1]
+    kw = dict(MIN=(1e-9, 1e-9), MAX=tuple(float(c) for c in cells))
+    g = G.GPUCellList((x, y), (1.0, 1.0), 0.25, **kw)
+    o = O.CellList((x, y), (1.0, 1.0), 0.25, **kw)
+    assert_same_celllist(g, o)
+    G.update_(g)
+    o.update()
+    assert_same_celllist(g, o)
+
+
+@pytest.mark.parametrize("n", [2_097_153, 2_200_007, 4_300_001, 8_500_009])
+def test_pair_offsets_of_millions_of_points(G, n):
+    """Pair offsets are a scan over the points: 8 rows a tile from 2.1 M points,
+    16 from 4.2 M, more than 512 tiles from 8.4 M.  Points 4 apart along a row, two
+    of every five with a partner at 0.5, one of them with a second one at 0.25
+    from that: every pair is known."""
+    i = np.arange(n)
+    k = i % 8  # of eight consecutive points: 0, 1 | 2 | 3, 4, 5 | 6 | 7
+    head = np.array([0, 0, 2, 3, 3, 3, 6, 7])[k]
+    site = (i // 8) * 5 + np.array([0, 0, 1, 2, 2, 2, 3, 4])[k]
+    row = 3000
+    x = (site % row) * 4.0 + np.array([0, 0.5, 0.75])[k - head]
+    y = (site // row) * 4.0
+    e, m = n // 8 * 8 + 8, 8
+    lo = np.concatenate([np.arange(0, e, m), np.arange(3, e, m), np.arange(3, e, m), np.arange(4, e, m)])
+    hi = np.concatenate([np.arange(1, e, m), np.arange(4, e, m), np.arange(5, e, m), np.arange(5, e, m)])
+    want = np.stack([lo, hi], 1)[hi < n] + 1
+    g = G.GPUCellList((x, y), (16.0, 16.0), 1.0)
+    for _ in range(2):
+        assert g.pairsn == len(want)
+        got = G.neighborlistview(g)
+        assert np.array_equal(got[np.lexsort(got.T[::-1])], want[np.lexsort(want.T[::-1])])
+        G.update_(g)
+
+
 def test_config1_update_and_partialupdate(G, O, S):
     """200,000 uniform points, cellsize = dist = 0.016, jittered by N(0, 0.001^2) per step."""
     pts = S.config1_points()
