@@ -17,12 +17,13 @@
 
 namespace gclsph {
 
-// The page-locked slots, shared by all objects: allocated at the first copy,
-// freed with the last object (Ref).  One copy at a time uses them.
+// The page-locked slots: a set of them for each copy that runs.  Up to kKept sets
+// stay for the next copies, of any object and device; the last object (Ref) to
+// go frees them.  The lock is held to take a set and to give it back only.
 class HostSlots {
  public:
   static constexpr size_t kSlot = size_t(1) << 20;
-  static constexpr int kThreads = 4, kSlots = 2 * kThreads;
+  static constexpr int kThreads = 4, kSlots = 2 * kThreads, kKept = 4;
 
   // Held by every object that may copy.
   struct Ref {
@@ -33,10 +34,8 @@ class HostSlots {
     ~Ref() {
       HostSlots& s = self();
       std::lock_guard<std::mutex> l(s.mutex_);
-      if (--s.refs_ == 0 && s.mem_) {
-        (void)hipHostFree(s.mem_);
-        s.mem_ = nullptr;
-      }
+      if (--s.refs_ > 0) return;
+      while (s.kept_ > 0) (void)hipHostFree(s.free_[--s.kept_]);
     }
     Ref(const Ref&) = delete;
     Ref& operator=(const Ref&) = delete;
@@ -47,19 +46,13 @@ class HostSlots {
   // called from several threads, one chunk each).  Returns when out is complete.
   template <typename Fill>
   static void copy_out(void* out, size_t bytes, hipStream_t st, const Fill& fill) {
-    HostSlots& s = self();
-    std::lock_guard<std::mutex> l(s.mutex_);
-    if (!s.mem_) {
-      void* p = nullptr;
-      GCL_HIP(hipHostMalloc(&p, kSlot * kSlots, hipHostMallocPortable));
-      s.mem_ = static_cast<char*>(p);
-    }
+    if (bytes == 0) return;
+    const Set set;
     char* dst = static_cast<char*>(out);
     if (bytes <= kSlot) {
-      if (bytes == 0) return;
-      fill(s.mem_, size_t(0), bytes);
+      fill(set.mem, size_t(0), bytes);
       GCL_HIP(hipStreamSynchronize(st));
-      std::memcpy(dst, s.mem_, bytes);
+      std::memcpy(dst, set.mem, bytes);
       return;
     }
     const size_t chunks = (bytes + kSlot - 1) / kSlot;
@@ -74,7 +67,7 @@ class HostSlots {
         GCL_HIP(hipSetDevice(dev));
         for (auto& e : ev) GCL_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
         auto start = [&](size_t c, int k) {
-          fill(s.mem_ + kSlot * size_t(2 * t + k), c * kSlot, std::min(kSlot, bytes - c * kSlot));
+          fill(set.mem + kSlot * size_t(2 * t + k), c * kSlot, std::min(kSlot, bytes - c * kSlot));
           GCL_HIP(hipEventRecord(ev[k], st));
         };
         for (int k = 0; k < 2; ++k)
@@ -82,7 +75,7 @@ class HostSlots {
         int k = 0;
         for (size_t c = size_t(t); c < chunks; c += size_t(threads), k ^= 1) {
           GCL_HIP(hipEventSynchronize(ev[k]));
-          std::memcpy(dst + c * kSlot, s.mem_ + kSlot * size_t(2 * t + k), std::min(kSlot, bytes - c * kSlot));
+          std::memcpy(dst + c * kSlot, set.mem + kSlot * size_t(2 * t + k), std::min(kSlot, bytes - c * kSlot));
           if (c + 2 * size_t(threads) < chunks) start(c + 2 * size_t(threads), k);
         }
       } catch (...) {
@@ -105,13 +98,42 @@ class HostSlots {
   }
 
  private:
+  // A copy's own slots.
+  struct Set {
+    char* mem = nullptr;
+    Set() {
+      HostSlots& s = self();
+      {
+        std::lock_guard<std::mutex> l(s.mutex_);
+        if (s.kept_ > 0) mem = s.free_[--s.kept_];
+      }
+      if (mem) return;
+      void* p = nullptr;
+      GCL_HIP(hipHostMalloc(&p, kSlot * kSlots, hipHostMallocPortable));
+      mem = static_cast<char*>(p);
+    }
+    ~Set() {
+      HostSlots& s = self();
+      {
+        std::lock_guard<std::mutex> l(s.mutex_);
+        if (s.refs_ > 0 && s.kept_ < kKept) {
+          s.free_[s.kept_++] = mem;
+          return;
+        }
+      }
+      (void)hipHostFree(mem);
+    }
+    Set(const Set&) = delete;
+    Set& operator=(const Set&) = delete;
+  };
+
   static HostSlots& self() {
     static HostSlots s;
     return s;
   }
   std::mutex mutex_;
-  int refs_ = 0;
-  char* mem_ = nullptr;
+  int refs_ = 0, kept_ = 0;
+  char* free_[kKept] = {};
 };
 
 }  // namespace gclsph

@@ -1,13 +1,16 @@
-// The part of the HIP language that csrc/blockscan.hpp uses, for the host: the
-// threads of one block as fibers that run in turn and meet at the collectives.
+// The part of HIP that csrc/blockscan.hpp and csrc/readback.hpp use, for the host:
+// the threads of one block as fibers that run in turn and meet at the
+// collectives, and streams and events that do what a test gives them to do.
 #pragma once
 
 #include <ucontext.h>
 
+#include <atomic>
 #include <cstdint>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <functional>
 #include <vector>
 
 #define __global__
@@ -17,8 +20,61 @@
 #define __shared__ static  // one block at a time
 #define __launch_bounds__(...)
 
+// ---- runtime
 enum hipError_t { hipSuccess = 0, hipErrorUnknown = 1 };
 inline const char* hipGetErrorString(hipError_t) { return "error"; }
+
+struct ihipStream_t {
+  std::function<void()> wait;  // until the stream's work is done
+};
+using hipStream_t = ihipStream_t*;
+struct ihipEvent_t {
+  hipStream_t stream = nullptr;
+};
+using hipEvent_t = ihipEvent_t*;
+constexpr unsigned hipEventDisableTiming = 2, hipHostMallocPortable = 1;
+
+inline hipError_t hipGetDevice(int* d) {
+  *d = 0;
+  return hipSuccess;
+}
+inline hipError_t hipSetDevice(int) { return hipSuccess; }
+inline hipError_t hipStreamSynchronize(hipStream_t s) {
+  if (s->wait) s->wait();
+  return hipSuccess;
+}
+inline hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
+  *e = new ihipEvent_t;
+  return hipSuccess;
+}
+inline hipError_t hipEventDestroy(hipEvent_t e) {
+  delete e;
+  return hipSuccess;
+}
+inline hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
+  e->stream = s;
+  return hipSuccess;
+}
+inline hipError_t hipEventSynchronize(hipEvent_t e) { return hipStreamSynchronize(e->stream); }
+inline std::atomic<int64_t>& pinned_bytes() {
+  static std::atomic<int64_t> b{0};
+  return b;
+}
+inline hipError_t hipHostMalloc(void** p, size_t bytes, unsigned) {
+  auto* m = static_cast<size_t*>(std::malloc(bytes + 64));
+  *m = bytes;
+  pinned_bytes() += int64_t(bytes);
+  *p = reinterpret_cast<char*>(m) + 64;
+  return hipSuccess;
+}
+inline hipError_t hipHostFree(void* p) {
+  auto* m = reinterpret_cast<size_t*>(static_cast<char*>(p) - 64);
+  pinned_bytes() -= int64_t(*m);
+  std::free(m);
+  return hipSuccess;
+}
+
+// ---- device code
 
 struct uint3 {
   unsigned x = 0, y = 0, z = 0;
