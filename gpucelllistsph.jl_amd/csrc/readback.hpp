@@ -7,8 +7,8 @@
 #pragma once
 
 #include <algorithm>
-#include <atomic>
 #include <cstring>
+#include <exception>
 #include <mutex>
 #include <thread>
 #include <vector>
@@ -60,7 +60,8 @@ class HostSlots {
     const int threads = int(std::min<size_t>(kThreads, (chunks + 1) / 2));
     int dev = 0;
     GCL_HIP(hipGetDevice(&dev));
-    std::atomic<int> failed{0};
+    std::exception_ptr failed;  // the first failure of a thread
+    std::mutex failed_mutex;
     auto work = [&](int t) noexcept {
       hipEvent_t ev[2] = {nullptr, nullptr};
       try {
@@ -79,7 +80,8 @@ class HostSlots {
           if (c + 2 * size_t(threads) < chunks) start(c + 2 * size_t(threads), k);
         }
       } catch (...) {
-        failed = 1;
+        std::lock_guard<std::mutex> l(failed_mutex);
+        if (!failed) failed = std::current_exception();
       }
       for (auto& e : ev)
         if (e) (void)hipEventDestroy(e);
@@ -93,8 +95,9 @@ class HostSlots {
     work(0);
     for (auto& t : pool) t.join();
     for (int t = started; t < threads; ++t) work(t);
-    GCL_HIP(hipStreamSynchronize(st));  // the slots are free again, also after a failure
-    GCL_CHECK(!failed, kErrHip, "copying results to the host failed");
+    const hipError_t end = hipStreamSynchronize(st);  // the slots are free again, also after a failure
+    if (failed) std::rethrow_exception(failed);
+    GCL_HIP(end);
   }
 
  private:

@@ -22,10 +22,11 @@
 
 // ---- runtime
 enum hipError_t { hipSuccess = 0, hipErrorUnknown = 1 };
-inline const char* hipGetErrorString(hipError_t) { return "error"; }
+inline const char* hipGetErrorString(hipError_t) { return "unknown error"; }
 
 struct ihipStream_t {
   std::function<void()> wait;  // until the stream's work is done
+  hipError_t result = hipSuccess;  // of that work
 };
 using hipStream_t = ihipStream_t*;
 struct ihipEvent_t {
@@ -41,7 +42,7 @@ inline hipError_t hipGetDevice(int* d) {
 inline hipError_t hipSetDevice(int) { return hipSuccess; }
 inline hipError_t hipStreamSynchronize(hipStream_t s) {
   if (s->wait) s->wait();
-  return hipSuccess;
+  return s->result;
 }
 inline hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
   *e = new ihipEvent_t;

@@ -83,6 +83,36 @@ void many() {
   }
   expect(pinned_bytes() == 0, "page-locked memory is left");
 }
+
+// The caller learns what failed: a launch, or the work of the stream.
+void errors() {
+  HostSlots::Ref a;
+  for (size_t chunks : {1, 2, 3, 20}) {
+    for (size_t bad : {size_t(0), chunks / 2, chunks - 1}) {
+      std::vector<char> out(chunks * HostSlots::kSlot);
+      ihipStream_t st;
+      std::string got;
+      try {
+        HostSlots::copy_out(out.data(), out.size(), &st, [&](void*, size_t off, size_t) {
+          if (off == bad * HostSlots::kSlot) throw Error(kErrHip, "launch: out of resources");
+        });
+      } catch (const Error& e) {
+        if (e.code == kErrHip) got = e.what();
+      }
+      expect(got == "launch: out of resources", "a failed launch is reported otherwise");
+    }
+    std::vector<char> out(chunks * HostSlots::kSlot);
+    ihipStream_t st;
+    st.result = hipErrorUnknown;
+    std::string got;
+    try {
+      copy(out, out, &st);
+    } catch (const Error& e) {
+      if (e.code == kErrHip) got = e.what();
+    }
+    expect(got.find("unknown error") != std::string::npos, "a failed stream is reported otherwise");
+  }
+}
 }  // namespace
 
 int main(int, char** argv) {
@@ -92,6 +122,8 @@ int main(int, char** argv) {
     overlap(9 * HostSlots::kSlot + 5);
   } else if (what == "many") {
     many();
+  } else if (what == "errors") {
+    errors();
   }
   return failures ? 1 : 0;
 }

@@ -29,3 +29,8 @@ def test_copies_of_different_streams_overlap(readback):
 def test_page_locked_memory_is_bounded_and_given_back(readback):
     """24 threads copy at once, sizes at and around a slot and beyond a set."""
     check(readback, "many")
+
+
+def test_the_failure_of_a_copy_is_reported(readback):
+    """What a launch or the stream failed with reaches the caller, from every thread of a copy."""
+    check(readback, "errors")
