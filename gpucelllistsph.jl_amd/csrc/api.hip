@@ -569,6 +569,7 @@ struct sph_s {
   // comps components of a sorted field to out (comps blocks of n) in caller order.
   template <typename T>
   void export_fields(const T* const* src, int comps, double add, double* out) {
+    const OnDeviceOf on(stream);
     const int32_t* inv = slots_by_id();
     const Fields<T> f{{src[0], src[comps > 1 ? 1 : 0], src[comps > 2 ? 2 : 0]}};
     HostSlots::copy_out(out, sizeof(double) * size_t(n) * size_t(comps), stream,

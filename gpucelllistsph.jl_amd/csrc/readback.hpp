@@ -17,6 +17,27 @@
 
 namespace gclsph {
 
+// The stream's device is the thread's current one within the scope: an event can
+// be recorded on a stream of its own device only, and a thread that reads results
+// may have another one current (a new thread has device 0).
+class OnDeviceOf {
+ public:
+  explicit OnDeviceOf(hipStream_t st) {
+    GCL_HIP(hipStreamGetDevice(st, &device));
+    GCL_HIP(hipGetDevice(&before_));
+    if (before_ != device) GCL_HIP(hipSetDevice(device));
+  }
+  ~OnDeviceOf() {
+    if (before_ != device) (void)hipSetDevice(before_);
+  }
+  OnDeviceOf(const OnDeviceOf&) = delete;
+  OnDeviceOf& operator=(const OnDeviceOf&) = delete;
+  int device = 0;
+
+ private:
+  int before_ = 0;
+};
+
 // The page-locked slots: a set of them for each copy that runs.  Up to kKept sets
 // stay for the next copies, of any object and device; the last object (Ref) to
 // go frees them.  The lock is held to take a set and to give it back only.
@@ -47,6 +68,7 @@ class HostSlots {
   template <typename Fill>
   static void copy_out(void* out, size_t bytes, hipStream_t st, const Fill& fill) {
     if (bytes == 0) return;
+    const OnDeviceOf on(st);
     const Set set;
     char* dst = static_cast<char*>(out);
     if (bytes <= kSlot) {
@@ -58,14 +80,12 @@ class HostSlots {
     const size_t chunks = (bytes + kSlot - 1) / kSlot;
     // a thread pays from about a megabyte on (~20 us to start one)
     const int threads = int(std::min<size_t>(kThreads, (chunks + 1) / 2));
-    int dev = 0;
-    GCL_HIP(hipGetDevice(&dev));
     std::exception_ptr failed;  // the first failure of a thread
     std::mutex failed_mutex;
     auto work = [&](int t) noexcept {
       hipEvent_t ev[2] = {nullptr, nullptr};
       try {
-        GCL_HIP(hipSetDevice(dev));
+        GCL_HIP(hipSetDevice(on.device));
         for (auto& e : ev) GCL_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
         auto start = [&](size_t c, int k) {
           fill(set.mem + kSlot * size_t(2 * t + k), c * kSlot, std::min(kSlot, bytes - c * kSlot));

@@ -21,31 +21,45 @@
 #define __launch_bounds__(...)
 
 // ---- runtime
-enum hipError_t { hipSuccess = 0, hipErrorUnknown = 1 };
-inline const char* hipGetErrorString(hipError_t) { return "unknown error"; }
+enum hipError_t { hipSuccess = 0, hipErrorUnknown = 1, hipErrorInvalidHandle = 2 };
+inline const char* hipGetErrorString(hipError_t e) {
+  return e == hipErrorInvalidHandle ? "invalid resource handle" : "unknown error";
+}
 
 struct ihipStream_t {
   std::function<void()> wait;  // until the stream's work is done
   hipError_t result = hipSuccess;  // of that work
+  int device = 0;
 };
 using hipStream_t = ihipStream_t*;
 struct ihipEvent_t {
   hipStream_t stream = nullptr;
+  int device = 0;
 };
 using hipEvent_t = ihipEvent_t*;
+using hipDevice_t = int;
 constexpr unsigned hipEventDisableTiming = 2, hipHostMallocPortable = 1;
 
+inline thread_local int current_device = 0;  // a new thread has device 0
 inline hipError_t hipGetDevice(int* d) {
-  *d = 0;
+  *d = current_device;
   return hipSuccess;
 }
-inline hipError_t hipSetDevice(int) { return hipSuccess; }
+inline hipError_t hipSetDevice(int d) {
+  current_device = d;
+  return hipSuccess;
+}
+inline hipError_t hipStreamGetDevice(hipStream_t s, hipDevice_t* d) {
+  *d = s->device;
+  return hipSuccess;
+}
 inline hipError_t hipStreamSynchronize(hipStream_t s) {
   if (s->wait) s->wait();
   return s->result;
 }
 inline hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
   *e = new ihipEvent_t;
+  (*e)->device = current_device;
   return hipSuccess;
 }
 inline hipError_t hipEventDestroy(hipEvent_t e) {
@@ -53,6 +67,7 @@ inline hipError_t hipEventDestroy(hipEvent_t e) {
   return hipSuccess;
 }
 inline hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
+  if (e->device != s->device) return hipErrorInvalidHandle;
   e->stream = s;
   return hipSuccess;
 }

@@ -113,6 +113,33 @@ void errors() {
     expect(got.find("unknown error") != std::string::npos, "a failed stream is reported otherwise");
   }
 }
+
+// A thread whose current device is not the stream's reads as any other, and keeps
+// its device.
+void devices() {
+  HostSlots::Ref a;
+  for (int current : {0, 1}) {
+    for (size_t bytes : {size_t(1000), 9 * HostSlots::kSlot + 5}) {
+      current_device = current;
+      ihipStream_t st;
+      st.device = 1;
+      const auto src = pattern(bytes, 3);
+      std::vector<char> out(bytes);
+      std::atomic<int> elsewhere{0};
+      try {
+        HostSlots::copy_out(out.data(), bytes, &st, [&](void* slot, size_t off, size_t len) {
+          elsewhere += current_device != st.device;
+          std::memcpy(slot, src.data() + off, len);
+        });
+      } catch (const Error& e) {
+        expect(false, e.what());
+      }
+      expect(out == src, "wrong bytes");
+      expect(elsewhere == 0, "a launch with another device current");
+      expect(current_device == current, "the thread's device changed");
+    }
+  }
+}
 }  // namespace
 
 int main(int, char** argv) {
@@ -124,6 +151,8 @@ int main(int, char** argv) {
     many();
   } else if (what == "errors") {
     errors();
+  } else if (what == "devices") {
+    devices();
   }
   return failures ? 1 : 0;
 }

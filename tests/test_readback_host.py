@@ -34,3 +34,8 @@ def test_page_locked_memory_is_bounded_and_given_back(readback):
 def test_the_failure_of_a_copy_is_reported(readback):
     """What a launch or the stream failed with reaches the caller, from every thread of a copy."""
     check(readback, "errors")
+
+
+def test_copies_with_another_device_current(readback):
+    """The stream's device need not be the one that is current in the thread that reads."""
+    check(readback, "devices")
