@@ -134,14 +134,16 @@ double sqrt_threshold(double r) {
 // 219 k.  In 3D FP64 the passes are bound by the L1, not by the VALU that a quad
 // costs, and the four lanes of a particle ask for records that lie together: 1.05
 // at 91 k, 1.09 at 219 k, 1.04 at 488 k, 1.05 at 709 k, 1.02 at 1.16 M (with every
-// term 1.12 at 155 k, 1.06 at 488 k).
+// term 1.12 at 155 k, 1.06 at 488 k).  The FP64 passes of another γ are bound by
+// the VALU again: 2D 1.12 at 59 k and 1.14 at 96 k, 3D 1.18 at 87 k, 1.10 at 149 k,
+// 0.96 at 186 k.
 // GCLSPH_PAIR_LANES=1|4 forces one of them.
-bool pair_quads(int64_t n, int dim, bool split) {
+bool pair_quads(int64_t n, int dim, bool split, bool gamma7) {
   if (const char* env = std::getenv("GCLSPH_PAIR_LANES")) {
     if (std::strcmp(env, "1") == 0) return false;
     if (std::strcmp(env, "4") == 0) return true;
   }
-  return n <= (dim == 2 ? (split ? 110000 : 95000) : (split ? 140000 : 700000));
+  return n <= (dim == 2 ? (split ? 110000 : 95000) : (split ? 140000 : (gamma7 ? 700000 : 160000)));
 }
 
 int64_t ceil_div08(int64_t v) { return int64_t(std::ceil(double(v) / 0.8)); }
@@ -774,7 +776,8 @@ void LaunchSet::build(const int64_t* n, const int64_t* ncells, unsigned cnt, int
     for (unsigned i = 0; i < cnt; ++i) tiles += scan_tiles(ncells[i], scan_rows);
     if (tiles <= kScanTiles) break;
   }
-  quad = pair_quads(total, dim, split);
+  quad = pair_quads(total, dim, split, true);
+  quad_general = pair_quads(total, dim, split, false);
   for (unsigned i = 0; i < cnt; ++i) {
     blocks(pm, i, n[i], kBlock);
     blocks(pm512, i, n[i], 512);  // the pass kernels' 512-thread blocks
@@ -807,6 +810,14 @@ void LaunchSet::release() {
   scenes = nullptr;
   pmap = cmap = pmap512 = qmap = nullptr;
   pblocks = ctiles = count = pblocks512 = qblocks = 0;
+}
+
+void LaunchSet::variants(int32_t* out4) const {
+  for (int k = 0; k < 2; ++k) {
+    const int v = one_shape ? 0 : pass_variant[k];  // one shape: 256 threads, as variant 0
+    out4[k] = v;
+    out4[2 + k] = v >= 0 ? pass_block_size(v) : -1;
+  }
 }
 
 namespace {
@@ -870,14 +881,20 @@ void run_steps(sph_s* const* P, unsigned count, LaunchSet& L, hipStream_t st, in
     }
   }
   const char* no_tune = std::getenv("GCLSPH_AUTOTUNE");
-  bool tune = !forced && L.pass_variant[0] < 0 && nsteps > kTuneTimed && !(no_tune && no_tune[0] == '0');
-  if (!forced && L.quad) {  // one shape, nothing to time; reported as variant 0, whose blocks it has
-    pv[0] = pv[1] = kPassQuad;
-    if (tune) L.pass_variant[0] = L.pass_variant[1] = 0;
+  const bool tunable = !forced && nsteps > kTuneTimed && !(no_tune && no_tune[0] == '0');
+  bool tune = tunable && L.pass_variant[0] < 0;
+  const bool general = std::is_same<R, double>::value && !L.gamma7;
+  const bool quad = general ? L.quad_general : L.quad;
+  if (!forced && (quad || general)) {  // one shape, nothing to time
+    pv[0] = pv[1] = quad ? kPassQuad : 0;
+    L.one_shape |= tunable;
     tune = false;
-  } else if (!forced && L.pass_variant[0] >= 0) {
-    pv[0] = L.pass_variant[0];
-    pv[1] = L.pass_variant[1];
+  } else if (!forced) {
+    L.one_shape = false;
+    if (L.pass_variant[0] >= 0) {
+      pv[0] = L.pass_variant[0];
+      pv[1] = L.pass_variant[1];
+    }
   }
   // one step's launches; with the corrections of every problem that may need
   // them (each kernel returns at once for a problem that does not)
@@ -1654,11 +1671,7 @@ int sph_get_timing(sph_t h, double* ms, int64_t* launches, int cap, int* nstages
 int sph_get_pass_variants(sph_t h, int32_t* out4) {
   return guard([&] {
     GCL_CHECK(h != nullptr && out4 != nullptr, kErrArgument, "NULL argument");
-    for (int k = 0; k < 2; ++k) {
-      const int v = h->own.pass_variant[k];
-      out4[k] = v;
-      out4[2 + k] = v >= 0 ? pass_block_size(v) : -1;
-    }
+    h->own.variants(out4);
   });
 }
 
@@ -1727,10 +1740,6 @@ int sph_batch_stepsolve(sph_batch_t b, int64_t n, int timestepping, const double
 int sph_batch_get_pass_variants(sph_batch_t b, int32_t* out4) {
   return guard([&] {
     GCL_CHECK(b != nullptr && out4 != nullptr, kErrArgument, "NULL argument");
-    for (int k = 0; k < 2; ++k) {
-      const int v = b->L.pass_variant[k];
-      out4[k] = v;
-      out4[2 + k] = v >= 0 ? pass_block_size(v) : -1;
-    }
+    b->L.variants(out4);
   });
 }

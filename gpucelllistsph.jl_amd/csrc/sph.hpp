@@ -308,16 +308,19 @@ struct LaunchSet {
   unsigned pblocks = 0, ctiles = 0, count = 0, pblocks512 = 0, qblocks = 0;
   int scan_rows = 4;  // rows per tile of the cell scan
   bool quad = false;  // the pair kernels run a quad of lanes per particle
+  bool quad_general = false;  // FP64 passes of another γ do (only where quad)
   bool gamma7 = true;  // γ = 7 in every problem (the FP64 passes have kernels for it)
   size_t scene_bytes = 0;
   // pass variants chosen by timing (-1: not yet)
   int pass_variant[2] = {-1, -1};
+  bool one_shape = false;  // the passes have one shape (quads; FP64 with another γ): nothing was timed
   // the captured step of the last call and what it was captured for
   hipGraphExec_t step_graph = nullptr;
   std::vector<unsigned char> graph_key;
   // n[i] particles and ncells[i] cells of problem i
   void build(const int64_t* n, const int64_t* ncells, unsigned count, int dim, bool split, size_t scene_bytes);
   void release();
+  void variants(int32_t* out4) const;  // what sph_get_pass_variants reports
 };
 
 // Rebuild stage of one step for every problem whose control block asks for it:

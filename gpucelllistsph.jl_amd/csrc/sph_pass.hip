@@ -533,8 +533,9 @@ void pass2_cg(const LaunchSet& L, hipStream_t s, int cg, size_t lds) {
 template <int D, typename R>
 void launch_pass1(const LaunchSet& L, hipStream_t s, int variant) {
   if constexpr (std::is_same<R, double>::value) {
-    if (!L.gamma7) {  // another γ: one kernel, whatever the variant
-      pass1_as<D, R, false, 1, 256, false>(L, s, 0);
+    if (!L.gamma7) {  // another γ: one kernel, whatever the variant, and its quads
+      if (variant == kPassQuad) pass1_as<D, R, false, 1, 256, false, true>(L, s, 0);
+      else pass1_as<D, R, false, 1, 256, false>(L, s, 0);
       return;
     }
   }
@@ -553,8 +554,9 @@ void launch_pass1(const LaunchSet& L, hipStream_t s, int variant) {
 template <int D, typename R>
 void launch_pass2(const LaunchSet& L, hipStream_t s, int variant) {
   if constexpr (std::is_same<R, double>::value) {
-    if (!L.gamma7) {  // another γ: one kernel, whatever the variant
-      pass2_as<D, R, false, 1, 256, false>(L, s, 0);
+    if (!L.gamma7) {  // another γ: one kernel, whatever the variant, and its quads
+      if (variant == kPassQuad) pass2_as<D, R, false, 1, 256, false, true>(L, s, 0);
+      else pass2_as<D, R, false, 1, 256, false>(L, s, 0);
       return;
     }
   }

@@ -196,8 +196,8 @@ int sph_get_timing(sph_t h, double* ms, int64_t* launches, int cap, int* nstages
  * 31 steps, after up to 16 untimed ones (the device warming up).
  * out4: variant of pass 1, variant of pass 2, threads per block of pass 1,
  * of pass 2; -1 until tuned (a problem too small to fill the GPU with a thread
- * per particle runs one fixed shape, four threads per particle, reported as
- * variant 0).  A variant is codegen + 4·b + 12·c, codegen in
+ * per particle runs one fixed shape, four threads per particle, and Float64
+ * problems with a gamma other than 7 one of their own: reported as variant 0).  A variant is codegen + 4·b + 12·c, codegen in
  * [0, 4) (partner prefetch on/off, occupancy target), b the block size (0:
  * 256, 1: 128, 2: 512 threads) and c an occupancy cap (1: at most 4 waves per
  * SIMD); 2D has the block sizes alone.  Every variant gives identical results. */

@@ -377,6 +377,33 @@ def test_gamma_other_than_7(G, O, S):
         G.SPHProblem.from_params(cl2, sc.params, sc.rho, sc.ptype, precision="f32split")
 
 
+@pytest.mark.parametrize("case", ["dam2d_allphys", "dam3d_allphys"])
+def test_gamma_other_than_7_has_one_shape(G, monkeypatch, case):
+    """Float64 passes with γ = 5 have one kernel and its quads: equal steps, and
+    the tuner, which has nothing to choose from, reports variant 0 for each; γ = 7
+    set afterwards is tuned."""
+    sc, _, ts = golden_cases()[case]
+
+    def run(lanes):
+        monkeypatch.setenv("GCLSPH_PAIR_LANES", lanes)
+        cl = G.GPUCellList(sc.points, sc.cellsize, sc.dist)
+        prob = G.SPHProblem.from_params(cl, sc.params, sc.rho, sc.ptype, v=sc.v, precision="f64")
+        prob.gamma = 5
+        out = [G.stepsolve_(prob, n, timestepping=ts) for n in (1, 33, 2)]
+        assert prob.pass_variants() == {"pass1": 0, "pass2": 0, "pass1_threads": 256, "pass2_threads": 256}
+        return prob, out + [np.asarray(gpu_fields(G, prob)[f]) for f in FIELDS]
+
+    _, quads = run("4")
+    prob, lanes = run("1")
+    for a, b in zip(quads, lanes):
+        assert np.array_equal(np.asarray(a), np.asarray(b))
+    prob.gamma = 7
+    G.stepsolve_(prob, 2, timestepping=ts)
+    assert prob.pass_variants()["pass1"] == -1
+    G.stepsolve_(prob, 33, timestepping=ts)
+    assert prob.pass_variants()["pass1"] >= 0
+
+
 @pytest.mark.parametrize("c0", [88.6, 47.0, 46.0, 20.0])
 def test_f64_hydrostatic_term_ranges(G, O, S, c0):
     """The δ-SPH hydrostatic term of γ = 7 is a series while |ρ0 g Δy / Cb| < 2^-8
