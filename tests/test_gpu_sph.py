@@ -635,6 +635,46 @@ def test_pass_variants_bit_identical(G, monkeypatch, prec):
 
 
 @pytest.mark.parametrize("prec", ["f64", "f32split"])
+@pytest.mark.parametrize("case", ["dam2d_allphys", "dam3d_allphys"])
+def test_one_lane_variants_and_tuner(G, monkeypatch, case, prec):
+    """The pass variants with one lane per particle (GCLSPH_PAIR_LANES=1, whatever
+    the size): the block sizes in 2D; in 3D every code generation, block size and
+    occupancy cap.  The tuner runs on the first call of more than 15 steps, not on
+    a shorter one, keeps its choice, and every step is bit-identical."""
+    sc, _, ts = golden_cases()[case]
+    monkeypatch.setenv("GCLSPH_PAIR_LANES", "1")
+
+    def run(variant, calls=(2, 33, 20)):
+        if variant is None:
+            monkeypatch.delenv("GCLSPH_PASS_VARIANT", raising=False)
+        else:
+            monkeypatch.setenv("GCLSPH_PASS_VARIANT", variant)
+        cl = G.GPUCellList(sc.points, sc.cellsize, sc.dist)
+        prob = G.SPHProblem.from_params(cl, sc.params, sc.rho, sc.ptype, v=sc.v, precision=prec)
+        out, chosen = [], []
+        for n in calls:
+            out.append(G.stepsolve_(prob, n, timestepping=ts))
+            chosen.append(prob.pass_variants())
+        return chosen, out + [np.asarray(gpu_fields(G, prob)[f]) for f in FIELDS]
+
+    _, ref = run("0,0")
+    variants = ["4,4", "8,8", "4,8"] if case == "dam2d_allphys" else [f"{v},{v}" for v in range(1, 24)] + ["3,18"]
+    for v in variants:
+        for a, b in zip(run(v)[1], ref):
+            assert np.array_equal(np.asarray(a), np.asarray(b)), v
+    chosen, got = run(None)
+    for a, b in zip(got, ref):
+        assert np.array_equal(np.asarray(a), np.asarray(b))
+    assert set(chosen[0].values()) == {-1}
+    assert chosen[1] == chosen[2]
+    for k in ("pass1", "pass2"):
+        v = chosen[1][k]
+        assert v in ((0, 4, 8) if case == "dam2d_allphys" else range(24))
+        assert chosen[1][k + "_threads"] == (256, 128, 512)[v // 4 % 3]
+        assert not (case == "dam3d_allphys" and prec == "f64" and v % 4 == 3)
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32split"])
 @pytest.mark.parametrize("case", ["dam2d", "dam2d_allphys", "dam3d_allphys", 1, 3, 63, 65, 129])
 def test_pair_quads_equal_one_lane(G, S, monkeypatch, prec, case):
     """Small problems give a particle four lanes in the pair kernels, which add
