@@ -344,7 +344,6 @@ struct sph_s {
     B.PN = dalloc<R>(n);
     B.PH = dalloc<R>(n);
     B.TMP = dalloc<double>(n);
-    B.nblk = int(grid_for(n));
     B.RED = dalloc<double>(3 * 64);  // zeroed here; k_finalize clears it after every step
     B.SUMW = dalloc<double>(n);
     B.start = sb.start;
@@ -489,7 +488,6 @@ struct sph_s {
     C.f_DDTgz = float(C.DDTgz);
     C.f_P0 = float(C.P0);
     C.f_wnorm = float(C.wnorm);
-    C.f_dwnorm = float(C.dwnorm);
     C.f_inv_rho0 = float(1.0 / C.rho0);
     C.f_st_turn = float(C.st_c / (2.0 * M_PI * C.st_2h));
     C.f_dwr = float(C.dwr);
@@ -500,7 +498,6 @@ struct sph_s {
       C.f_fb_eta2[k] = float(C.fb_eta2[k]);
     }
     C.f_st_2h = float(C.st_2h);
-    C.f_st_c = float(C.st_c);
     C.f_st_01h = float(C.st_01h);
     C.f_xsph_c = float(C.xsph_c);
     C.f_dpc_l0inv = float(C.dpc_l0inv);
@@ -852,7 +849,6 @@ void run_steps(sph_s* const* P, unsigned count, LaunchSet& L, hipStream_t st, in
     h.maxcdx_out = 0;
     h.dt = p->par[SPH_DT];
     h.etime = p->par[SPH_ETIME];
-    h.red_cdx = h.red_acc = h.red_visc = 0;
     h.iter = 1;
     h.nsteps = int(nsteps);
     h.synced = p->synced_prev ? 1 : 0;

@@ -237,7 +237,7 @@ __global__ __launch_bounds__(256) void k_pair_count2(XPtrs xsp, const int32_t* _
   const T* x[3] = {static_cast<const T*>(xsp.p[0]), static_cast<const T*>(xsp.p[1]),
                    static_cast<const T*>(xsp.p[1])};
   RowUnion u;
-  row_union(u, start, skey, g, n, s0, 0, 64);
+  row_union(u, start, skey, g, n, s0);
   const int32_t total = u.uo[3] - u.uo[1];  // rows 1 and 2
   const bool staged = total <= kCountWave;   // uniform over the wave
   T2* wl = lds[w];

@@ -155,26 +155,24 @@ __device__ __forceinline__ Rows<D> stencil_rows(const CellGeom& g, const int32_t
   return r;
 }
 
-// The union of the stencil rows of `span` consecutive particles from a0 (a
-// block or a wave) in one plane (2D: the only plane; 3D: the plane dz ∈ {-1,
-// 0, 1}).  The particles a0..a1 occupy one contiguous range of cells [c0, c1],
-// so for each row offset k the cells [c0 + o - 1, c1 + o + 1], o = (k-1)·gx +
-// dz·gx·gy, hold every candidate of that row of every one of them: three
-// contiguous ranges of sorted particles starting at ub[k], laid out one after
-// the other from LDS slot uo[k].
+// The union of the stencil rows of the 64 consecutive particles of a wave from a0
+// in 2D.  The particles a0..a1 occupy one contiguous range of cells [c0, c1], so
+// for each row offset k the cells [c0 + o - 1, c1 + o + 1], o = (k-1)·gx, hold
+// every candidate of that row of every one of them: three contiguous ranges of
+// sorted particles starting at ub[k], laid out one after the other from LDS slot
+// uo[k].
 struct RowUnion {
   int32_t ub[3], uo[4];
 };
 
 __device__ __forceinline__ void row_union(RowUnion& u, const int32_t* start, const int32_t* skey, const CellGeom& G,
-                                          int64_t n, int64_t a0, int dz = 0, int span = kBlock) {
-  const int64_t a1 = (a0 + span < n ? a0 + span : n) - 1;
+                                          int64_t n, int64_t a0) {
+  const int64_t a1 = (a0 + 64 < n ? a0 + 64 : n) - 1;
   const int64_t c0 = skey[a0], c1 = skey[a1];
   const int64_t gx = G.grid[0], nc = G.ncells();
-  const int64_t zo = int64_t(dz) * gx * G.grid[1];
   int32_t o = 0;
   for (int k = 0; k < 3; ++k) {
-    int64_t lo = c0 + (k - 1) * gx + zo - 1, hi = c1 + (k - 1) * gx + zo + 1;
+    int64_t lo = c0 + (k - 1) * gx - 1, hi = c1 + (k - 1) * gx + 1;
     lo = lo < 0 ? 0 : (lo > nc - 1 ? nc - 1 : lo);
     hi = hi < 0 ? 0 : (hi > nc - 1 ? nc - 1 : hi);
     const int32_t b = start[lo], e = start[hi + 1];

@@ -62,11 +62,6 @@ struct StepCtl {
   double dt;
   double etime;
   double maxcdx_out;  // max over steps of max |cdx|
-  // reduction slots (non-negative doubles compared as uint64 bit patterns)
-  unsigned long long red_cdx;
-  unsigned long long red_acc;
-  unsigned long long red_visc;
-  unsigned long long red_maxcell;
 };
 
 // Device helpers ------------------------------------------------------------
@@ -85,7 +80,5 @@ __device__ inline void atomic_max_nonneg(unsigned long long* slot, double v) {
   if (b & 0x8000000000000000ull) b = 0;  // -0.0 and negatives clamp to 0
   atomicMax(slot, b);
 }
-
-__device__ inline double bits_to_double(unsigned long long b) { return __longlong_as_double((long long)b); }
 
 }  // namespace gclsph

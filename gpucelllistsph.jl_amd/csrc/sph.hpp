@@ -36,7 +36,7 @@ struct SphConst {
   double CFL, nui, tl0, tl1;
   // single-precision copies for the FP32-split kernels
   float f_h, f_Hinv, f_rho0, f_m0, f_alpha, f_c0, f_g, f_s, f_nu, f_eta2, f_DDTkh, f_DDTgz, f_P0, f_wnorm,
-      f_dwnorm, f_fb_d[2], f_fb_r0[2], f_fb_eta2[2], f_st_2h, f_st_c, f_st_01h, f_xsph_c;
+      f_fb_d[2], f_fb_r0[2], f_fb_eta2[2], f_st_2h, f_st_01h, f_xsph_c;
   float f_dpc_l0inv, f_dpc_eta2, f_dpc_whinv, f_dpc_lim, f_dpc_wnorm, f_dpc_lambda, f_dpc_pmin, f_dpc_pmax;
   float f_inv_rho0;  // 1/ρ0
   float f_inv_m0;    // 1/m0
@@ -111,8 +111,7 @@ struct SphBufs {
   const int32_t* perm;
   const int32_t* maxcell;
   StepCtl* ctl;
-  double* RED;  // per-block partial maxima: [|cdx|, |a|, visc] x nblk
-  int nblk;
+  double* RED;  // partial maxima: [|cdx|, |a|, visc] in 64 slots each
   // neighbour-list membership of the last rebuild (written with the reorder): entry e of
   // particle a at NE[e * n + a] = (window base << 32) | member bits; NC[a]
   // entries, or -1 when more than necap were needed; NE has necap + 1 rows

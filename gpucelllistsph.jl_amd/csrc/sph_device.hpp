@@ -306,19 +306,6 @@ struct Sums {
 };
 
 template <int D>
-__device__ __forceinline__ bool member(const double* const* XM, int64_t a, int64_t b, double dist2) {
-#pragma clang fp contract(off)
-  double d0 = XM[0][a] - XM[0][b];
-  double d1 = XM[1][a] - XM[1][b];
-  double s = d0 * d0 + d1 * d1;
-  if (D == 3) {
-    double d2 = XM[2][a] - XM[2][b];
-    s = s + d2 * d2;
-  }
-  return s < dist2;
-}
-
-template <int D>
 __device__ __forceinline__ double dotd(const double* a, const double* b) {
 #pragma clang fp contract(off)
   double s = a[0] * b[0] + a[1] * b[1];

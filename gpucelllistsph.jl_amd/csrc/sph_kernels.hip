@@ -402,7 +402,7 @@ __device__ __forceinline__ void nmask2_new(const SphBufs<R>& B, const SphConst& 
   const int64_t aw = a0 + 64 * w;
   if (aw >= B.n) return;  // whole wave
   RowUnion u;
-  row_union(u, B.start, B.skey, G, B.n, aw, 0, 64);
+  row_union(u, B.start, B.skey, G, B.n, aw);
   const int32_t total = u.uo[3];
   if (total <= kNmaskWave) {  // uniform over the wave
     double2* wl = lds[w];
@@ -917,9 +917,6 @@ __global__ void k_finalize(SS ss) {
     dt = jl_min(jl_max(dt, C.tl0), C.tl1);
     ctl->dt = dt;
   }
-  ctl->red_cdx = 0;
-  ctl->red_acc = 0;
-  ctl->red_visc = 0;
   ctl->parity ^= 1;
   ctl->synced = corr_on ? 0 : 1;
   ctl->iter += 1;
