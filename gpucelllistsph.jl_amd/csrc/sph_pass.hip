@@ -497,11 +497,14 @@ size_t cap_lds(int bs) {
 // per SIMD; 3 (FP32-split) not pipelined, >= 5 waves/SIMD, which makes FP64
 // spill: there it is 1.  2D, where the records are staged, has one: four waves
 // per SIMD, as the staged records allow (FP64 pass 2 by itself would take the
-// registers of three: 246 us, 230 so, 1.02 M particles).
+// registers of three: 246 us, 230 so, 1.02 M particles).  Prefetch concerns its
+// blocks whose rows don't fit alone: FP32-split has it (614,072 particles, smoothing
+// length 2.2 and 3 times the usual: a step 899 -> 843, 1841 -> 1789 us), FP64 has
+// no registers for it.
 template <int D, typename R, int BS>
 void pass1_cg(const LaunchSet& L, hipStream_t s, int cg, size_t lds) {
   if constexpr (D == 2) {
-    pass1_as<D, R, false, 4, BS>(L, s, 0);
+    pass1_as<D, R, std::is_same<R, float>::value, 4, BS>(L, s, 0);
   } else {
     constexpr bool f32 = std::is_same<R, float>::value;
     switch (cg) {
@@ -515,7 +518,7 @@ void pass1_cg(const LaunchSet& L, hipStream_t s, int cg, size_t lds) {
 template <int D, typename R, int BS>
 void pass2_cg(const LaunchSet& L, hipStream_t s, int cg, size_t lds) {
   if constexpr (D == 2) {
-    pass2_as<D, R, false, 4, BS>(L, s, 0);
+    pass2_as<D, R, std::is_same<R, float>::value, 4, BS>(L, s, 0);
   } else {
     constexpr bool f32 = std::is_same<R, float>::value;
     switch (cg) {
