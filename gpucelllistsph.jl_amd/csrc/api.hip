@@ -75,6 +75,11 @@ __global__ void k_export(Fields<T> src, const int32_t* __restrict__ inv, double*
   const T* v = c == 0 ? src.c[0] : (c == 1 ? src.c[1] : src.c[2]);
   out[j] = double(v[inv[e - c * n]]) + add;
 }
+// Points of cells [0, count) from their starts (to page-locked host memory).
+__global__ void k_cell_points(const int32_t* __restrict__ start, int32_t* __restrict__ out, int64_t count) {
+  const int64_t c = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (c < count) out[c] = start[c + 1] - start[c];
+}
 template <typename T>
 __global__ void k_scatter_by(const T* __restrict__ src, T* __restrict__ dst, const int32_t* __restrict__ id,
                              int64_t n) {
@@ -1391,11 +1396,11 @@ int gcl_get_cellpnum(gcl_t h, int32_t* out) {
     GCL_CHECK(h != nullptr && out != nullptr, kErrArgument, "NULL argument");
     SortBuffers& sb = h->attached ? h->attached->sb : h->sb;
     hipStream_t s = h->attached ? h->attached->stream : h->stream;
-    const size_t nc = size_t(h->G.ncells());
-    std::vector<int32_t> start(nc + 1);
-    GCL_HIP(hipMemcpyAsync(start.data(), sb.start, 4 * (nc + 1), hipMemcpyDeviceToHost, s));
-    GCL_HIP(hipStreamSynchronize(s));
-    for (size_t c = 0; c < nc; ++c) out[c] = start[c + 1] - start[c];
+    HostSlots::copy_out(out, sizeof(int32_t) * size_t(h->G.ncells()), s, [&](void* slot, size_t off, size_t len) {
+      const int64_t first = int64_t(off / sizeof(int32_t)), count = int64_t(len / sizeof(int32_t));
+      k_cell_points<<<grid_for(count), kBlock, 0, s>>>(sb.start + first, static_cast<int32_t*>(slot), count);
+      GCL_HIP(hipGetLastError());
+    });
   });
 }
 
