@@ -378,7 +378,7 @@ def main():
                 "achieved": prof["valu_instructions_per_dispatch"] / (dom_ms * 1e-3) / 1e9,
                 "peak": VALU_PEAK_GIPS, "unit": "G wave64 VALU instructions/s",
                 "frac": prof["valu_instructions_per_dispatch"] / (dom_ms * 1e-3) / 1e9 / VALU_PEAK_GIPS},
-            "note": "pair passes are co-limited by vector-L1 access rate and VALU issue, not HBM: "
+            "note": "pair passes are limited by VALU issue, not HBM (partner records are read from LDS): "
                     "achieved = algorithmic bytes / measured kernel time; "
                     "valu_busy (share of SIMD cycles issuing VALU) and traffic come from the committed PMC profile",
         },

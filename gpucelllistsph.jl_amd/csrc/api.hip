@@ -835,6 +835,7 @@ void run_steps(sph_s* const* P, unsigned count, LaunchSet& L, hipStream_t st, in
   std::vector<SceneDev<R>> descs(count);
   std::vector<StepFlags> flags(count);
   bool any_dpc = false, any_xsph = false, any_dtv = false;
+  bool any_ax = false;  // viscosity or surface tension
   L.gamma7 = true;
   for (unsigned i = 0; i < count; ++i) {
     sph_s* p = P[i];
@@ -848,6 +849,7 @@ void run_steps(sph_s* const* P, unsigned count, LaunchSet& L, hipStream_t st, in
     any_dpc |= F.dpc_on != 0;
     any_xsph |= F.xsph_on != 0;
     any_dtv |= F.ts && !F.visc_in_pass2;
+    any_ax |= F.nu_on || F.s_on;
     StepCtl& h = p->hctl;
     h.rebuild = 1;  // the first iteration of every call rebuilds (src/sphproblem.jl:212,222)
     h.updaten = 0;
@@ -868,9 +870,12 @@ void run_steps(sph_s* const* P, unsigned count, LaunchSet& L, hipStream_t st, in
   // timing, else the fastest measured on the dam-break scenes per dimension
   // and precision until it has been tuned.
   int pv[2];
-  // 3D: prefetch, three waves per SIMD (191,232 particles FP64 299 + 320 us,
-  // 303 + 376 without prefetch); 2D has block sizes only
+  // 3D: prefetch, three waves per SIMD.  Held to three, FP64 pass 2 spills 20
+  // registers, some of them in the viscosity and surface terms: with those it takes
+  // what two waves have (1,003,514 particles: a step with every term 7.26 -> 5.48
+  // ms; without them 3.34, 3.39 so).  2D has block sizes only.
   pv[0] = pv[1] = D == 3 ? 2 : 0;
+  if (D == 3 && std::is_same<R, double>::value && any_ax) pv[1] = 0;
   bool forced = false;
   if (const char* env = std::getenv("GCLSPH_PASS_VARIANT")) {
     int v1 = -1, v2 = -1;

@@ -490,7 +490,7 @@ size_t cap_lds(int bs) {
   }
   const size_t cu = size_t(per_cu[dev].load()), blk = size_t(per_block[dev].load());
   const size_t blocks = size_t(4 * kPassCapWaves * 64 / bs);
-  const size_t lds = cu / (blocks + 1) + 1024;  // the static LDS of a pass block is below 1 KiB
+  const size_t lds = cu / (blocks + 1) + 1024;  // the static LDS of a 3D pass block is below 1 KiB (2D has no cap)
   return blocks * lds <= cu && lds <= blk ? lds : 0;
 }
 // Code generation cg, 3D: 0 pipelined; 1 not pipelined; 2 pipelined, three waves
